@@ -470,12 +470,6 @@ void by_dtype(int dtype, F&& f) {
 // Every op runs on its context's device, whichever thread calls it.
 void use(const dmrg_ctx* c) { DMRG_HIP(hipSetDevice(c->device)); }
 
-template <class T>
-std::vector<T> d2h(const void* p, size_t n) {
-  std::vector<T> h(n);
-  DMRG_HIP(hipMemcpy(h.data(), p, n * sizeof(T), hipMemcpyDeviceToHost));
-  return h;
-}
 }  // namespace
 
 extern "C" {
@@ -509,15 +503,13 @@ int dmrg_op_heff2(dmrg_ctx_handle c, void* stream, int dtype, int cL, int cR, in
       using T = decltype(tag);
       auto& x = ctx_of<T>(c);
       hipStream_t st = (hipStream_t)stream;
-      // the caller's pending writes of the MPO and the previous call's reads
-      // of the context's MPO buffer are ordered on the stream: drain it first
-      DMRG_HIP(hipStreamSynchronize((hipStream_t)stream));
-      const size_t wsz = (size_t)D * d * d * D, K = (size_t)D * d * d;
-      auto h1 = d2h<T>(W1, wsz), h2 = d2h<T>(W2, wsz);
-      std::vector<T> ww(K * K);
-      build_ww2<T>(h1.data(), h2.data(), d, D, ww.data());
+      // fused on the device: the caller's pending writes of the MPO and the
+      // previous call's reads of the context's MPO buffer are ordered on the
+      // stream (fusing on the host cost a drained stream, two read-backs and a
+      // copy: 45 us of a 57 us call at cL = 16, cR = 32)
+      const size_t K = (size_t)D * d * d;
       T* dww = x.need_buf(K * K);
-      DMRG_HIP(hipMemcpy(dww, ww.data(), K * K * sizeof(T), hipMemcpyHostToDevice));
+      build_ww2_dev<T, T>(st, (const T*)W1, (const T*)W2, d, D, dww);
       x.need_sc((size_t)D * d * d * cL * cR);
       heff2_apply<T>(st, (const T*)L, (const T*)R, dww, (const T*)theta, (T*)out, cL, cR, d, D, x.sc);
     });
@@ -533,18 +525,10 @@ int dmrg_op_heff2_f32(dmrg_ctx_handle c, void* stream, int prec, int cL, int cR,
     DMRG_REQUIRE(cL >= 1 && cR >= 1 && d >= 1 && D >= 1, "bad shape");
     DMRG_REQUIRE(prec == DMRG_PREC_FP32 || prec == DMRG_PREC_BF16X3, "prec must be FP32 or BF16X3");
     hipStream_t st = (hipStream_t)stream;
-    // the caller's pending writes of the MPO and the previous call's reads
-    // of the context's MPO buffer are ordered on the stream: drain it first
-    DMRG_HIP(hipStreamSynchronize(st));
     auto& x = c->f;
-    const size_t wsz = (size_t)D * d * d * D, K = (size_t)D * d * d;
-    auto h1 = d2h<double>(W1, wsz), h2 = d2h<double>(W2, wsz);
-    std::vector<double> ww(K * K);
-    build_ww2<double>(h1.data(), h2.data(), d, D, ww.data());
-    std::vector<float> wwf(K * K);
-    for (size_t i = 0; i < K * K; ++i) wwf[i] = (float)ww[i];
+    const size_t K = (size_t)D * d * d;
     float* dww = x.need_buf(K * K);
-    DMRG_HIP(hipMemcpy(dww, wwf.data(), K * K * sizeof(float), hipMemcpyHostToDevice));
+    build_ww2_dev<double, float>(st, W1, W2, d, D, dww);
     x.need_sc((size_t)D * d * d * cL * cR);
     x.sc.split_bf16 = prec == DMRG_PREC_BF16X3;
     heff2_apply<float>(st, L, R, dww, theta, out, cL, cR, d, D, x.sc);
@@ -599,15 +583,9 @@ int dmrg_op_env_right(dmrg_ctx_handle c, void* stream, int dtype, int ci, int co
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
       auto& x = ctx_of<T>(c);
-      // the caller's pending writes of the MPO and the previous call's reads
-      // of the context's MPO buffer are ordered on the stream: drain it first
-      DMRG_HIP(hipStreamSynchronize((hipStream_t)stream));
       const size_t wsz = (size_t)D * d * d * D;
-      auto hw = d2h<T>(W, wsz);
-      std::vector<T> wr(wsz);
-      build_wright<T>(hw.data(), d, D, wr.data());
       T* dwr = x.need_buf(wsz);
-      DMRG_HIP(hipMemcpy(dwr, wr.data(), wsz * sizeof(T), hipMemcpyHostToDevice));
+      build_wright_dev<T>((hipStream_t)stream, (const T*)W, d, D, dwr);
       x.need_sc((size_t)D * d * ci * co);
       env_right<T>((hipStream_t)stream, (const T*)R, (const T*)A, dwr, (T*)Rnew, ci, co, d, D, x.sc);
     });
@@ -710,15 +688,9 @@ int dmrg_op_lanczos2(dmrg_ctx_handle c, void* stream, int dtype, int cL, int cR,
       auto& x = ctx_of<T>(c);
       hipStream_t st = (hipStream_t)stream;
       const size_t n = (size_t)cL * d * d * cR;
-      // the caller's pending writes of the MPO and the previous call's reads
-      // of the context's MPO buffer are ordered on the stream: drain it first
-      DMRG_HIP(hipStreamSynchronize((hipStream_t)stream));
-      const size_t wsz = (size_t)D * d * d * D, K = (size_t)D * d * d;
-      auto h1 = d2h<T>(W1, wsz), h2 = d2h<T>(W2, wsz);
-      std::vector<T> ww(K * K);
-      build_ww2<T>(h1.data(), h2.data(), d, D, ww.data());
+      const size_t K = (size_t)D * d * d;
       T* dww = x.need_buf(K * K);
-      DMRG_HIP(hipMemcpy(dww, ww.data(), K * K * sizeof(T), hipMemcpyHostToDevice));
+      build_ww2_dev<T, T>(st, (const T*)W1, (const T*)W2, d, D, dww);
       x.need_sc((size_t)D * d * d * cL * cR);
       const int kmax = (int)std::min<size_t>(krylov_max, n);
       if ((size_t)kmax * n > x.V_cap) {

@@ -179,6 +179,37 @@ void build_wright(const T* W, int d, int D, T* Wr) {
 }
 
 namespace {
+// One thread per entry of the fused two-site MPO (row w1 + D (s1 + d s2),
+// column (s1' + d s2') + d^2 n), summing over the middle bond in the order of
+// build_ww2.  At most (D d^2)^2 entries: a launch, nothing else, bounds it.
+template <class T, class TO>
+__global__ __launch_bounds__(256) void k_build_ww(const T* __restrict__ W1, const T* __restrict__ W2,
+                                                  int d, int D, TO* __restrict__ WW) {
+  const int dd = d * d, K = D * dd;
+  const size_t tot = (size_t)K * K;
+  for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < tot; e += (size_t)gridDim.x * 256) {
+    const int row = (int)(e % K), col = (int)(e / K);
+    const int a = row % D, s = row / D, s1 = s % d, s2 = s / d;
+    const int n = col / dd, sp = col % dd, s1p = sp % d, s2p = sp / d;
+    const T* p1 = W1 + a + (size_t)D * (s1 + (size_t)d * s1p);
+    const T* p2 = W2 + (size_t)D * (s2 + (size_t)d * (s2p + (size_t)d * n));
+    T v(0);
+    for (int m = 0; m < D; ++m) v = v + p1[(size_t)D * d * d * m] * p2[m];
+    WW[e] = (TO)v;
+  }
+}
+// Wr[(s + d w') + d D (w + D sp)] = W[w, s, sp, w'], one thread per entry.
+template <class T>
+__global__ __launch_bounds__(256) void k_build_wright(const T* __restrict__ W, int d, int D,
+                                                      T* __restrict__ Wr) {
+  const int K = d * D;
+  const size_t tot = (size_t)K * K;
+  for (size_t e = blockIdx.x * (size_t)256 + threadIdx.x; e < tot; e += (size_t)gridDim.x * 256) {
+    const int row = (int)(e % K), col = (int)(e / K);
+    const int s = row % d, wp = row / d, w = col % D, sp = col / D;
+    Wr[e] = W[w + (size_t)D * (s + (size_t)d * (sp + (size_t)d * wp))];
+  }
+}
 __global__ void k_f64_f32(const double* in, float* out, size_t n) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
@@ -279,6 +310,27 @@ __global__ void k_unit(T* env, int D, int w) {
   if (i < D) env[i] = (i == w) ? T(1) : T(0);
 }
 }  // namespace
+
+template <class T, class TO>
+void build_ww2_dev(hipStream_t st, const T* W1, const T* W2, int d, int D, TO* WW) {
+  const size_t K = (size_t)D * d * d;
+  hipLaunchKernelGGL((k_build_ww<T, TO>), dim3(std::min<size_t>(cdiv(K * K, 256), 4096)), dim3(256),
+                     0, st, W1, W2, d, D, WW);
+  DMRG_LAUNCH_CHECK();
+}
+template void build_ww2_dev<double, double>(hipStream_t, const double*, const double*, int, int, double*);
+template void build_ww2_dev<double, float>(hipStream_t, const double*, const double*, int, int, float*);
+template void build_ww2_dev<cdouble, cdouble>(hipStream_t, const cdouble*, const cdouble*, int, int,
+                                              cdouble*);
+template <class T>
+void build_wright_dev(hipStream_t st, const T* W, int d, int D, T* Wr) {
+  const size_t K = (size_t)D * d;
+  hipLaunchKernelGGL(k_build_wright<T>, dim3(std::min<size_t>(cdiv(K * K, 256), 4096)), dim3(256), 0,
+                     st, W, d, D, Wr);
+  DMRG_LAUNCH_CHECK();
+}
+template void build_wright_dev<double>(hipStream_t, const double*, int, int, double*);
+template void build_wright_dev<cdouble>(hipStream_t, const cdouble*, int, int, cdouble*);
 
 void convert_f64_f32(hipStream_t st, const double* in, float* out, size_t n) {
   if (!n) return;

@@ -63,6 +63,12 @@ template <class T>
 void build_ww2(const T* W1, const T* W2, int d, int D, T* WW);
 template <class T>
 void build_wright(const T* W, int d, int D, T* Wr);
+// The same two matrices formed on the device from device tensors, in stream
+// order (W1, W2, W must be complete on `st`; TO = float rounds the FP64 sum).
+template <class T, class TO>
+void build_ww2_dev(hipStream_t st, const T* W1, const T* W2, int d, int D, TO* WW);
+template <class T>
+void build_wright_dev(hipStream_t st, const T* W, int d, int D, T* Wr);
 
 // Elementwise helpers.
 void convert_f64_f32(hipStream_t st, const double* in, float* out, size_t n);

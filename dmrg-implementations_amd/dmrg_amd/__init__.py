@@ -415,7 +415,7 @@ class Ops:
 
     def heff2_f32(self, L, R, W1, W2, theta, out, prec=PREC_FP32, stream=None):
         """Mixed-mode two-site matvec: float32 L, R, theta, out; float64 W1, W2
-        (fused on the host, rounded to FP32); FP32 MFMA or split-BF16 (prec)."""
+        (fused on the device, rounded to FP32); FP32 MFMA or split-BF16 (prec)."""
         cL, D = L.shape[0], L.shape[1]
         cR, d = R.shape[0], theta.shape[1]
         self._expect(np.float32, L=(L, (cL, D, cL)), R=(R, (cR, D, cR)),
