@@ -8,9 +8,6 @@
 namespace dmrg {
 
 namespace {
-inline GemmTile pick(int M, int N, int K) {
-  return gemm_pick_tile(M, N, K, false);
-}
 template <class T> inline GemmTile pickT(int M, int N, int K) {
   return gemm_pick_tile(M, N, K, is_cplx<T>::value);
 }
@@ -21,7 +18,7 @@ template <class T>
 void mpo_step(hipStream_t st, int M, int N, int K, const T* X, View2 vx, const T* W, T* Y,
               View2 vy) {
   if (gemm_rows_small<T>(st, M, N, K, X, vx, W, Y, vy)) return;
-  gemm_tensor<T>(st, M, N, K, T(1), X, vx, false, false, W, view_colmajor(K), false, true, T(0), Y,
+  gemm_tensor<T>(st, M, N, K, T(1), X, vx, W, view_colmajor(K), T(0), Y,
                  vy, pickT<T>(M, N, K));
 }
 
@@ -64,10 +61,11 @@ void heff2_apply(hipStream_t st, const T* Lenv, const T* Renv, const T* WW, cons
       done = true;
     }
   }
-  // X is free again here: it serves as the split-K workspace
+  // X is free again here: it serves as the split-K workspace (`need` of it,
+  // whatever its capacity, so that the slicing depends on the shape alone)
   if (!done)
-    done = gemm_nn_splitk<T>(st, cL * dd, cR, D * cR, sc.Y, cL * dd, Renv, cR * D, out, cL * dd,
-                             sc.X, sc.cap);
+    done = gemm_splitk<T>(st, OP_N, OP_N, cL * dd, cR, D * cR, sc.Y, cL * dd, Renv, cR * D, out,
+                          cL * dd, sc.X, need);
   if (!done)
     gemm<T>(st, OP_N, OP_N, cL * dd, cR, D * cR, one, sc.Y, cL * dd, Renv, cR * D, zero, out,
             cL * dd, pickT<T>(cL * dd, cR, D * cR));
@@ -88,7 +86,7 @@ void heff2_apply_f32_io64(hipStream_t st, const float* Lenv, const float* Renv, 
   if (!sc.split_bf16 && heff2_x_mpo<float>(st, cL, cR, d, D, Lenv, thf, WW, sc.Y)) {
     // X is free: it serves as the split-K workspace
     if (gemm_nn_splitk_to_f64(st, cL * dd, cR, D * cR, sc.Y, cL * dd, Renv, cR * D, out, cL * dd,
-                              sc.X, sc.cap, sL, sR))
+                              sc.X, need, sL, sR))
       return;
     gemm<float>(st, OP_N, OP_N, cL * dd, cR, D * cR, 1.f, sc.Y, cL * dd, Renv, cR * D, 0.f, outf,
                 cL * dd, pickT<float>(cL * dd, cR, D * cR));
@@ -110,8 +108,11 @@ void heff1_apply(hipStream_t st, const T* Lenv, const T* Renv, const T* W, const
   View2 vx{{cL, (long long)D, (long long)D * cL * d}, {D, 1, (long long)D * cL}};
   View2 vy{{cL, 1, (long long)cL * d}, {d, (long long)cL, (long long)cL * d * cR}};
   mpo_step<T>(st, cL * cR, d * D, D * d, sc.X, vx, W, sc.Y, vy);
-  gemm<T>(st, OP_N, OP_N, cL * d, cR, D * cR, one, sc.Y, cL * d, Renv, cR * D, zero, out, cL * d,
-          pickT<T>(cL * d, cR, D * cR));
+  // X is free again: the split-K workspace
+  if (!gemm_splitk<T>(st, OP_N, OP_N, cL * d, cR, D * cR, sc.Y, cL * d, Renv, cR * D, out, cL * d,
+                      sc.X, need))
+    gemm<T>(st, OP_N, OP_N, cL * d, cR, D * cR, one, sc.Y, cL * d, Renv, cR * D, zero, out, cL * d,
+            pickT<T>(cL * d, cR, D * cR));
 }
 
 template <class T>
@@ -125,8 +126,10 @@ void env_left(hipStream_t st, const T* Lenv, const T* A, const T* W, T* Lnew, in
   View2 vx{{ci, (long long)D, (long long)D * ci * d}, {D, 1, (long long)D * ci}};
   View2 vy{{ci, 1, (long long)ci * d}, {d, (long long)ci, (long long)ci * d * co}};
   mpo_step<T>(st, ci * co, d * D, D * d, sc.X, vx, W, sc.Y, vy);
-  gemm<T>(st, OP_T, OP_C, co * D, co, ci * d, one, sc.Y, ci * d, A, ci * d, zero, Lnew, co * D,
-          pickT<T>(co * D, co, ci * d));
+  if (!gemm_splitk<T>(st, OP_T, OP_C, co * D, co, ci * d, sc.Y, ci * d, A, ci * d, Lnew, co * D,
+                      sc.X, need))
+    gemm<T>(st, OP_T, OP_C, co * D, co, ci * d, one, sc.Y, ci * d, A, ci * d, zero, Lnew, co * D,
+            pickT<T>(co * D, co, ci * d));
 }
 
 template <class T>
@@ -143,8 +146,10 @@ void env_right(hipStream_t st, const T* Renv, const T* A, const T* Wr, T* Rnew, 
   View2 vy{{co, 1, (long long)co * D * d}, {D, (long long)co, (long long)co * D}};
   mpo_step<T>(st, co * ci, D * d, d * D, sc.X, vx, Wr, sc.Y, vy);
   // Rnew[(a + co w), a'] = sum_{(sp, b')} Y * conj(A[a', sp, b'])
-  gemm<T>(st, OP_N, OP_H, co * D, co, d * ci, one, sc.Y, co * D, A, co, zero, Rnew, co * D,
-          pickT<T>(co * D, co, d * ci));
+  if (!gemm_splitk<T>(st, OP_N, OP_H, co * D, co, d * ci, sc.Y, co * D, A, co, Rnew, co * D, sc.X,
+                      need))
+    gemm<T>(st, OP_N, OP_H, co * D, co, d * ci, one, sc.Y, co * D, A, co, zero, Rnew, co * D,
+            pickT<T>(co * D, co, d * ci));
 }
 
 template <class T>

@@ -1,13 +1,26 @@
 // MFMA GEMM kernels for gfx950 (see gemm.hpp).
 //
-// Workgroup: 256 threads = 4 wave64s in a 2x2 grid.  Each wave owns a
-// (BM/2) x (BN/2) sub-tile made of 16x16 MFMA blocks.  Operand tiles of depth
-// BK (16 or 32) are staged through LDS (double buffered, one-element row
-// padding), with the global loads of the next tile (PF=1) or of the next two
-// tiles (PF=2) issued before the MFMAs of the current one.  The MFMA is issued with the B fragment in the "A" slot so
-// that each lane's four accumulator registers land on four columns of C with
-// consecutive lanes on consecutive rows: epilogue stores of a column-major C
-// are 128-byte runs.
+// Tile (the struct TileLoop) is the k-loop of every plain product and of the
+// fused first H_eff step; k_gemm below it serves two-level operands only.
+//
+// What bounds these products on the card: FP64 MFMA at 64 cycles per
+// 16x16x4 step (78.6 TF/s at 2.4 GHz, but a large FP64 product settles near
+// 2.1 GHz, and lower the more operand traffic it causes), and everything a
+// wave issues between two MFMAs.  Hence:
+//  * operands travel in 16-byte chunks (2 FP64, 4 FP32, 1 complex128 value)
+//    from memory to LDS to registers;
+//  * the k-loop has no branch and no conditional load, so that the compiler
+//    can count outstanding loads exactly: every load of a tile is issued with
+//    its address clamped into the operand, and only the tiles that touch the
+//    end of k (or, for an operand that is contiguous along its other index,
+//    the end of that index) mask or shift what they got on the way to LDS;
+//  * the memory instructions of one tile are interleaved with the MFMAs of
+//    another: fragments of the next half tile are read while the present half
+//    multiplies, also across the barrier (one per tile).
+// Measured against the loop it replaces (element-wise LDS rows, loads under a
+// branch, which made every wait a wait for all loads): FP64 2048x512x2560
+// 120 -> 106 us, four k-slices 98 -> 88, 1024^3 50 -> 44, 512^3 10.9 -> 9.3;
+// FP32 2560x2048x512 69 -> 55, 2048x512x2560 87 -> 59 (two k-slices 69 -> 51).
 #include "gemm.hpp"
 
 #include <type_traits>
@@ -49,13 +62,6 @@ template <> __device__ inline void split<cdouble>(cdouble v, double* o) { o[0] =
 template <class T> __device__ inline T conj_v(T v) { return conj(v); }
 template <> __device__ inline float conj_v<float>(float v) { return v; }
 
-// Plain column-major operand; TR: stored transposed.
-template <bool TR> struct AddrPlain {
-  long long ld;
-  __device__ long long operator()(int r, int c) const {
-    return TR ? (long long)c + (long long)r * ld : (long long)r + (long long)c * ld;
-  }
-};
 // Two-level operand.
 struct AddrTensor {
   View2 v;
@@ -65,51 +71,360 @@ struct AddrTensor {
   __device__ long long operator()(int r, int c) const { return dim(v.row, r) + dim(v.col, c); }
 };
 
-// KS = 2: eight waves, two per output sub-tile, each multiplying one half of
-// every k-tile; the halves are summed through LDS at the end (twice the waves
-// per SIMD to hide latency when a grid has about one workgroup per CU).
-template <class T, bool CA, bool CB, bool KFA, bool KFB, int BM, int BN, int BK, int PF, int KS,
-          class AA, class AB, class AC>
-__global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
-                                                   const T* __restrict__ A, AA aa, long long sA,
-                                                   const T* __restrict__ B, AB ab, long long sB,
-                                                   T beta, T* __restrict__ C, AC ac, long long sC,
-                                                   int herm) {
+typedef unsigned u4_t __attribute__((ext_vector_type(4)));
+
+// The order of one half tile's instructions: after MFMA i of MH, its share of
+// NR LDS reads (spread over the first half of the MFMAs) and of NX
+// instructions of class MX (over the first half, or the second when X2).
+template <int I, int MH, int NR, int MX, int NX, bool X2>
+__device__ inline void interleave() {
+  if constexpr (I < MH) {
+    constexpr int h = MH / 2;
+    constexpr int r = I < h ? NR * (I + 1) / h - NR * I / h : 0;
+    constexpr int x = X2 ? (I >= h ? NX * (I - h + 1) / (MH - h) - NX * (I - h) / (MH - h) : 0)
+                         : (I < h ? NX * (I + 1) / h - NX * I / h : 0);
+    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+    if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);
+    if constexpr (x > 0) __builtin_amdgcn_sched_group_barrier(MX, x, 0);
+    interleave<I + 1, MH, NR, MX, NX, X2>();
+  }
+}
+constexpr int kSchedDsWrite = 0x200, kSchedVmemRead = 0x20;
+
+// One workgroup tile of C = op(A) op(B) over k in [kb, ke): WM x WN waves of
+// FM x FN MFMA blocks of 16x16.  KFA / KFB: the operand is contiguous along k
+// (A(m, k) at A[k + m lda], B(k, n) at B[k + n ldb]), otherwise along m / n.
+// CA / CB conjugate.  VEC: 16-byte loads, which need the contiguous dimension
+// to hold at least one chunk (any alignment); otherwise element loads.
+//
+// A k-tile is 128 bytes deep: eight chunks of VE values.  In LDS a k-contiguous
+// operand is one 128-byte row per m (n), chunk c of row r at position
+// c ^ (r % 8), so that the sixteen rows of a fragment read hit all banks; the
+// other kind is one row of m (n) per k, padded by a chunk.  Lane (li, lk) =
+// (lane % 16, lane / 16) holds, for MFMA e of half j, the value at
+// k = (lk + 4j) VE + e: which four k an MFMA sums does not depend on the tile
+// or on the operand's storage, so results depend on neither.  Real products
+// add the two halves of every k-tile in accumulators of their own (CH = 2):
+// two chains of half the length lose less to rounding (the split's
+// first-order steps, which stop at 1e-14 |rho|, took 385 steps over 16 sweeps
+// at chi = 256 against 737 with one chain).  An operand that
+// is contiguous along m is read RV values of m at a time: MFMA block i of the
+// wave then holds rows (i / RV) 16 RV + RV li + i % RV (row_of).
+template <class T, bool CA, bool CB, bool KFA, bool KFB, int FM, int FN, int WM, int WN, bool VEC,
+          int CH = GT<T>::P == 1 ? 2 : 1>
+struct TileLoop {
+  using V4 = typename GT<T>::V4;
+  static constexpr int P = GT<T>::P, VE = 16 / sizeof(T), BK = 8 * VE;
+  static constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN, NT = 64 * WM * WN;
+  static constexpr int RVA = FM % VE == 0 ? VE : (FM % 2 == 0 && VE >= 2 ? 2 : 1);
+  static constexpr int RVB = FN % VE == 0 ? VE : (FN % 2 == 0 && VE >= 2 ? 2 : 1);
+  static constexpr int NCA = BM * 8, NCB = BN * 8;  // chunks of one tile in memory
+  static constexpr int NA = (NCA + NT - 1) / NT, NB = (NCB + NT - 1) / NT;
+  // LDS chunks of one tile; every thread stores all its chunks, those past the
+  // tile behind it
+  static constexpr int SA = KFA ? NA * NT : BK * (BM / VE + 1);
+  static constexpr int SB = KFB ? NB * NT : BK * (BN / VE + 1);
+  static_assert((KFA || NCA % NT == 0) && (KFB || NCB % NT == 0), "chunks per thread");
+  static constexpr int SMEM = 2 * (SA + SB);  // chunks of LDS
+  using Acc = V4[P][FM][FN];
+  struct Chunk { T v[VE]; };
+
+  // row (column) of the wave's sub-tile that MFMA block i holds at lane index l
+  __device__ static int row_of(bool kf, int rv, int i, int l) {
+    return kf ? i * 16 + l : (i / rv) * 16 * rv + rv * l + i % rv;
+  }
+
+  // chunk c of an operand tile at (r0, k0); every address is in bounds
+  template <bool KF, int ROWS>
+  __device__ static u4_t load_chunk(const T* __restrict__ X, long long ld, int r0, int nr, int K,
+                                    int k0, int c) {
+    constexpr int NCH = KF ? 8 : ROWS / VE;
+    const int lo = c % NCH, hi = c / NCH;
+    const int x = (KF ? k0 : r0) + lo * VE, nx = KF ? K : nr;  // along the contiguous dimension
+    const int y = min((KF ? r0 : k0) + hi, (KF ? nr : K) - 1);
+    const T* p = X + (long long)y * ld;
+    Chunk v;
+    if constexpr (VEC) {
+      __builtin_memcpy(&v, p + min(x, nx - VE), 16);
+    } else {
+#pragma unroll
+      for (int q = 0; q < VE; ++q) v.v[q] = p[min(x + q, nx - 1)];
+    }
+    u4_t u;
+    __builtin_memcpy(&u, &v, 16);
+    return u;
+  }
+  // the chunk with values past the end of k zeroed, and those of a chunk that
+  // was moved back into its row moved to their places
+  template <bool KF, int ROWS>
+  __device__ static u4_t mask_chunk(u4_t u, int r0, int nr, int K, int k0, int c) {
+    constexpr int NCH = KF ? 8 : ROWS / VE;
+    const int lo = c % NCH, hi = c / NCH;
+    const int x = (KF ? k0 : r0) + lo * VE, nx = KF ? K : nr;
+    const int back = VEC ? x - min(x, nx - VE) : 0;
+    const bool in_k = KF || k0 + hi < K;
+    Chunk v, w;
+    __builtin_memcpy(&v, &u, 16);
+#pragma unroll
+    for (int q = 0; q < VE; ++q) {
+      T y = v.v[q];
+#pragma unroll
+      for (int z = 1; z + q < VE; ++z) y = back == z ? v.v[q + z] : y;
+      w.v[q] = (KF ? x + q < K : in_k) ? y : T(0);
+    }
+    __builtin_memcpy(&u, &w, 16);
+    return u;
+  }
+  template <bool KF, int ROWS>
+  __device__ static int slot_of(int c) {
+    if constexpr (KF) return (c & ~7) | ((c ^ (c >> 3)) & 7);
+    else return (c / (ROWS / VE)) * (ROWS / VE + 1) + c % (ROWS / VE);
+  }
+  template <bool CJ>
+  __device__ static u4_t conj_chunk(u4_t u) {
+    if constexpr (CJ && P == 2) u[3] ^= 0x80000000u;
+    return u;
+  }
+  // fragments of half j of the tile in S, rows w0 .. w0 + 16 F
+  template <bool KF, int F, int RV, int ROWS>
+  __device__ static void read_frag(const u4_t* S, int w0, int j, int li, int lk, T (&f)[F][VE]) {
+    if constexpr (KF) {
+      const u4_t* p = S + (w0 + li) * 8 + ((lk + 4 * j) ^ (li & 7));
+#pragma unroll
+      for (int i = 0; i < F; ++i) {
+        const u4_t u = p[16 * 8 * i];
+        __builtin_memcpy(&f[i][0], &u, 16);
+      }
+    } else {
+      const T* Sp = reinterpret_cast<const T*>(S) + w0 + RV * li;
+#pragma unroll
+      for (int e = 0; e < VE; ++e)
+#pragma unroll
+        for (int i = 0; i < F; i += RV) {
+          T v[RV];
+          __builtin_memcpy(v, __builtin_assume_aligned(
+                                  Sp + ((lk + 4 * j) * VE + e) * (ROWS + VE) + 16 * i,
+                                  RV * sizeof(T)), RV * sizeof(T));
+#pragma unroll
+          for (int q = 0; q < RV; ++q) f[i + q][e] = v[q];
+        }
+    }
+  }
+
+  // M, N, K: extents of the operands (K of the whole product: the last slice
+  // ends there); the slice starts at a multiple of BK.  Returns with every
+  // wave past its last LDS read (a barrier).
+  __device__ static void run(u4_t* smem, int M, int N, int K, int kb, int ke, int m0, int n0,
+                             const T* __restrict__ A, long long lda, const T* __restrict__ B,
+                             long long ldb, Acc& acc) {
+    u4_t(*As)[SA] = reinterpret_cast<u4_t(*)[SA]>(smem);
+    u4_t(*Bs)[SB] = reinterpret_cast<u4_t(*)[SB]>(smem + 2 * SA);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wm = wave % WM, wn = wave / WM;
+    const int li = lane & 15, lk = lane >> 4;
+    u4_t ra[2][NA], rb[2][NB];  // two tiles in flight
+    auto load = [&](int s, int k0) {
+#pragma unroll
+      for (int r = 0; r < NA; ++r)
+        ra[s][r] = load_chunk<KFA, BM>(A, lda, m0, M, K, k0, NCA % NT ? min(t + r * NT, NCA - 1) : t + r * NT);
+#pragma unroll
+      for (int r = 0; r < NB; ++r)
+        rb[s][r] = load_chunk<KFB, BN>(B, ldb, n0, N, K, k0, NCB % NT ? min(t + r * NT, NCB - 1) : t + r * NT);
+    };
+    auto store = [&](auto masked, int s, int k0, int buf) {
+#pragma unroll
+      for (int r = 0; r < NA; ++r) {
+        const int c = t + r * NT;
+        u4_t u = ra[s][r];
+        if constexpr (decltype(masked)::value) u = mask_chunk<KFA, BM>(u, m0, M, K, k0, c);
+        As[buf][slot_of<KFA, BM>(c)] = conj_chunk<CA>(u);
+      }
+#pragma unroll
+      for (int r = 0; r < NB; ++r) {
+        const int c = t + r * NT;
+        u4_t u = rb[s][r];
+        if constexpr (decltype(masked)::value) u = mask_chunk<KFB, BN>(u, n0, N, K, k0, c);
+        Bs[buf][slot_of<KFB, BN>(c)] = conj_chunk<CB>(u);
+      }
+    };
+    T fa[2][FM][VE], fb[2][FN][VE];
+    auto read = [&](int slot, int buf, int j) {
+      read_frag<KFA, FM, RVA, BM>(As[buf], wm * 16 * FM, j, li, lk, fa[slot]);
+      read_frag<KFB, FN, RVB, BN>(Bs[buf], wn * 16 * FN, j, li, lk, fb[slot]);
+    };
+    V4 sum[CH][P][FM][FN];
+    auto mul = [&](int slot) {
+      auto& acc = sum[CH == 2 ? slot : 0];
+#pragma unroll
+      for (int e = 0; e < VE; ++e)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int n = 0; n < FN; ++n) {
+            const T a = fa[slot][i][e], b = fb[slot][n][e];
+            if constexpr (P == 1) {
+              acc[0][i][n] = mfma(b, a, acc[0][i][n]);
+            } else {
+              acc[0][i][n] = mfma(b.x, a.x, acc[0][i][n]);
+              acc[1][i][n] = mfma(b.y, a.x, acc[1][i][n]);
+              acc[0][i][n] = mfma(-b.y, a.y, acc[0][i][n]);
+              acc[1][i][n] = mfma(b.x, a.y, acc[1][i][n]);
+            }
+          }
+    };
+    // instructions of one half tile; FP32 is left to the compiler's own order
+    // (measured: 55 us against 60 for 2560x2048x512)
+    constexpr bool ORD = !std::is_same<T, float>::value;
+    constexpr int MH = VE * FM * FN * (P == 2 ? 4 : 1);
+    constexpr int NR = (KFA ? FM : VE * FM / RVA) + (KFB ? FN : VE * FN / RVB);
+    constexpr int NL = (VEC ? 1 : VE) * (NA + NB);
+    const int nk = (ke - kb + BK - 1) / BK;
+    const int kl = kb + (nk - 1) * BK;  // last tile: later ones load it again, unused
+    // Tile kt: its fragments are read half by half; tile kt + 1 goes to the
+    // other LDS buffer, and the registers it leaves are loaded with kt + 3.
+    auto body = [&](auto masked, auto uc, int kt) {
+      constexpr int u = decltype(uc)::value;
+      const int k0 = kb + kt * BK;
+      read(1, u, 1);
+      store(masked, u ^ 1, min(k0 + BK, kl), u ^ 1);
+      mul(0);
+      if constexpr (ORD) {
+        interleave<0, MH, NR, kSchedDsWrite, NA + NB, false>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+      read(0, u ^ 1, 0);
+      mul(1);
+      load(u ^ 1, min(k0 + 3 * BK, kl));
+      if constexpr (ORD) {
+        interleave<0, MH, NR, kSchedVmemRead, NL, true>();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int n = 0; n < FN; ++n) sum[c][p][i][n] = V4{0, 0, 0, 0};
+    std::integral_constant<int, 0> u0;
+    std::integral_constant<int, 1> u1;
+    load(0, kb);
+    load(1, min(kb + BK, kl));
+    store(std::true_type{}, 0, kb, 0);
+    load(0, min(kb + 2 * BK, kl));
+    __syncthreads();
+    read(0, 0, 0);
+    // tiles whose successor is neither the last one nor at an edge
+    const bool edge = (!KFA && m0 + BM > M) || (!KFB && n0 + BN > N);
+    const int free = edge ? 0 : nk - 2;
+    int kt = 0;
+    for (; kt + 2 <= free; kt += 2) {
+      body(std::false_type{}, u0, kt);
+      body(std::false_type{}, u1, kt + 1);
+    }
+    for (; kt + 2 <= nk; kt += 2) {
+      body(std::true_type{}, u0, kt);
+      body(std::true_type{}, u1, kt + 1);
+    }
+    if (kt < nk) body(std::true_type{}, u0, kt);
+    __syncthreads();  // the last body read ahead
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int n = 0; n < FN; ++n) {
+          acc[p][i][n] = sum[0][p][i][n];
+          if constexpr (CH == 2) acc[p][i][n] += sum[CH - 1][p][i][n];
+        }
+  }
+};
+
+// C = alpha op(A) op(B) + beta C (plain operands).  Block z of the grid takes
+// the k-slice [z Kc, z Kc + Kc) into C + z sC.  herm: a Hermitian product
+// (M == N, BM == BN, beta == 0): only tiles on and above the diagonal are
+// computed, each writes its conjugate mirror too.
+template <class T, bool CA, bool CB, bool KFA, bool KFB, int FM, int FN, bool VEC>
+__global__ __launch_bounds__(256) void k_tile(int M, int N, int K, int Kc, T alpha,
+                                              const T* __restrict__ A, long long lda,
+                                              const T* __restrict__ B, long long ldb, T beta,
+                                              T* __restrict__ C, long long ldc, long long sC,
+                                              int herm) {
+  using TL = TileLoop<T, CA, CB, KFA, KFB, FM, FN, 2, 2, VEC>;
+  __shared__ u4_t smem[TL::SMEM];
+  if (herm && blockIdx.x > blockIdx.y) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave & 1, wn = wave >> 1;
+  const int m0 = blockIdx.x * TL::BM, n0 = blockIdx.y * TL::BN;
+  const int kb = blockIdx.z * Kc, ke = min(K, kb + Kc);
+  typename TL::Acc acc;
+  TL::run(smem, M, N, K, kb, ke, m0, n0, A, lda, B, ldb, acc);
+  C += blockIdx.z * sC;
+  const int li = lane & 15, lk = lane >> 4;
+  const bool use_beta = !(real(beta) == 0.0 && imag(beta) == 0.0);
+  // lane -> row of C, register r -> column lk + 4r (f64) or 4 lk + r (f32)
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int n = 0; n < FN; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gm = m0 + wm * 16 * FM + TL::row_of(KFA, TL::RVA, i, li);
+        const int gn = n0 + wn * 16 * FN +
+                       TL::row_of(KFB, TL::RVB, n, GT<T>::G1 ? lk + 4 * r : 4 * lk + r);
+        if (gm < M && gn < N) {
+          T v;
+          if constexpr (TL::P == 1) v = T(acc[0][i][n][r]);
+          else v = make_scalar<T>(acc[0][i][n][r], acc[1][i][n][r]);
+          v = alpha * v;
+          const long long idx = gm + (long long)gn * ldc;
+          if (use_beta) v = v + beta * C[idx];
+          C[idx] = v;
+          if (herm && blockIdx.x != blockIdx.y) C[gn + (long long)gm * ldc] = conj_v(v);
+        }
+      }
+}
+
+// ---------------------------------------------------------------------------
+// Two-level operands (gemm_tensor).
+// Workgroup: 256 threads = 4 wave64s in a 2x2 grid, each owning a
+// (BM/2) x (BN/2) sub-tile of 16x16 MFMA blocks; operand tiles of depth BK are
+// staged through LDS (double buffered, one-element row padding), with the
+// global loads of the next PF tiles issued before the MFMAs of the current one.
+// ---------------------------------------------------------------------------
+template <class T, int BM, int BN, int BK>
+__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, T alpha,
+                                              const T* __restrict__ A, AddrTensor aa,
+                                              const T* __restrict__ B, AddrTensor ab, T beta,
+                                              T* __restrict__ C, AddrTensor ac) {
   using E = typename GT<T>::E;
   using V4 = typename GT<T>::V4;
   constexpr int P = GT<T>::P;
-  constexpr int NT = 256 * KS;
+  constexpr int NT = 256, PF = 2;
   constexpr int PADM = BM + 1, PADN = BN + 1;
   constexpr int FM = BM / 32, FN = BN / 32;  // 16x16 blocks per wave
   constexpr int NA = BM * BK / NT, NB = BN * BK / NT;
-  static_assert(KS == 1 || KS == 2, "k split");
-  static_assert(NA >= 1 && NB >= 1 && BK % (4 * KS) == 0, "tile too small for the k split");
 
   __shared__ E As[2][P][BK][PADM];
   __shared__ E Bs[2][P][BK][PADN];
-  __shared__ E Red[KS > 1 ? 4 * P * FM * FN * 4 * 64 : 1];
 
-  // Hermitian product (M == N, BM == BN, beta == 0): only the tiles on and
-  // above the diagonal are computed; each writes its conjugate mirror too.
-  if (herm && blockIdx.x > blockIdx.y) return;
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
-  const int wm = wave & 1, wn = (wave >> 1) & 1, wk = wave >> 2;
+  const int wm = wave & 1, wn = wave >> 1;
   const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  A += blockIdx.z * sA;
-  B += blockIdx.z * sB;
-  C += blockIdx.z * sC;
 
-  static_assert(PF >= 1 && PF <= 4, "prefetch depth");
   T ra[PF][NA], rb[PF][NB];
 
   auto idxA = [&](int r, int& m, int& k) {
-    if (!KFA) { m = t % BM; k = t / BM + r * (NT / BM); }
-    else      { k = t % BK; m = t / BK + r * (NT / BK); }
+    m = t % BM;
+    k = t / BM + r * (NT / BM);
   };
   auto idxB = [&](int r, int& n, int& k) {
-    if (!KFB) { n = t % BN; k = t / BN + r * (NT / BN); }
-    else      { k = t % BK; n = t / BK + r * (NT / BK); }
+    k = t % BK;
+    n = t / BK + r * (NT / BK);
   };
   // register stage `s` <- operand tiles at depth k0; a tile inside all three
   // bounds loads without per-element checks (one branch for the whole stage)
@@ -120,15 +435,13 @@ __global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
       for (int r = 0; r < NA; ++r) {
         int m, k;
         idxA(r, m, k);
-        const T v = A[aa(m0 + m, k0 + k)];
-        ra[s][r] = CA ? conj_v(v) : v;
+        ra[s][r] = A[aa(m0 + m, k0 + k)];
       }
 #pragma unroll
       for (int r = 0; r < NB; ++r) {
         int n, k;
         idxB(r, n, k);
-        const T v = B[ab(k0 + k, n0 + n)];
-        rb[s][r] = CB ? conj_v(v) : v;
+        rb[s][r] = B[ab(k0 + k, n0 + n)];
       }
       return;
     }
@@ -137,18 +450,14 @@ __global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
       int m, k;
       idxA(r, m, k);
       int gm = m0 + m, gk = k0 + k;
-      T v = T(0);
-      if (gm < M && gk < K) v = A[aa(gm, gk)];
-      ra[s][r] = CA ? conj_v(v) : v;
+      ra[s][r] = (gm < M && gk < K) ? A[aa(gm, gk)] : T(0);
     }
 #pragma unroll
     for (int r = 0; r < NB; ++r) {
       int n, k;
       idxB(r, n, k);
       int gn = n0 + n, gk = k0 + k;
-      T v = T(0);
-      if (gn < N && gk < K) v = B[ab(gk, gn)];
-      rb[s][r] = CB ? conj_v(v) : v;
+      rb[s][r] = (gn < N && gk < K) ? B[ab(gk, gn)] : T(0);
     }
   };
   // LDS buffer `buf` <- register stage `s`
@@ -185,7 +494,7 @@ __global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
   const int li = lane & 15, lk = lane >> 4;
   auto compute = [&](int buf) {
 #pragma unroll
-    for (int kk = wk * (BK / KS); kk < (wk + 1) * (BK / KS); kk += 4) {
+    for (int kk = 0; kk < BK; kk += 4) {
       E af[P][FM], bf[P][FN];
 #pragma unroll
       for (int p = 0; p < P; ++p) {
@@ -233,31 +542,6 @@ __global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
     }
   }
 
-  if constexpr (KS > 1) {
-    // the second k-half's partial sums join the first's (the loop ended at
-    // a barrier, so no wave reads As/Bs any more)
-    E* red = Red + (size_t)(wave & 3) * (P * FM * FN * 4 * 64);
-    if (wk == 1) {
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-          for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) red[(((p * FM + i) * FN + j) * 4 + r) * 64 + lane] = acc[p][i][j][r];
-    }
-    __syncthreads();
-    if (wk == 1) return;
-#pragma unroll
-    for (int p = 0; p < P; ++p)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[p][i][j][r] += red[(((p * FM + i) * FN + j) * 4 + r) * 64 + lane];
-  }
   // Epilogue: lane -> row li of C; register r -> column lk + 4r (f64) or
   // 4*lk + r (f32) of each 16x16 block.
   const bool use_beta = !(real(beta) == 0.0 && imag(beta) == 0.0);
@@ -277,61 +561,49 @@ __global__ __launch_bounds__(256 * KS) void k_gemm(int M, int N, int K, T alpha,
           long long idx = ac(gm, gn);
           if (use_beta) v = v + beta * C[idx];
           C[idx] = v;
-          if (herm && blockIdx.x != blockIdx.y) C[ac(gn, gm)] = conj_v(v);
         }
       }
 }
 
-template <class T, bool CA, bool CB, bool KFA, bool KFB, class AA, class AB, class AC>
-void launch(hipStream_t st, GemmTile tl, int M, int N, int K, T alpha, const T* A, AA aa,
-            long long sA, const T* B, AB ab, long long sB, T beta, T* C, AC ac, long long sC,
-            int batch, int herm = 0) {
-#define DMRG_GEMM_LAUNCH(BM_, BN_, BK_, PF_)                                                \
-  if (tl.ks == 2)                                                                          \
-    hipLaunchKernelGGL((k_gemm<T, CA, CB, KFA, KFB, BM_, BN_, BK_, PF_, 2, AA, AB, AC>),    \
-                       dim3(cdiv(M, BM_), cdiv(N, BN_), batch), dim3(512), 0, st, M, N, K,  \
-                       alpha, A, aa, sA, B, ab, sB, beta, C, ac, sC, herm);                 \
-  else                                                                                     \
-    hipLaunchKernelGGL((k_gemm<T, CA, CB, KFA, KFB, BM_, BN_, BK_, PF_, 1, AA, AB, AC>),    \
-                       dim3(cdiv(M, BM_), cdiv(N, BN_), batch), dim3(256), 0, st, M, N, K,  \
-                       alpha, A, aa, sA, B, ab, sB, beta, C, ac, sC, herm)
-  // 32x32 tiles serve grids that cannot fill the chip with 64x64 ones; a deep
-  // k-step and two register stages then hide the load latency that the low
-  // tile count per CU leaves exposed.
-  // 64x64 tiles: two register stages as well (measured on the H_eff shapes:
-  // FP64 +12-15 % with BK=16, FP32 +5-26 % with BK=32).  Complex: BK=16 and
-  // two stages for both tiles (+4-13 % on the C3 shapes; four MFMAs per k-step).
-  if (tl.bm == 32 && tl.bn == 32) {
-    if constexpr (is_cplx<T>::value) DMRG_GEMM_LAUNCH(32, 32, 16, 2);
-    else DMRG_GEMM_LAUNCH(32, 32, 32, 2);
-  } else {
-    if constexpr (is_cplx<T>::value) DMRG_GEMM_LAUNCH(64, 64, 16, 2);
-    else if constexpr (std::is_same<T, float>::value) DMRG_GEMM_LAUNCH(64, 64, 32, 2);
-    else DMRG_GEMM_LAUNCH(64, 64, 16, 2);
+
+// One launch: `slices` slices of Kc (a multiple of the k-tile depth when there
+// is more than one).
+template <class T, bool CA, bool CB, bool KFA, bool KFB>
+void launch(hipStream_t st, GemmTile tl, int M, int N, int K, int Kc, int slices, T alpha,
+            const T* A, int lda, const T* B, int ldb, T beta, T* C, int ldc, long long sC,
+            int herm) {
+#define DMRG_TILE(FM_, FN_, VEC_)                                                              \
+  hipLaunchKernelGGL((k_tile<T, CA, CB, KFA, KFB, FM_, FN_, VEC_>),                            \
+                     dim3(cdiv(M, 32 * FM_), cdiv(N, 32 * FN_), slices), dim3(256), 0, st, M, N, \
+                     K, Kc, alpha, A, (long long)lda, B, (long long)ldb, beta, C,              \
+                     (long long)ldc, sC, herm)
+  // 16-byte loads need one whole chunk along each operand's contiguous
+  // dimension (2 FP64, 4 FP32, 1 complex128 value); the products that do not
+  // have it, at the ends of a chain, are tiny
+  constexpr int VE = 16 / (int)sizeof(T);
+  if constexpr (VE > 1) {
+    if ((KFA ? K : M) < VE || (KFB ? K : N) < VE) {
+      DMRG_TILE(1, 1, false);
+      DMRG_LAUNCH_CHECK();
+      return;
+    }
   }
-#undef DMRG_GEMM_LAUNCH
+  if (tl.bm == 32) DMRG_TILE(1, 1, true);
+  else if (tl.bn == 32) DMRG_TILE(2, 1, true);
+  else DMRG_TILE(2, 2, true);
+#undef DMRG_TILE
   DMRG_LAUNCH_CHECK();
 }
 
-template <class T, bool TA, bool TB, bool CA, bool CB>
-void plain4(hipStream_t st, GemmTile tl, int M, int N, int K, T alpha, const T* A, int lda,
-            long long sA, const T* B, int ldb, long long sB, T beta, T* C, int ldc, long long sC,
-            int batch, int herm) {
-  launch<T, CA, CB, TA, !TB>(st, tl, M, N, K, alpha, A, AddrPlain<TA>{lda}, sA, B,
-                             AddrPlain<TB>{ldb}, sB, beta, C, AddrPlain<false>{ldc}, sC, batch,
-                             herm);
-}
-
 template <class T>
-void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K, T alpha,
-              const T* A, int lda, long long sA, const T* B, int ldb, long long sB, T beta, T* C,
-              int ldc, long long sC, int batch, int herm) {
+void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K, int Kc,
+              int slices, T alpha, const T* A, int lda, const T* B, int ldb, T beta, T* C, int ldc,
+              long long sC, int herm) {
   const bool ta = op_trans(opA), tb = op_trans(opB);
   bool ca = op_conj(opA), cb = op_conj(opB);
   if (!is_cplx<T>::value) ca = cb = false;
 #define DMRG_P4(TA_, TB_, CA_, CB_) \
-  plain4<T, TA_, TB_, CA_, CB_>(st, tl, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, \
-                                batch, herm)
+  launch<T, CA_, CB_, TA_, !TB_>(st, tl, M, N, K, Kc, slices, alpha, A, lda, B, ldb, beta, C, ldc, sC, herm)
   if (!ca && !cb) {
     if (!ta && !tb) DMRG_P4(false, false, false, false);
     else if (!ta && tb) DMRG_P4(false, true, false, false);
@@ -361,9 +633,8 @@ void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K
 
 // ---------------------------------------------------------------------------
 // Tile autotuner.  When enabled (gemm_autotune), the first non-batched call
-// of each (scalar type, ops, M, N, K, Hermitian) shape whose caller tile has
-// one wave per output sub-tile times the 32x32 and 64x64 tiles on the
-// caller's stream, with the device otherwise idle (one warm-up each, then
+// of each (scalar type, ops, M, N, K, Hermitian) shape times the 32x32, 64x32
+// (not for a Hermitian product) and 64x64 tiles on the caller's stream, with the device otherwise idle (one warm-up each, then
 // four interleaved rounds of one launch each into a scratch output, keeping
 // each tile's fastest), and keeps the fastest for the rest of the process --
 // the caller's tile unless the other is at least 3 % faster; later calls of
@@ -406,11 +677,8 @@ template <class T> constexpr int dt_code() { return is_cplx<T>::value ? 1 : (std
 template <class T>
 GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K,
                     const T* A, int lda, const T* B, int ldb, int herm) {
-  // Only tiles that sum over k in the caller's order are candidates, so the
-  // choice never changes a result: with one wave per output sub-tile every
-  // tile size accumulates k in the same sequence; an eight-wave (k-split)
-  // tile's order depends on its k-tile, so a k-split caller tile stands.
-  if (tl.ks != 1) return tl;
+  // Every tile accumulates k in the same sequence, so the choice never changes
+  // a result.
   const TuneKey key{dt_code<T>(), opA, opB, M, N, K, herm};
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune.find(key);
@@ -433,23 +701,24 @@ GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N,
   hipEvent_t e0, e1;
   DMRG_HIP(hipEventCreate(&e0));
   DMRG_HIP(hipEventCreate(&e1));
-  constexpr int NC = 2, ROUNDS = 4;
-  const GemmTile cand[NC] = {{32, 32, 1}, {64, 64, 1}};
-  float t_min[NC];
+  constexpr int ROUNDS = 4;
+  const GemmTile cand[3] = {{32, 32}, {64, 64}, {64, 32}};
+  const int NC = herm ? 2 : 3;
+  float t_min[3] = {0.f, 0.f, 0.f};
   GemmTile best = tl;
   float best_ms = 1e30f;
   try {
     // Time on an idle device: other streams' work (the environment updates
     // that overlap a bond) would otherwise bias whichever candidate it meets.
     DMRG_HIP(hipDeviceSynchronize());
-    for (const GemmTile& c : cand)  // warm-up: code and operands into the caches
-      dispatch<T>(st, opA, opB, c, M, N, K, T(1), A, lda, 0, B, ldb, 0, T(0), Cs, M, 0, 1, herm);
+    for (int c = 0; c < NC; ++c)  // warm-up: code and operands into the caches
+      dispatch<T>(st, opA, opB, cand[c], M, N, K, K, 1, T(1), A, lda, B, ldb, T(0), Cs, M, 0, herm);
     // Rounds interleave the candidates, and each keeps its fastest launch,
     // so work that other streams run meanwhile biases no candidate.
     for (int r = 0; r < ROUNDS; ++r)
       for (int c = 0; c < NC; ++c) {
         DMRG_HIP(hipEventRecord(e0, st));
-        dispatch<T>(st, opA, opB, cand[c], M, N, K, T(1), A, lda, 0, B, ldb, 0, T(0), Cs, M, 0, 1,
+        dispatch<T>(st, opA, opB, cand[c], M, N, K, K, 1, T(1), A, lda, B, ldb, T(0), Cs, M, 0,
                     herm);
         DMRG_HIP(hipEventRecord(e1, st));
         DMRG_HIP(hipEventSynchronize(e1));
@@ -459,7 +728,7 @@ GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N,
       }
     // the caller's tile stands unless another is at least 3 % faster
     for (int c = 0; c < NC; ++c)
-      if (cand[c].bm == tl.bm && cand[c].bn == tl.bn && cand[c].ks == tl.ks) best_ms = t_min[c];
+      if (cand[c].bm == tl.bm && cand[c].bn == tl.bn) best_ms = t_min[c];
     for (int c = 0; c < NC; ++c)
       if (t_min[c] < 0.97f * best_ms) {
         best_ms = t_min[c];
@@ -467,10 +736,10 @@ GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N,
       }
     if (g_tune_log)
       std::fprintf(stderr,
-                   "[gemm autotune] dt %d op %d%d%s M %d N %d K %d: 32x32 %.1f, 64x64 %.1f us -> "
-                   "%dx%d\n",
+                   "[gemm autotune] dt %d op %d%d%s M %d N %d K %d: 32x32 %.1f, 64x64 %.1f, "
+                   "64x32 %.1f us -> %dx%d\n",
                    key.dt, opA, opB, herm ? " herm" : "", M, N, K, 1e3f * t_min[0],
-                   1e3f * t_min[1], best.bm, best.bn);
+                   1e3f * t_min[1], 1e3f * t_min[2], best.bm, best.bn);
   } catch (...) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -484,15 +753,14 @@ GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N,
 
 template <class T>
 void plain(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K, T alpha, const T* A,
-           int lda, long long sA, const T* B, int ldb, long long sB, T beta, T* C, int ldc,
-           long long sC, int batch, int herm = 0) {
-  DMRG_REQUIRE(M >= 0 && N >= 0 && K >= 0 && batch >= 0, "gemm: negative size");
+           int lda, const T* B, int ldb, T beta, T* C, int ldc, int herm) {
+  DMRG_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm: negative size");
   DMRG_REQUIRE(opA >= 0 && opA <= 3 && opB >= 0 && opB <= 3, "gemm: bad op");
-  if (M == 0 || N == 0 || batch == 0) return;
-  if (batch == 1 && g_tune_on.load(std::memory_order_relaxed))
+  if (M == 0 || N == 0) return;
+  DMRG_REQUIRE(K >= 1, "gemm: empty sum");
+  if (g_tune_on.load(std::memory_order_relaxed))
     tl = tuned_tile<T>(st, opA, opB, tl, M, N, K, A, lda, B, ldb, herm);
-  dispatch<T>(st, opA, opB, tl, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
-              herm);
+  dispatch<T>(st, opA, opB, tl, M, N, K, K, 1, alpha, A, lda, B, ldb, beta, C, ldc, 0, herm);
 }
 
 }  // namespace
@@ -503,17 +771,46 @@ int gemm_autotune_entries() {
   return (int)g_tune.size();
 }
 
+namespace {
+// Cycles (at 2.1 GHz) of one k-tile on a CU that holds w workgroups of the
+// grid, from FP64 products with K = 1024 and 8192 (MFMA alone: 1024, 512 and
+// 256 cycles per workgroup).  A single workgroup is bound by its own chain of
+// barrier and LDS reads, several by the MFMAs and, for the small tiles, by the
+// lower clock that their operand traffic leaves.  Complex k-tiles hold the same
+// bytes and twice the MFMAs; their 64x64 tile fits fewer workgroups on a CU
+// (1280^3: 310 us against 294 with 32x32).
+double tile_cycles(const GemmTile& t, int w, bool cplx) {
+  if (cplx) return 2.0 * w * (t.bm == 32 ? 320.0 : t.bn == 32 ? 600.0 : 1180.0);
+  if (t.bm == 32) return std::max(430.0, 332.0 * w);
+  if (t.bn == 32) return std::max(620.0, 610.0 * w);
+  return std::max(1250.0, 1050.0 * w);
+}
+constexpr int kCUs = 256;
+inline int per_cu(const GemmTile& t, int M, int N, int slices) {
+  const long long tiles = (long long)cdiv(M, t.bm) * cdiv(N, t.bn) * slices;
+  return (int)((tiles + kCUs - 1) / kCUs);
+}
+GemmTile pick_square(int N, bool cplx) {
+  const GemmTile a{32, 32}, b{64, 64};
+  return tile_cycles(a, per_cu(a, N, N, 1), cplx) < tile_cycles(b, per_cu(b, N, N, 1), cplx) ? a : b;
+}
+}  // namespace
+
+// The tile with the fewest modelled cycles; they agree with the measured order
+// on the sweep's shapes (us for 64x64, 64x32, 32x32: 1024^3 44, 43, 46;
+// 512^3 21, 12.5, 9.3; 1280x1024x256 24, 19, 17; 2560x2048x512 98, 105, 109).
 GemmTile gemm_pick_tile(int M, int N, int K, bool complex_) {
   (void)K;
-  const long long t64 = (long long)cdiv(M, 64) * cdiv(N, 64);
-  const long long t32 = (long long)cdiv(M, 32) * cdiv(N, 32);
-  // 64x64 once there are about four tiles per CU (256 CUs); complex too
-  // (measured at 1280^3: 32x32 with two stages 53.8 TF/s, 64x64 48.3).
-  // At most one 32x32 tile per CU: eight waves splitting every k-tile
-  // (512^3: 24.5 TF/s against 21.3 with four waves).
-  (void)complex_;
-  if (t64 >= 1024) return {64, 64, 1};
-  return {32, 32, t32 <= 256 ? 2 : 1};
+  GemmTile best{64, 64};
+  double c = tile_cycles(best, per_cu(best, M, N, 1), complex_);
+  for (const GemmTile t : {GemmTile{64, 32}, GemmTile{32, 32}}) {
+    const double ct = tile_cycles(t, per_cu(t, M, N, 1), complex_);
+    if (ct < c) {
+      c = ct;
+      best = t;
+    }
+  }
+  return best;
 }
 
 namespace {
@@ -753,24 +1050,44 @@ __global__ void k_splitk_sum(const T* __restrict__ W, int S, long long stride, i
 }
 
 template <class T, class TO>
-bool splitk_impl(hipStream_t st, int M, int N, int K, const T* A, int lda, const T* B, int ldb,
-                 TO* C, int ldc, T* ws, size_t ws_elems, const double* s1, const double* s2) {
-  // S equal slices (S | K) in one batched launch, while the 64x64 grid
-  // leaves CUs idle and each slice keeps K/S >= 512.  FP32 (BK = 32 tiles)
-  // stops at two slices: measured 80 TF/s against 74 for four on the C4
-  // out-step (2048 x 512 x 2560); FP64 (BK = 16) is best at four.
-  const int smax = std::is_same<T, float>::value ? 2 : 8;
-  const long long t64 = (long long)cdiv(M, 64) * cdiv(N, 64);
+bool splitk_impl(hipStream_t st, int opA, int opB, int M, int N, int K, const T* A, int lda,
+                 const T* B, int ldb, TO* C, int ldc, T* ws, size_t ws_elems, const double* s1,
+                 const double* s2) {
+  // Slices of whole k-tiles in one launch.  The number of slices and the tile
+  // are those with the fewest modelled cycles: the k-tiles of one slice, the
+  // start and end of a workgroup, and the pass that sums the partial products
+  // (5.5 TB/s and 2 us for its launch; 2048 x 512 x 2560 in FP64: one slice 108
+  // us, two 93 + 6, four 88 + 9).
+  constexpr int BK = 128 / (int)sizeof(T);
+  const int nkt = (int)cdiv(K, BK);
+  const GemmTile tiles[3] = {{64, 64}, {64, 32}, {32, 32}};
+  GemmTile tile{64, 64};
   int S = 1;
-  while (S < smax && t64 * S * 2 <= 1024 && K % (S * 2) == 0 && K / (S * 2) >= 512 &&
-         (size_t)(S * 2) * M * N <= ws_elems)
-    S *= 2;
+  double best = 1e300;
+  bool was_long = false;
+  for (int sl : {1, 2, 3, 4, 6, 8, 12, 16}) {
+    if (sl > 1 && ((size_t)sl * M * N > ws_elems || nkt < 4 * sl)) break;
+    // FP32: a slice sums at most 768 values per accumulator (two per slice)
+    // where the workspace allows it, however many slices are fastest
+    const bool long_sum = std::is_same<T, float>::value && K > 2 * 768 * sl;
+    const double per = (double)cdiv(nkt, sl);
+    const double sum =
+        sl == 1 ? 0.0 : 2.1e9 * (2e-6 + ((double)sl * sizeof(T) + sizeof(TO)) * M * N / 5.5e12);
+    for (const GemmTile& t : tiles) {
+      const double c = (per + 3.0) * tile_cycles(t, per_cu(t, M, N, sl), is_cplx<T>::value) + sum;
+      if (c < best || (was_long && !long_sum)) {
+        best = c;
+        S = sl;
+        tile = t;
+        was_long = long_sum;
+      }
+    }
+  }
   if (S == 1) return false;
-  const int Kc = K / S;
-  // slice z: A(:, z Kc ..) (A + z Kc lda), B(z Kc .., :) (B + z Kc) -> ws + z M N
-  // eight-wave tiles: +11 % (FP64) and +17 % (FP32) on the C4 out-step slices
-  gemm_strided<T>(st, OP_N, OP_N, M, N, Kc, T(1), A, lda, (long long)Kc * lda, B, ldb,
-                  (long long)Kc, T(0), ws, M, (long long)M * N, S, GemmTile{64, 64, 2});
+  const int Kc = (int)cdiv(nkt, S) * BK;
+  S = (int)cdiv(K, Kc);  // no empty slice
+  dispatch<T>(st, opA, opB, tile, M, N, K, Kc, S, T(1), A, lda, B, ldb, T(0), ws, M,
+              (long long)M * N, 0);
   const long long tot = (long long)M * N;
   hipLaunchKernelGGL((k_splitk_sum<T, TO>),
                      dim3((unsigned)std::min<long long>(cdiv(tot, 256), 4096)), dim3(256), 0, st,
@@ -781,15 +1098,17 @@ bool splitk_impl(hipStream_t st, int M, int N, int K, const T* A, int lda, const
 }  // namespace
 
 template <class T>
-bool gemm_nn_splitk(hipStream_t st, int M, int N, int K, const T* A, int lda, const T* B, int ldb,
-                    T* C, int ldc, T* ws, size_t ws_elems) {
-  return splitk_impl<T, T>(st, M, N, K, A, lda, B, ldb, C, ldc, ws, ws_elems, nullptr, nullptr);
+bool gemm_splitk(hipStream_t st, int opA, int opB, int M, int N, int K, const T* A, int lda,
+                 const T* B, int ldb, T* C, int ldc, T* ws, size_t ws_elems) {
+  return splitk_impl<T, T>(st, opA, opB, M, N, K, A, lda, B, ldb, C, ldc, ws, ws_elems, nullptr,
+                           nullptr);
 }
 
 bool gemm_nn_splitk_to_f64(hipStream_t st, int M, int N, int K, const float* A, int lda,
                            const float* B, int ldb, double* C, int ldc, float* ws,
                            size_t ws_elems, const double* s1, const double* s2) {
-  return splitk_impl<float, double>(st, M, N, K, A, lda, B, ldb, C, ldc, ws, ws_elems, s1, s2);
+  return splitk_impl<float, double>(st, OP_N, OP_N, M, N, K, A, lda, B, ldb, C, ldc, ws, ws_elems,
+                                    s1, s2);
 }
 
 namespace {
@@ -797,129 +1116,89 @@ namespace {
 // epilogue (d = 2, real scalars).  The workgroup computes the tile of
 // X = L^T theta with rows (w + D a') for 16 consecutive a' (all D values of w)
 // and columns (ss + 4 b) for 16 consecutive b (all four ss): wave j owns the
-// columns 16 j .. 16 j + 15 and all D row blocks, one 16x16 MFMA block each
-// per 4-deep k step, with the k-loop of k_gemm (two register stages, two LDS
-// buffers).  The finished tile goes to LDS (over the operand buffers, which
-// the k-loop no longer reads), and thread (a', b) contracts its 4D values
-// with WW into the 4D outputs Y[a' + cL ss' + 4 cL b + 4 cL cR n], summing
-// over c = w + D ss in the order of k_rows_small.  X never reaches HBM.
-// theta may be stored in another precision (TB): each element is converted
-// to T on load.
-template <class T, class TB, int D, int BK>
+// columns 16 j .. 16 j + 15, four b, and all D row blocks.  The finished tile
+// changes lanes through LDS inside each wave, and lane (a', b) contracts its
+// 4D values with WW into the 4D outputs Y[a' + cL ss' + 4 cL b + 4 cL cR n],
+// summing over c = w + D ss in order.  WW is the same for every lane and comes
+// through scalar loads.  X never reaches HBM.
+// MFMA-bound; LDS is held to 40 KB for D <= 5, four workgroups a CU: the 1024
+// tiles of cL = cR = 512 are then resident at once.
+template <class T, int D, bool VEC>
 __global__ __launch_bounds__(256) void k_heff2_x_mpo(int cL, int cR, const T* __restrict__ Lenv,
-                                                     const TB* __restrict__ theta,
+                                                     const T* __restrict__ theta,
                                                      const T* __restrict__ WW,
                                                      T* __restrict__ Y) {
-  using V4 = typename GT<T>::V4;
-  constexpr int DD = 4, BM = 16 * D, BN = 16 * DD, K2 = D * DD;
-  constexpr int NA = BM * BK / 256, NB = BN * BK / 256;
-  static_assert(NA * 256 == BM * BK && NB * 256 == BN * BK, "tile");
-  constexpr int OPS = 2 * BK * (BM + 1) + 2 * BK * (BN + 1), XS = BM * (BN + 1);
-  __shared__ T smem[OPS > XS ? OPS : XS];
-  __shared__ T Ws[K2 * K2];
-  T(*As)[BK][BM + 1] = reinterpret_cast<T(*)[BK][BM + 1]>(smem);
-  T(*Bs)[BK][BN + 1] = reinterpret_cast<T(*)[BK][BN + 1]>(smem + 2 * BK * (BM + 1));
-  T(*Xs)[BN + 1] = reinterpret_cast<T(*)[BN + 1]>(smem);
-  const int t = threadIdx.x, lane = t & 63, wn = t >> 6;
-  const int M = D * cL, N = DD * cR, K = cL;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  for (int e = t; e < K2 * K2; e += 256) Ws[e] = WW[e];
-  // A(m, k) = Lenv[k + m cL], B(k, n) = theta[k + n cL]: both k-fast
-  T ra[2][NA], rb[2][NB];
-  const bool inner = m0 + BM <= M && n0 + BN <= N;
-  auto load = [&](int s, int k0) {
-    const bool full = inner && k0 + BK <= K;
-#pragma unroll
-    for (int r = 0; r < NA; ++r) {
-      const int k = t % BK, m = t / BK + r * (256 / BK);
-      const int gm = m0 + m, gk = k0 + k;
-      ra[s][r] = (full || (gm < M && gk < K)) ? Lenv[gk + (size_t)gm * cL] : T(0);
-    }
-#pragma unroll
-    for (int r = 0; r < NB; ++r) {
-      const int k = t % BK, n = t / BK + r * (256 / BK);
-      const int gn = n0 + n, gk = k0 + k;
-      rb[s][r] = (full || (gn < N && gk < K)) ? (T)theta[gk + (size_t)gn * cL] : T(0);
-    }
-  };
-  auto store = [&](int s, int buf) {
-#pragma unroll
-    for (int r = 0; r < NA; ++r) As[buf][t % BK][t / BK + r * (256 / BK)] = ra[s][r];
-#pragma unroll
-    for (int r = 0; r < NB; ++r) Bs[buf][t % BK][t / BK + r * (256 / BK)] = rb[s][r];
-  };
-  V4 acc[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) acc[i] = V4{0, 0, 0, 0};
+  constexpr int DD = 4, K2 = D * DD, BM = 16 * D;
+  // a second accumulator chain only where the registers leave room for it
+  constexpr int CH = sizeof(T) == 4 || D <= 3 ? 2 : 1;
+  using TL = TileLoop<T, false, false, true, true, D, 1, 1, 4, VEC, CH>;
+  constexpr int XC = 16 * (int)sizeof(T) / 16;  // chunks of a row of one wave's 16 columns
+  constexpr int XS = 4 * BM * XC;
+  __shared__ u4_t smem[TL::SMEM > XS ? TL::SMEM : XS];
+  const int lane = threadIdx.x & 63, wn = threadIdx.x >> 6;
+  typename TL::Acc acc;
+  // A(m, k) = Lenv[k + m cL], B(k, n) = theta[k + n cL]
+  TL::run(smem, D * cL, DD * cR, cL, 0, cL, blockIdx.x * BM, blockIdx.y * 64, Lenv, cL, theta, cL,
+          acc);
   const int li = lane & 15, lk = lane >> 4;
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      T af[D];
-#pragma unroll
-      for (int i = 0; i < D; ++i) af[i] = As[buf][kk + lk][i * 16 + li];
-      const T bf = Bs[buf][kk + lk][wn * 16 + li];
-#pragma unroll
-      for (int i = 0; i < D; ++i) acc[i] = mfma(bf, af[i], acc[i]);
-    }
+  // value (row, ss + 4 bq) of the wave's block at T index of chunk
+  // (column / VE) ^ (row % XC): the sixteen rows of a store spread over banks
+  T* const xw = reinterpret_cast<T*>(smem + wn * BM * XC);
+  auto at = [&](int row, int col) {
+    return row * 16 + (((col / TL::VE) ^ (row & (XC - 1))) * TL::VE) + col % TL::VE;
   };
-  const int nk = (K + BK - 1) / BK;
-  load(0, 0);
-  store(0, 0);
-  if (nk > 1) load(1, BK);
-  __syncthreads();
-  for (int kt = 0; kt < nk; kt += 2) {
-    if (kt + 2 < nk) load(0, (kt + 2) * BK);
-    compute(0);
-    if (kt + 1 < nk) store(1, 1);
-    __syncthreads();
-    if (kt + 1 >= nk) break;
-    if (kt + 3 < nk) load(1, (kt + 3) * BK);
-    compute(1);
-    if (kt + 2 < nk) store(0, 0);
-    __syncthreads();
-  }
-  // every exit of the loop passed a barrier: the operand buffers are free
 #pragma unroll
   for (int i = 0; i < D; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      Xs[i * 16 + li][wn * 16 + (GT<T>::G1 ? lk + 4 * r : 4 * lk + r)] = acc[i][r];
-  __syncthreads();
-  const int al = t & 15, bl = t >> 4;
-  const int a = blockIdx.x * 16 + al, b = blockIdx.y * 16 + bl;
+      xw[at(i * 16 + li, GT<T>::G1 ? lk + 4 * r : 4 * lk + r)] = acc[0][i][0][r];
+  __builtin_amdgcn_wave_barrier();
+  __threadfence_block();
+  const int a = blockIdx.x * 16 + li, b = blockIdx.y * 16 + wn * 4 + lk;
   if (a >= cL || b >= cR) return;
   T x[K2];
 #pragma unroll
   for (int w = 0; w < D; ++w)
 #pragma unroll
-    for (int ss = 0; ss < DD; ++ss) x[w + D * ss] = Xs[w + D * al][ss + DD * bl];
+    for (int ss = 0; ss < DD; ++ss) x[w + D * ss] = xw[at(w + D * li, ss + DD * lk)];
   T* const yb = Y + a + (size_t)cL * DD * b;
   const size_t sn = (size_t)cL * DD * cR;
-#pragma unroll
+  // the constant address space: nothing in the launch writes WW, and past a
+  // barrier the compiler would load it into vector registers otherwise
+  typedef const T __attribute__((address_space(4))) ConstT;
+  const ConstT* const Wc = (const ConstT*)(uintptr_t)WW;
+#pragma unroll 1
   for (int n = 0; n < D; ++n)
 #pragma unroll
     for (int sp = 0; sp < DD; ++sp) {
-      const int c2 = sp + DD * n;
+      const ConstT* const wc = Wc + K2 * (sp + DD * n);
       T y = T(0);
 #pragma unroll
-      for (int c = 0; c < K2; ++c) y = y + x[c] * Ws[c + K2 * c2];
+      for (int c = 0; c < K2; ++c) y = y + x[c] * wc[c];
       yb[(size_t)cL * sp + sn * n] = y;
     }
 }
 }  // namespace
 
-template <class T, class TB>
-bool heff2_x_mpo(hipStream_t st, int cL, int cR, int d, int D, const T* Lenv, const TB* theta,
+template <class T>
+bool heff2_x_mpo(hipStream_t st, int cL, int cR, int d, int D, const T* Lenv, const T* theta,
                  const T* WW, T* Y) {
-  if constexpr (is_cplx<T>::value || is_cplx<TB>::value) {
+  if constexpr (is_cplx<T>::value) {
     return false;
   } else {
     if (d != 2 || D < 2 || D > 8 || cL < 1 || cR < 1) return false;
     const dim3 grid(cdiv(cL, 16), cdiv(cR, 16));
+    const bool vec = cL >= 16 / (int)sizeof(T);  // both operands are contiguous along cL
     switch (D) {
-#define DMRG_XM(D_) \
-  case D_: hipLaunchKernelGGL((k_heff2_x_mpo<T, TB, D_, 16>), grid, dim3(256), 0, st, cL, cR, Lenv, theta, WW, Y); break
+#define DMRG_XM(D_)                                                                             \
+  case D_:                                                                                      \
+    if (vec)                                                                                    \
+      hipLaunchKernelGGL((k_heff2_x_mpo<T, D_, true>), grid, dim3(256), 0, st, cL, cR, Lenv,    \
+                         theta, WW, Y);                                                         \
+    else                                                                                        \
+      hipLaunchKernelGGL((k_heff2_x_mpo<T, D_, false>), grid, dim3(256), 0, st, cL, cR, Lenv,   \
+                         theta, WW, Y);                                                         \
+    break
       DMRG_XM(2); DMRG_XM(3); DMRG_XM(4); DMRG_XM(5); DMRG_XM(6); DMRG_XM(7); DMRG_XM(8);
 #undef DMRG_XM
       default: return false;
@@ -948,62 +1227,31 @@ bool gemm_rows_small(hipStream_t st, int M, int N, int K, const T* A, View2 va, 
 template <class T>
 void gemm(hipStream_t st, int opA, int opB, int M, int N, int K, T alpha, const T* A, int lda,
           const T* B, int ldb, T beta, T* C, int ldc, GemmTile tile) {
-  plain<T>(st, opA, opB, tile, M, N, K, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 1);
+  plain<T>(st, opA, opB, tile, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 0);
 }
 
 template <class T>
 void gemm_herm(hipStream_t st, int opA, int opB, int N, int K, T alpha, const T* A, int lda,
                const T* B, int ldb, T* C, int ldc, GemmTile tile) {
-  DMRG_REQUIRE(tile.bm == tile.bn, "gemm_herm: square tiles only");
-  plain<T>(st, opA, opB, tile, N, N, K, alpha, A, lda, 0, B, ldb, 0, T(0), C, ldc, 0, 1, 1);
+  if (tile.bm != tile.bn) tile = pick_square(N, is_cplx<T>::value);  // mirrored tile by tile
+  plain<T>(st, opA, opB, tile, N, N, K, alpha, A, lda, B, ldb, T(0), C, ldc, 1);
 }
 
 template <class T>
-void gemm_strided(hipStream_t st, int opA, int opB, int M, int N, int K, T alpha, const T* A,
-                  int lda, long long sA, const T* B, int ldb, long long sB, T beta, T* C, int ldc,
-                  long long sC, int batch, GemmTile tile) {
-  plain<T>(st, opA, opB, tile, M, N, K, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch);
-}
-
-template <class T>
-void gemm_tensor(hipStream_t st, int M, int N, int K, T alpha, const T* A, View2 va, bool conjA,
-                 bool a_kfast, const T* B, View2 vb, bool conjB, bool b_kfast, T beta, T* C,
-                 View2 vc, GemmTile tile) {
+void gemm_tensor(hipStream_t st, int M, int N, int K, T alpha, const T* A, View2 va, const T* B,
+                 View2 vb, T beta, T* C, View2 vc, GemmTile tile) {
   DMRG_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_tensor: negative size");
   if (M == 0 || N == 0) return;
-  if (!is_cplx<T>::value) conjA = conjB = false;
-  AddrTensor aa{va}, ab{vb}, ac{vc};
-#define DMRG_GT(CA_, CB_, KA_, KB_) \
-  launch<T, CA_, CB_, KA_, KB_>(st, tile, M, N, K, alpha, A, aa, 0, B, ab, 0, beta, C, ac, 0, 1)
-  int code = (conjA ? 8 : 0) | (conjB ? 4 : 0) | (a_kfast ? 2 : 0) | (b_kfast ? 1 : 0);
-  if constexpr (is_cplx<T>::value) {
-    switch (code) {
-      case 0: DMRG_GT(false, false, false, false); break;
-      case 1: DMRG_GT(false, false, false, true); break;
-      case 2: DMRG_GT(false, false, true, false); break;
-      case 3: DMRG_GT(false, false, true, true); break;
-      case 4: DMRG_GT(false, true, false, false); break;
-      case 5: DMRG_GT(false, true, false, true); break;
-      case 6: DMRG_GT(false, true, true, false); break;
-      case 7: DMRG_GT(false, true, true, true); break;
-      case 8: DMRG_GT(true, false, false, false); break;
-      case 9: DMRG_GT(true, false, false, true); break;
-      case 10: DMRG_GT(true, false, true, false); break;
-      case 11: DMRG_GT(true, false, true, true); break;
-      case 12: DMRG_GT(true, true, false, false); break;
-      case 13: DMRG_GT(true, true, false, true); break;
-      case 14: DMRG_GT(true, true, true, false); break;
-      default: DMRG_GT(true, true, true, true); break;
-    }
-  } else {
-    switch (code & 3) {
-      case 0: DMRG_GT(false, false, false, false); break;
-      case 1: DMRG_GT(false, false, false, true); break;
-      case 2: DMRG_GT(false, false, true, false); break;
-      default: DMRG_GT(false, false, true, true); break;
-    }
-  }
-#undef DMRG_GT
+  // 32x32 tiles serve grids that cannot fill the chip with 64x64 ones
+  constexpr int BK = is_cplx<T>::value ? 16 : 32;
+  const AddrTensor aa{va}, ab{vb}, ac{vc};
+  if (tile.bm == 32)
+    hipLaunchKernelGGL((k_gemm<T, 32, 32, BK>), dim3(cdiv(M, 32), cdiv(N, 32)), dim3(256), 0, st, M,
+                       N, K, alpha, A, aa, B, ab, beta, C, ac);
+  else
+    hipLaunchKernelGGL((k_gemm<T, 64, 64, 16>), dim3(cdiv(M, 64), cdiv(N, 64)), dim3(256), 0, st, M,
+                       N, K, alpha, A, aa, B, ab, beta, C, ac);
+  DMRG_LAUNCH_CHECK();
 }
 
 #define DMRG_INST(T)                                                                         \
@@ -1011,17 +1259,13 @@ void gemm_tensor(hipStream_t st, int M, int N, int K, T alpha, const T* A, View2
                         T, T*, int, GemmTile);                                                 \
   template void gemm_herm<T>(hipStream_t, int, int, int, int, T, const T*, int, const T*, int,  \
                              T*, int, GemmTile);                                                \
-  template void gemm_strided<T>(hipStream_t, int, int, int, int, int, T, const T*, int,        \
-                                long long, const T*, int, long long, T, T*, int, long long,    \
-                                int, GemmTile);                                                \
-  template void gemm_tensor<T>(hipStream_t, int, int, int, T, const T*, View2, bool, bool,     \
-                               const T*, View2, bool, bool, T, T*, View2, GemmTile);           \
+  template void gemm_tensor<T>(hipStream_t, int, int, int, T, const T*, View2, const T*, View2, \
+                               T, T*, View2, GemmTile);                                        \
   template bool gemm_rows_small<T>(hipStream_t, int, int, int, const T*, View2, const T*, T*,  \
                                    View2);                                                      \
-  template bool gemm_nn_splitk<T>(hipStream_t, int, int, int, const T*, int, const T*, int, T*, \
-                                  int, T*, size_t);                                             \
-  template bool heff2_x_mpo<T, T>(hipStream_t, int, int, int, int, const T*, const T*, const T*, \
-                                  T*);
+  template bool gemm_splitk<T>(hipStream_t, int, int, int, int, int, const T*, int, const T*,   \
+                               int, T*, int, T*, size_t);                                       \
+  template bool heff2_x_mpo<T>(hipStream_t, int, int, int, int, const T*, const T*, const T*, T*);
 DMRG_INST(double)
 DMRG_INST(cdouble)
 DMRG_INST(float)

@@ -238,7 +238,7 @@ void warm_basis_right(hipStream_t st, const T* Z, int cR, int d, const T* X, T* 
   // rows i = (s, j) -> s + N*j (two-level, n1 = d); k = b' -> d*b'; n = b -> d*b
   const View2 vx{{d, 1, N}, {1 << 30, d, 0}};
   const View2 vz{{1 << 30, 1, 0}, {1 << 30, cR, 0}};  // Z(b', b) at b' + cR b
-  gemm_tensor<T>(st, d * N, cR, cR, T(1), X, vx, false, false, Z, vz, true, true, T(0), out, vx,
+  gemm_tensor<T>(st, d * N, cR, cR, T(1), X, vx, Z, vz, T(0), out, vx,
                  gemm_pick_tile(d * N, cR, cR, is_cplx<T>::value));
 }
 
