@@ -283,9 +283,9 @@ __global__ void k_permute(const T* __restrict__ A, const T* __restrict__ V, T* _
 // No other thread touches those entries in that round.  Threads QT0 and up
 // (waves 2-3) apply the round's rotations to the columns of Q.  A pair with |a_ab| <= thr gets (c, s) = (1, 0), which leaves every
 // entry bit-for-bit unchanged, so the updates need no flags.  A sub-problem
-// whose off-diagonal is already below 1e-6 |rho|_F gets one inner sweep (the
-// next outer sweep re-checks it), others up to inner_max; a sweep without a
-// rotation ends the loop.
+// whose off-diagonal is already below 1e-6 |rho|_F gets one inner sweep,
+// others up to inner_max (one, except for a matrix of a single pair); a sweep
+// without a rotation ends the loop.
 constexpr int NTA = 256;
 constexpr int HP = JP / 2;                  // pairs per inner round
 constexpr int NBLK = HP * (HP - 1) / 2;     // off-diagonal 2x2 blocks per round
@@ -1144,6 +1144,240 @@ __global__ __launch_bounds__(256) void k_block_orth(T* __restrict__ Y, int len, 
 
 inline unsigned grid_for(size_t tot) { return (unsigned)std::min<size_t>(cdiv(tot, 256), 8192); }
 
+// ---------------------------------------------------------------------------
+// Householder QR of a matrix held as Np columns of Np rows: one workgroup
+// reduces a panel of 16 CPW columns, rows j0 .. Np - 1, and GEMMs apply it to
+// the rest.
+//
+// Sixteen waves own CPW columns each (column w + 16 s), in registers: lane l
+// holds the rows l, l + 64, ...  Step j reflects with H_j = I - v v^H,
+// v = (x + phase(x_j) |x| e_j) / sqrt(|x|^2 + |x_j| |x|) for x = column j from
+// row j down (|v|^2 = 2; v = 0 and H_j = I for a zero column), so H_j is
+// Hermitian and unitary whatever the scalar type.  v goes to the others through
+// LDS (two buffers); the wave that owns column j + 1 updates it first and
+// forms the next v from its registers: one barrier per step.  The panel's
+// product is H_0 H_1 ... = I - V T V^H with T^-1 = I + (V^H V, strictly upper).
+// What bounds it is that chain: LDS read of v, dot product, wave reduction,
+// update, norm, reduction, square root.
+// ---------------------------------------------------------------------------
+// Sum over the wave, in every lane, by DPP adds (row shifts, then row
+// broadcasts into the last lane): no trip through LDS.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  int p[2], q[2];
+  __builtin_memcpy(p, &v, 8);
+  q[0] = __builtin_amdgcn_update_dpp(0, p[0], CTRL, ROWS, 0xf, true);
+  q[1] = __builtin_amdgcn_update_dpp(0, p[1], CTRL, ROWS, 0xf, true);
+  double u;
+  __builtin_memcpy(&u, q, 8);
+  return v + u;
+}
+__device__ inline double read_lane(double v, int l) {
+  int p[2];
+  __builtin_memcpy(p, &v, 8);
+  p[0] = __builtin_amdgcn_readlane(p[0], l);
+  p[1] = __builtin_amdgcn_readlane(p[1], l);
+  __builtin_memcpy(&v, p, 8);
+  return v;
+}
+__device__ inline double wave_sum_all(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return read_lane(v, 63);
+}
+__device__ inline cdouble wave_sum_all(cdouble v) {
+  return cdouble(wave_sum_all(v.x), wave_sum_all(v.y));
+}
+__device__ inline cdouble read_lane(cdouble v, int l) {
+  return cdouble(read_lane(v.x, l), read_lane(v.y, l));
+}
+
+template <class T, int EPL, int CPW>
+__global__ __launch_bounds__(1024) void k_qr_panel(T* __restrict__ A, int ld, int j0, int rows,
+                                                   T* __restrict__ V, int ldv,
+                                                   T* __restrict__ Tm) {
+  constexpr int B = 16 * CPW;
+  __shared__ T vb[2][EPL * 64];
+  __shared__ T Z[B][B + 1], Ts[B][B + 1];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  T a[CPW][EPL];
+#pragma unroll
+  for (int s = 0; s < CPW; ++s) {
+    const T* col = A + j0 + (size_t)(j0 + w + 16 * s) * ld;
+#pragma unroll
+    for (int q = 0; q < EPL; ++q) a[s][q] = lane + 64 * q < rows ? col[lane + 64 * q] : T(0);
+  }
+  // column j of the panel in slot s becomes R above and on the diagonal
+  // (stored), v in the registers and in buffer `buf`
+  auto reflect = [&](int s, int j, int buf) {
+    double part = 0.0;
+#pragma unroll
+    for (int q = 0; q < EPL; ++q) part += lane + 64 * q > j ? abs2(a[s][q]) : 0.0;
+    part = wave_sum_all(part);
+    const T alpha = read_lane(a[s][0], j);
+    const double a2 = abs2(alpha), x2 = part + a2;
+    const bool ok = x2 > 1e-290, oka = a2 > 1e-290;
+    const double ya = oka ? rsqrt_refined(a2) : 0.0, xn = ok ? x2 * rsqrt_refined(x2) : 0.0;
+    const T phase = oka ? alpha * ya : T(1);
+    const double f = ok ? rsqrt_refined(x2 + a2 * ya * xn) : 0.0;
+    T* col = A + j0 + (size_t)(j0 + j) * ld;
+    if (lane <= j) col[lane] = lane < j ? a[s][0] : (ok ? -phase * xn : alpha);
+#pragma unroll
+    for (int q = 0; q < EPL; ++q) {
+      const int i = lane + 64 * q;
+      if (i > j && i < rows) col[i] = T(0);
+      T v = a[s][q];
+      if (i == j) v = alpha + phase * xn;
+      v = i < j ? T(0) : v * f;
+      a[s][q] = v;
+      vb[buf][i] = v;
+    }
+  };
+  // T(:, j) = -T(:, :j) Z(:j, j): row i in lanes i and i + 32, each summing
+  // every other k.  The wave that owned column j does it during step j + 1.
+  auto t_column = [&](int j) {
+    const int i = lane & 31, h = lane >> 5;
+    T x(0);
+    if (i < j) {
+#pragma unroll 4
+      for (int k = i + ((i + h) & 1); k < j; k += 2) x -= Ts[i][k] * Z[k][j];
+    }
+    if constexpr (is_cplx<T>::value) x += cdouble(__shfl_xor(real(x), 32), __shfl_xor(imag(x), 32));
+    else x += __shfl_xor(x, 32);
+    if (h == 0 && i < B) Ts[i][j] = i < j ? x : T(i == j ? 1.0 : 0.0);
+  };
+  if (w == 0) reflect(0, 0, 0);
+  __syncthreads();
+  for (int j = 0; j < B; ++j) {
+    const T* vs = vb[j & 1] + lane;
+    const int jn = j + 1;
+    // one LDS read of v per wave and step where the registers hold it, else
+    // one per use (all columns' reads share one CU's LDS: 2 x 4 cycles per
+    // column and row block)
+    constexpr bool KEEP = EPL * sizeof(T) <= 64;
+    T vr[KEEP ? EPL : 1];
+    if constexpr (KEEP) {
+#pragma unroll
+      for (int q = 0; q < EPL; ++q) vr[q] = vs[64 * q];
+    }
+    auto v = [&](int q) {
+      if constexpr (KEEP) return vr[q];
+      else return vs[64 * q];
+    };
+    auto update = [&](int s) {  // a_s <- H_j a_s
+      T dot(0);
+#pragma unroll
+      for (int q = 0; q < EPL; ++q) dot += conj(v(q)) * a[s][q];
+      dot = wave_sum_all(dot);
+      if constexpr (!KEEP) asm volatile("" ::: "memory");
+#pragma unroll
+      for (int q = 0; q < EPL; ++q) a[s][q] -= v(q) * dot;
+    };
+#pragma unroll
+    for (int s = 0; s < CPW; ++s)
+      if (w + 16 * s == jn) {
+        update(s);
+        reflect(s, jn, jn & 1);
+      }
+#pragma unroll
+    for (int s = 0; s < CPW; ++s) {
+      const int c = w + 16 * s;
+      if (c > jn) {
+        update(s);
+      } else if (c < j) {  // V^H V above the diagonal
+        T z(0);
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) z += conj(a[s][q]) * v(q);
+        z = wave_sum_all(z);
+        if (lane == 0) Z[c][j] = z;
+      }
+    }
+    if (j > 0 && w == ((j - 1) & 15)) t_column(j - 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int s = 0; s < CPW; ++s) {
+    T* out = V + (size_t)(w + 16 * s) * ldv;
+#pragma unroll
+    for (int q = 0; q < EPL; ++q)
+      if (lane + 64 * q < rows) out[lane + 64 * q] = a[s][q];
+  }
+  if (w == ((B - 1) & 15)) t_column(B - 1);
+  __syncthreads();
+  for (int e = threadIdx.x; e < B * B; e += 1024) Tm[e] = Ts[e % B][e / B];
+}
+
+template <class T>
+__global__ void k_identity(T* __restrict__ Q, int n) {
+  const size_t tot = (size_t)n * n;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
+       e += (size_t)gridDim.x * blockDim.x)
+    Q[e] = T(mod32(e, n) == div32(e, n) ? 1.0 : 0.0);
+}
+
+// Largest matrix whose panels fit the registers of one workgroup, and the
+// smallest one worth it (see jacobi).
+template <class T> constexpr int qr_max() { return is_cplx<T>::value ? 1536 : 2048; }
+constexpr int QR_MIN = 160;
+
+// A (Np x Np, ld Np) <- R, Q <- the unitary factor; work holds at least
+// 4 * 32 * Np + 32 * 32 values.
+template <class T>
+void qr_factor(hipStream_t st, T* A, T* Q, T* work, int Np) {
+  const bool cx = is_cplx<T>::value;
+  T* V = work;
+  T* U = V + (size_t)32 * Np;
+  T* W = U + (size_t)32 * Np;
+  T* Y = W + (size_t)32 * Np;
+  T* Tm = Y + (size_t)32 * Np;
+  hipLaunchKernelGGL(k_identity<T>, dim3(std::min<size_t>(cdiv((size_t)Np * Np, 256), 4096)),
+                     dim3(256), 0, st, Q, Np);
+  for (int j0 = 0; j0 < Np;) {
+    const int rows = Np - j0;
+    int b = 32;  // Np and every b are multiples of 16: no ragged panel
+#define DMRG_QR(EPL_, CPW_)                                                                     \
+  do {                                                                                          \
+    b = 16 * CPW_;                                                                              \
+    hipLaunchKernelGGL((k_qr_panel<T, EPL_, CPW_>), dim3(1), dim3(1024), 0, st, A, Np, j0, rows, \
+                       V, Np, Tm);                                                              \
+  } while (0)
+    if (rows < 32) DMRG_QR(1, 1);
+    else if (rows <= 256) DMRG_QR(4, 2);
+    else if (rows <= 512) DMRG_QR(8, 2);
+    else if constexpr (!is_cplx<T>::value) {
+      if (rows <= 1024) DMRG_QR(16, 2);
+      else DMRG_QR(32, 1);
+    } else {
+      if (rows <= 1024) DMRG_QR(16, 1);
+      else DMRG_QR(24, 1);
+    }
+#undef DMRG_QR
+    // U = V T;  A2 <- A2 - V (U^H A2);  Q2 <- Q2 - (Q2 U) V^H
+    gemm<T>(st, OP_N, OP_N, rows, b, b, T(1), V, Np, Tm, b, T(0), U, rows,
+            gemm_pick_tile(rows, b, b, cx));
+    const int nc = rows - b;
+    if (nc > 0) {
+      T* A2 = A + j0 + (size_t)(j0 + b) * Np;
+      gemm<T>(st, OP_H, OP_N, b, nc, rows, T(1), U, rows, A2, Np, T(0), W, b,
+              gemm_pick_tile(b, nc, rows, cx));
+      gemm<T>(st, OP_N, OP_N, rows, nc, b, T(-1), V, Np, W, b, T(1), A2, Np,
+              gemm_pick_tile(rows, nc, b, cx));
+    }
+    T* Q2 = Q + (size_t)j0 * Np;
+    gemm<T>(st, OP_N, OP_N, Np, b, rows, T(1), Q2, Np, U, rows, T(0), Y, Np,
+            gemm_pick_tile(Np, b, rows, cx));
+    gemm<T>(st, OP_N, OP_H, Np, rows, b, T(-1), Y, Np, V, Np, T(1), Q2, Np,
+            gemm_pick_tile(Np, rows, b, cx));
+    j0 += b;
+  }
+  DMRG_LAUNCH_CHECK();
+}
+
+
 // Block-Jacobi eigen-decomposition of the Hermitian matrix already stored in
 // w.A[0] (N x N, ld Np, padding arbitrary).  Leaves the diagonalised matrix in
 // w.A[cur], the eigenvectors in w.V[cur] and the descending order in w.perm.
@@ -1179,7 +1413,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   const double fro = hs[0];
   if (!(fro == fro) || std::isinf(fro)) throw Error(ST_NONFINITE, "svd: non-finite matrix entries");
   const double rot_tol = 0.125 * prm.tol;
-  const int inner_max = (nb == 2) ? 64 : 2;
+  // One inner sweep per block pair: a second one before the pairs meet other
+  // blocks saves one outer sweep in fourteen and costs as much again (256^2,
+  // Schmidt values falling to 1e-6: 14 sweeps of 31 inner rounds against 13 of
+  // 62).  A matrix of a single pair is diagonalised in place.
+  const int inner_max = (nb == 2) ? 64 : 1;
   const int noff = np * (np - 1) / 2, nvt = (Np / JP) * np;
   int cur = 0;
   sweeps = 0;
@@ -1225,22 +1463,59 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   };
   bool done = false;
   double last_off = INFINITY;  // latest convergence measure (criterion in force)
-  if (v_given) {
-    // Started from a basis near the eigenbasis: up to two first-order
-    // (all-pairs, GEMM-only) corrections before any Jacobi sweep.  A pair is
-    // corrected when its gap exceeds sep |A_ij| (the first-order step then
+  const double gate = keep > 0 ? 1e-4 : 1e-6;  // measure below which first-order steps are tried
+  bool near = v_given;                          // try them before the next sweep
+  if (!v_given && Np >= QR_MIN && Np <= qr_max<T>()) {
+    // No basis given: two steps of orthogonal iteration, Q R = rho with the
+    // columns in descending order of the diagonal, then R Q = Q^H rho Q, bring
+    // the graded spectrum of a truncation to within a few sweeps of diagonal
+    // (512^2, Schmidt values falling to 1e-6: 5 sweeps instead of 16; a bond
+    // of a first DMRG sweep at chi = 128: 1 instead of 5).  A step costs about
+    // as much as one sweep of the round robin; below QR_MIN a sweep is a few
+    // rounds and costs less.
+    for (int it = 0; it < 2; ++it) {
+      hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np,
+                         N, w.perm, nullptr);
+      hipLaunchKernelGGL(k_permute<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], w.V[cur],
+                         w.A[1 - cur], w.V[1 - cur], w.perm, Np);
+      cur = 1 - cur;
+      qr_factor<T>(st, w.A[cur], w.W, w.Y, Np);
+      // (R Q)^H: its upper triangle, which k_prep keeps, comes from the later,
+      // smaller rows of R
+      const GemmTile tl = gemm_pick_tile(Np, Np, Np, is_cplx<T>::value);
+      gemm<T>(st, OP_H, OP_H, Np, Np, Np, T(1), w.W, Np, w.A[cur], Np, T(0), w.A[1 - cur], Np, tl);
+      gemm<T>(st, OP_N, OP_N, Np, Np, Np, T(1), w.V[cur], Np, w.W, Np, T(0), w.V[1 - cur], Np, tl);
+      cur = 1 - cur;
+      hipLaunchKernelGGL(k_prep<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], w.V[cur], N, Np,
+                         0);
+      DMRG_LAUNCH_CHECK();
+    }
+    last_off = offmax(w.A[cur]);
+    if (last_off <= prm.tol * fro) last_off = accept_keep(w.A[cur], last_off);
+    off_rel = last_off / fro;
+    done = last_off <= prm.tol * fro;
+    near = last_off <= gate * fro;
+  }
+  // Near the eigenbasis: first-order (all-pairs, GEMM-only) corrections.  They
+  // run before any Jacobi sweep from a basis that was given, and between
+  // sweeps from one that was not, once the measure is below the gate.
+  // `known`: the measure of w.A[0] when it has been taken already.
+  auto first_order = [&](double known) {
+    // A pair is corrected when its gap exceeds sep |A_ij| (the first-order step then
     // leaves O(|A_ij|/sep)); the subspace criterion tolerates the rougher sep.
     // Steps go on while each one cuts the measure at least tenfold.  Pairs
     // near the cut whose gap is only 30-100 times their coupling stall the
     // step at sep = 1e2; the subspace criterion then retries with sep = 30
     // (first-order error |A_ij|/30 per step) before handing over to Jacobi.
     const GemmTile tl = gemm_pick_tile(Np, Np, Np, is_cplx<T>::value);
-    double sep = keep > 0 ? 1e2 : 1e4;
-    const double gate = keep > 0 ? 1e-4 : 1e-6;
-    const int max_steps = keep > 0 ? 5 : 2;
+    double sep = keep > 0 || !v_given ? 1e2 : 1e4;
+    const int max_steps = keep > 0 || !v_given ? 5 : 2;
     for (int it = 0; it <= max_steps && !done; ++it) {
-      double o = offmax(w.A[0]);
-      if (o <= prm.tol * fro) o = accept_keep(w.A[0], o);
+      double o = known;
+      if (it > 0 || known < 0.0) {
+        o = offmax(w.A[0]);
+        if (o <= prm.tol * fro) o = accept_keep(w.A[0], o);
+      }
       const double prev = last_off;
       last_off = o;
       off_rel = o / fro;
@@ -1325,10 +1600,21 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       DMRG_LAUNCH_CHECK();
       ++cnt.oa;
     }
-  }
+  };
+  int fo_left = v_given ? 1 : 2;  // stages of first-order steps left to try
   bool bip_ok = true;  // bipartite sweeps allowed (revoked once one stalls)
   int n_bip = 0;
   for (int sw = 0; sw < prm.max_sweeps && !done; ++sw) {
+    if (near && fo_left > 0) {
+      --fo_left;
+      if (cur == 1) {
+        std::swap(w.A[0], w.A[1]);
+        std::swap(w.V[0], w.V[1]);
+        cur = 0;
+      }
+      first_order(v_given ? -1.0 : last_off);
+      if (done) break;
+    }
     // sort the diagonal, permute rho and V into the other buffer
     hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np, N,
                        w.perm, nullptr);
@@ -1343,7 +1629,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     // turns couplings inside a group into cross couplings; so bipartite sweeps
     // run only while each cuts the measure tenfold (at most 4 per split), and
     // the full round robin finishes the job.
-    const int ka = (bip_ok && keep > 0 && keep % JB == 0 && keep < Np && v_given &&
+    const int ka = (bip_ok && keep > 0 && keep % JB == 0 && keep < Np && near &&
                     last_off <= 1e-4 * fro) ? keep / JB : 0;
     const double off_before = last_off;
     const int rounds = sched_rounds(nb, ka);
@@ -1359,6 +1645,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (ka > 0) ++cnt.bip;
     if (ka > 0 && (++n_bip >= 4 || off > 0.1 * off_before)) bip_ok = false;
     sweeps = sw + 1;
+    if (!v_given) near = Np >= QR_MIN && off <= gate * fro;
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
   }
