@@ -43,27 +43,15 @@ double LanczosRunner<T>::run(hipStream_t st, T* theta, size_t n, int kmax, int s
   // replaced by the seeded stream 42+site) before the first, the convergence
   // check after iteration b-1 when `check`.
   auto stretch = [&](int a, int b, bool check) {
-    if (a == 0) {
-      lz_reset(st, *lz);
-      lz_norm<T>(st, *lz, theta, n);
-      lz_fill_if_small<T>(st, *lz, theta, n, (uint64_t)(42 + site), 1e-14);
-      lz_norm<T>(st, *lz, theta, n);
-      lz_scale<T>(st, *lz, V, theta, n);
-    }
+    if (a == 0) lz_start<T>(st, *lz, theta, V, n, (uint64_t)(42 + site), 1e-14);
     for (int it = a; it < b; ++it) {
       T* vi = V + (size_t)it * n;
       if (timed) DMRG_HIP(hipEventRecord(ev[2 * it], st));
       matvec(vi, work);
       if (timed) DMRG_HIP(hipEventRecord(ev[2 * it + 1], st));
-      lz_alpha<T>(st, *lz, vi, work, n, it);
-      lz_sub_dots<T>(st, *lz, work, V, n, it);
-      lz_orth_norm<T>(st, *lz, work, V, n, it);
-      lz_next<T>(st, *lz, it + 1 < max_iter ? V + (size_t)(it + 1) * n : nullptr, work, n, it);
+      lz_step<T>(st, *lz, work, V, n, it, it + 1 < max_iter);
     }
-    if (check) {
-      lz_check(st, *lz, b, beta_tol, eig_tol, eig_rel);
-      DMRG_HIP(hipMemcpyAsync(h_status, lz->status, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
-    }
+    if (check) lz_check(st, *lz, b, beta_tol, eig_tol, eig_rel, h_status);
   };
   int niter = max_iter;
   int a = 0, chunk = 0;
@@ -119,9 +107,7 @@ double LanczosRunner<T>::run(hipStream_t st, T* theta, size_t n, int kmax, int s
     ++chunk;
   }
   lz_final(st, *lz, niter);
-  lz_ritz<T>(st, *lz, theta, V, n, niter);
-  lz_scale<T>(st, *lz, theta, theta, n);
-  DMRG_HIP(hipMemcpyAsync(h_scal, lz->scal, 8 * sizeof(double), hipMemcpyDeviceToHost, st));
+  lz_ritz<T>(st, *lz, theta, V, n, niter, h_scal);
   DMRG_HIP(hipStreamSynchronize(st));
   double ms = 0.0;
   for (int j = 0; timed && j < nmv; ++j) {
@@ -677,8 +663,7 @@ double Engine<T>::rayleigh2(int site) {
   const int cL = bond[site], cR = bond[site + 2];
   const size_t n = (size_t)cL * d * d * cR;
   matvec2(site, theta, work, true);
-  lz_alpha<T>(s_main, lz, theta, work, n, 0);
-  lz_alpha_value(s_main, lz, n, 0);
+  lz_dot<T>(s_main, lz, theta, work, n);
   double* const ha = reinterpret_cast<double*>(h_aux);
   DMRG_HIP(hipMemcpyAsync(ha, lz.alpha, sizeof(double), hipMemcpyDeviceToHost, s_main));
   DMRG_HIP(hipStreamSynchronize(s_main));

@@ -1,5 +1,6 @@
 // Lanczos vector kernels, tridiagonal eigensolver and the device generator.
 #include "lanczos.hpp"
+#include "wave.hpp"
 
 #include <algorithm>
 #include <cfloat>
@@ -8,13 +9,13 @@
 namespace dmrg {
 namespace {
 
+// The vector kernels run 1024 threads on chunks of 1024 E elements, thread t of
+// workgroup b on the elements b 1024 E + 1024 e + t, held in registers: one
+// workgroup a CU up to 2^20 elements, so the partial sums that the next kernel
+// reduces stay at 256 a value.
 constexpr int NT = 256;
-
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
+constexpr int NL = 1024;
+constexpr int NW = NL / 64;
 
 template <class T> struct Acc;
 template <> struct Acc<double> {
@@ -28,86 +29,131 @@ template <> struct Acc<cdouble> {
   __device__ static cdouble get(const double* o) { return cdouble(o[0], o[1]); }
 };
 
-__device__ inline void chunk_range(size_t n, size_t& b, size_t& e) {
-  size_t chunk = (n + gridDim.x - 1) / gridDim.x;
-  chunk = (chunk + NT - 1) / NT * NT;
-  b = blockIdx.x * chunk;
-  e = b + chunk < n ? b + chunk : n;
-}
-
 // Reductions across workgroups carry no fence or atomic: each producing
 // kernel writes one partial per workgroup, and the kernel that consumes the
-// sum re-reduces the partials itself (every workgroup, same fixed order, so
-// all workgroups see bit-identical values).  The kernel boundary makes the
-// partials visible.  A device-scope release inside a kernel would write back
-// the L2 of every XCD once per wave.
+// sum re-reduces the partials itself (every wave, same fixed order, so all see
+// bit-identical values).  The kernel boundary makes the partials visible.  A
+// device-scope release inside a kernel would write back the L2 of every XCD
+// once per wave.
 
-// Sum of part[0..nb) over the workgroup; the result is returned to every thread.
-__device__ inline double sum_parts(const double* __restrict__ part, int nb, double* sh) {
+// Sum of part[0..nb) in every lane of the calling wave.
+__device__ inline double sum_parts(const double* __restrict__ part, int nb) {
   double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += NT) s += part[b];
-  s = wave_sum(s);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  for (int b = threadIdx.x & 63; b < nb; b += 64) s += part[b];
+  return wave_sum_all(s);
+}
+
+// Sum of v over the workgroup, in every thread (sh: NW values, free on return).
+__device__ inline double block_sum(double v, double* sh) {
+  v = wave_sum_all(v);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   double r = 0.0;
 #pragma unroll
-  for (int i = 0; i < NT / 64; ++i) r += sh[i];
-  __syncthreads();  // sh is free again on return
+  for (int i = 0; i < NW; ++i) r += sh[i];
+  __syncthreads();
   return r;
 }
 
-// out[j] = sum_b part[j*nb + b] for j < cnt (one wave per j); ends with a barrier.
-__device__ inline void sum_parts_multi(const double* __restrict__ part, int nb, int cnt, double* out) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int j = w; j < cnt; j += NT / 64) {
-    double s = 0.0;
-    for (int b = lane; b < nb; b += 64) s += part[(size_t)j * nb + b];
-    s = wave_sum(s);
-    if (lane == 0) out[j] = s;
+// The thread's elements of x (zero, and an index inside the vector, past n).
+template <int E>
+struct Chunk {
+  unsigned idx[E];  // every vector has fewer than 2^32 elements
+  bool in[E];
+  __device__ explicit Chunk(size_t n) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const unsigned i = (blockIdx.x * E + e) * NL + threadIdx.x;
+      in[e] = i < (unsigned)n;
+      idx[e] = in[e] ? i : (unsigned)n - 1;
+    }
   }
-  __syncthreads();
+  template <class T> __device__ void load(const T* __restrict__ x, T (&v)[E]) const {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const T u = x[idx[e]];
+      v[e] = in[e] ? u : T(0);
+    }
+  }
+  template <class T> __device__ void store(T* __restrict__ x, const T (&v)[E]) const {
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (in[e]) x[idx[e]] = v[e];
+  }
+};
+template <class T, int E> __device__ inline double sum_abs2(const T (&v)[E]) {
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) s += abs2(v[e]);
+  return s;
 }
 
-// Partial sums of G values per thread -> part[(j0 + jj) * nb + blockIdx.x], jj < cnt.
-template <int G>
-__device__ inline void write_parts(const double (&v)[G], int cnt, double* part, int j0, int nb,
-                                   double* sh /*[G * NT/64]*/) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// Basis vectors taken at once: their loads are in flight together.
+template <class T, int E> constexpr int group() {
+  return E == 1 ? 8 : (is_cplx<T>::value ? 8 : 16) / E;
+}
+// v[g] = the thread's elements of basis vector j0 + g (of the last one past cnt).
+template <class T, int E, int G>
+__device__ inline void load_group(const Chunk<E>& c, const T* __restrict__ V, size_t n, int j0,
+                                  int cnt, T (&v)[G][E]) {
 #pragma unroll
-  for (int jj = 0; jj < G; ++jj) {
-    const double s = wave_sum(v[jj]);
-    if (lane == 0) sh[jj * (NT / 64) + w] = s;
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < cnt) {
-    double r = 0.0;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) r += sh[threadIdx.x * (NT / 64) + i];
-    part[(size_t)(j0 + threadIdx.x) * nb + blockIdx.x] = r;
-  }
-  __syncthreads();
+  for (int g = 0; g < G; ++g) c.load(V + (size_t)min(j0 + g, cnt - 1) * n, v[g]);
 }
 
-// partN[blk] = sum |x_i|^2 over the workgroup's chunk.
-template <class T>
-__global__ __launch_bounds__(NT) void k_norm(const T* __restrict__ x, size_t n,
-                                            double* __restrict__ partN) {
-  __shared__ double sh[NT / 64];
-  size_t b, e;
-  chunk_range(n, b, e);
-  // four independent accumulators keep four loads in flight per thread
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  size_t i = b + threadIdx.x;
-  for (; i + 3 * NT < e; i += 4 * NT) {
-    a0 += abs2(x[i]);
-    a1 += abs2(x[i + NT]);
-    a2 += abs2(x[i + 2 * NT]);
-    a3 += abs2(x[i + 3 * NT]);
+// sh[(j NC + c) NW + wave] = the wave's part of <v_j, x>, j < cnt.  v holds
+// the first group.
+template <class T, int E, int G>
+__device__ inline void wave_dots(const Chunk<E>& c, const T* __restrict__ V, size_t n, int cnt,
+                                 const T (&x)[E], T (&v)[G][E], double* sh) {
+  constexpr int NC = Acc<T>::N;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int j0 = 0; j0 < cnt; j0 += G) {
+    if (j0 > 0) load_group<T, E, G>(c, V, n, j0, cnt, v);
+    double o[G * NC];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      T a = conj(v[g][0]) * x[0];
+#pragma unroll
+      for (int e = 1; e < E; ++e) a += conj(v[g][e]) * x[e];
+      Acc<T>::put(a, o + g * NC);
+    }
+#pragma unroll
+    for (int q = 0; q < G * NC; ++q) o[q] = wave_sum_all(o[q]);
+    if (lane == 0)
+#pragma unroll
+      for (int q = 0; q < G * NC; ++q)
+        if (j0 * NC + q < cnt * NC) sh[(j0 * NC + q) * NW + w] = o[q];
   }
-  for (; i < e; i += NT) a0 += abs2(x[i]);
-  const double v[1] = {(a0 + a1) + (a2 + a3)};
-  write_parts<1>(v, 1, partN, 0, gridDim.x, sh);
+}
+
+// x -= sum_j c_j v_j, j < cnt.  v holds the first group.
+template <class T, int E, int G>
+__device__ inline void sub_basis(const Chunk<E>& c, const T* __restrict__ V, size_t n, int cnt,
+                                 const double* cs, T (&x)[E], T (&v)[G][E]) {
+  constexpr int NC = Acc<T>::N;
+  for (int j0 = 0; j0 < cnt; j0 += G) {
+    if (j0 > 0) load_group<T, E, G>(c, V, n, j0, cnt, v);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      if (j0 + g < cnt) {
+        const T cj = Acc<T>::get(cs + (j0 + g) * NC);
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] -= cj * v[g][e];
+      }
+  }
+}
+
+// partN[blk] = sum |x_i|^2 over the chunk; starts a Lanczos call.
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_norm(const T* __restrict__ x, size_t n,
+                                            double* __restrict__ partN, double* scal) {
+  __shared__ double sh[NW];
+  const Chunk<E> c(n);
+  T v[E];
+  c.load(x, v);
+  const double s = block_sum(sum_abs2<T, E>(v), sh);
+  if (threadIdx.x == 0) partN[blockIdx.x] = s;
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[2] = 1e30;
 }
 
 __device__ inline double u_pm1(uint64_t seed, uint64_t k) {
@@ -125,356 +171,542 @@ template <> __device__ inline cdouble rand_entry<cdouble>(uint64_t seed, uint64_
   return cdouble(u_pm1(seed, 2 * idx) * scale, u_pm1(seed, 2 * idx + 1) * scale);
 }
 
-// Fill x from the stream; with partN given, only when sqrt(sum partN) < thr.
+// Fill x from the stream.
 template <class T>
 __global__ __launch_bounds__(NT) void k_fill_random(T* x, size_t n, uint64_t seed, uint64_t offset,
-                                                   double scale, const double* partN, int nbp,
-                                                   double thr) {
-  __shared__ double sh[NT / 64];
-  if (partN && !(sqrt(sum_parts(partN, nbp, sh)) < thr)) return;
+                                                   double scale) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
     x[i] = rand_entry<T>(seed, offset + i, scale);
 }
 
-// nrm = sqrt(sum partN); scal[0] = nrm, scal[1] = 1/nrm (0 if nrm <= 1e-300),
-// *beta_out = nrm (if given); dst = src / nrm (if dst given).
-template <class T>
-__global__ __launch_bounds__(NT) void k_scale(T* dst, const T* src, size_t n,
+// x <- the stream when sqrt(sum partN) < thr; partO: the norm partials of the
+// result.
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_fill_small(T* x, size_t n, uint64_t seed, double thr,
+                                                  const double* __restrict__ partN,
+                                                  double* __restrict__ partO) {
+  __shared__ double sh[NW];
+  if (!(sqrt(sum_parts(partN, gridDim.x)) < thr)) {
+    if (threadIdx.x == 0) partO[blockIdx.x] = partN[blockIdx.x];
+    return;
+  }
+  const Chunk<E> c(n);
+  T v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = c.in[e] ? rand_entry<T>(seed, c.idx[e], 1.0) : T(0);
+  c.store(x, v);
+  const double s = block_sum(sum_abs2<T, E>(v), sh);
+  if (threadIdx.x == 0) partO[blockIdx.x] = s;
+}
+
+// scal[0] = nrm, scal[1] = s, *beta = nrm; host[0] = nrm, host[3] = scal[3] (each if given)
+__device__ inline void put_norm(double nrm, double s, double* scal, double* beta, double* host) {
+  scal[0] = nrm;
+  scal[1] = s;
+  if (beta) *beta = nrm;
+  if (host) {
+    host[0] = nrm;
+    host[3] = scal[3];
+  }
+}
+__device__ inline double inv_norm(double nrm) { return (nrm > 1e-300) ? 1.0 / nrm : 0.0; }
+
+// nrm = sqrt(sum partN); dst = src / nrm (if dst given; zero if nrm <= 1e-300).
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_scale(T* dst, const T* src, size_t n,
                                              const double* __restrict__ partN, int nbp,
-                                             double* scal, double* beta_out) {
-  __shared__ double sh[NT / 64];
-  const double nrm = sqrt(sum_parts(partN, nbp, sh));
-  const double s = (nrm > 1e-300) ? 1.0 / nrm : 0.0;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    scal[0] = nrm;
-    scal[1] = s;
-    if (beta_out) *beta_out = nrm;
-  }
+                                             double* scal, double* beta_out, double* host) {
+  const Chunk<E> c(n);
+  T v[E];
+  c.load(src, v);
+  const double nrm = sqrt(sum_parts(partN, nbp));
+  const double s = inv_norm(nrm);
+  if (blockIdx.x == 0 && threadIdx.x == 0) put_norm(nrm, s, scal, beta_out, host);
   if (!dst) return;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    dst[i] = src[i] * s;
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = v[e] * s;
+  c.store(dst, v);
 }
 
-// partA[blk] = Re <v, w> over the workgroup's chunk.
-template <class T>
-__global__ __launch_bounds__(NT) void k_alpha(const T* __restrict__ v, const T* __restrict__ w,
+// partA[blk] = Re <v, w> over the chunk.
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_alpha(const T* __restrict__ v, const T* __restrict__ w,
                                              size_t n, double* __restrict__ partA) {
-  __shared__ double sh[NT / 64];
-  size_t b, e;
-  chunk_range(n, b, e);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  size_t i = b + threadIdx.x;
-  for (; i + 3 * NT < e; i += 4 * NT) {
-    a0 += real(conj(v[i]) * w[i]);
-    a1 += real(conj(v[i + NT]) * w[i + NT]);
-    a2 += real(conj(v[i + 2 * NT]) * w[i + 2 * NT]);
-    a3 += real(conj(v[i + 3 * NT]) * w[i + 3 * NT]);
-  }
-  for (; i < e; i += NT) a0 += real(conj(v[i]) * w[i]);
-  const double vv[1] = {(a0 + a1) + (a2 + a3)};
-  write_parts<1>(vv, 1, partA, 0, gridDim.x, sh);
+  __shared__ double sh[NW];
+  const Chunk<E> c(n);
+  T a[E], b[E];
+  c.load(v, a);
+  c.load(w, b);
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) s += real(conj(a[e]) * b[e]);
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) partA[blockIdx.x] = s;
 }
 
-// out[it] = sum partA (one workgroup).
-__global__ __launch_bounds__(NT) void k_alpha_value(const double* __restrict__ partA, int nbp,
+// out[it] = sum partA (one wave).
+__global__ __launch_bounds__(64) void k_alpha_value(const double* __restrict__ partA, int nbp,
                                                     double* alpha, int it) {
-  __shared__ double sh[NT / 64];
-  const double a = sum_parts(partA, nbp, sh);
+  const double a = sum_parts(partA, nbp);
   if (threadIdx.x == 0) alpha[it] = a;
 }
 
 // alpha[it] = sum partA;  w -= alpha v_it + beta[it-1] v_{it-1};
 // partC[(j*NC + c)*nb + blk] = component c of <v_j, w> over the chunk, j <= it.
-// Dots are taken GD vectors at a time; the first group rides on the update pass.
-template <class T>
-__global__ __launch_bounds__(NT) void k_sub_dots(T* __restrict__ w, const T* __restrict__ V,
+// One pass over the basis, bound by the L2 and the Infinity Cache; every load
+// of a group of vectors is in flight before the first sum is needed (n = 2^18,
+// 20 iterations: 17.6 -> 8.3 us on average; four waves a CU and a reduction
+// through LDS per group of eight vectors before).
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_sub_dots(T* __restrict__ w, const T* __restrict__ V,
                                                 size_t n, int it, const double* __restrict__ partA,
                                                 double* alpha, const double* beta,
                                                 double* __restrict__ partC) {
-  constexpr int NC = Acc<T>::N;
-  constexpr int GD = 8;
-  __shared__ double sh[GD * NC * (NT / 64)];
-  const int nb = gridDim.x;
-  const double a = sum_parts(partA, nb, sh);
-  if (blockIdx.x == 0 && threadIdx.x == 0) alpha[it] = a;
-  size_t b, e;
-  chunk_range(n, b, e);
+  constexpr int NC = Acc<T>::N, G = group<T, E>();
+  __shared__ double sh[128 * NC * NW];
+  const int nb = gridDim.x, cnt = it + 1;
+  const Chunk<E> c(n);
+  T x[E], vi[E], vm[E], v[G][E];
+  c.load(w, x);
+  c.load(V + (size_t)it * n, vi);
+  c.load(V + (size_t)max(it - 1, 0) * n, vm);
+  load_group<T, E, G>(c, V, n, 0, cnt, v);
+  const double a = sum_parts(partA, nb);
   const double bm = it > 0 ? beta[it - 1] : 0.0;
-  const T* vi = V + (size_t)it * n;
-  const T* vm = it > 0 ? V + (size_t)(it - 1) * n : vi;
-  for (int j0 = 0; j0 <= it; j0 += GD) {
-    const int cnt = min(GD, it + 1 - j0);
-    T acc[GD];
+  if (blockIdx.x == 0 && threadIdx.x == 0) alpha[it] = a;
 #pragma unroll
-    for (int jj = 0; jj < GD; ++jj) acc[jj] = T(0);
-    for (size_t i = b + threadIdx.x; i < e; i += NT) {
-      T x = w[i];
-      if (j0 == 0) {
-        x = x - a * vi[i];
-        if (it > 0) x = x - bm * vm[i];
-        w[i] = x;
-      }
+  for (int e = 0; e < E; ++e) {
+    x[e] = x[e] - a * vi[e];
+    if (it > 0) x[e] = x[e] - bm * vm[e];
+  }
+  c.store(w, x);
+  wave_dots<T, E, G>(c, V, n, cnt, x, v, sh);
+  __syncthreads();
+  for (int q = threadIdx.x; q < cnt * NC; q += NL) {
+    double r = 0.0;
 #pragma unroll
-      for (int jj = 0; jj < GD; ++jj)
-        if (jj < cnt) acc[jj] += conj(V[(size_t)(j0 + jj) * n + i]) * x;
-    }
-    double o[GD * NC];
-#pragma unroll
-    for (int jj = 0; jj < GD; ++jj) Acc<T>::put(acc[jj], o + jj * NC);
-    write_parts<GD * NC>(o, cnt * NC, partC, j0 * NC, nb, sh);
+    for (int i = 0; i < NW; ++i) r += sh[q * NW + i];
+    partC[(size_t)q * nb + blockIdx.x] = r;
   }
 }
 
-// cvec[g] = sum_b partC[g*nb + b] (doubles; one workgroup per g, fixed order).
-__global__ __launch_bounds__(NT) void k_coeffs(const double* __restrict__ partC, int nb,
+// cvec[g] = sum_b partC[g*nb + b] (doubles; one wave per g, fixed order).
+__global__ __launch_bounds__(64) void k_coeffs(const double* __restrict__ partC, int nb,
                                                double* __restrict__ cvec) {
-  __shared__ double sh[NT / 64];
-  const double s = sum_parts(partC + (size_t)blockIdx.x * nb, nb, sh);
+  const double s = sum_parts(partC + (size_t)blockIdx.x * nb, nb);
   if (threadIdx.x == 0) cvec[blockIdx.x] = s;
 }
 
 // w -= sum_j c_j v_j (c from cvec, or re-reduced from partC when cvec is null);
 // partN[blk] = |w|^2 over the chunk.
-template <class T>
-__global__ __launch_bounds__(NT) void k_orth_norm(T* __restrict__ w, const T* __restrict__ V,
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_orth_norm(T* __restrict__ w, const T* __restrict__ V,
                                                  size_t n, int it, const double* __restrict__ partC,
-                                                 const T* cvec, double* __restrict__ partN) {
-  constexpr int NC = Acc<T>::N;
-  __shared__ double sh[NT / 64];
+                                                 const double* __restrict__ cvec,
+                                                 double* __restrict__ partN) {
+  constexpr int NC = Acc<T>::N, G = group<T, E>();
+  __shared__ double sh[NW];
   __shared__ double cs[128 * NC];
-  const int nb = gridDim.x;
+  const int nb = gridDim.x, cnt = it + 1;
+  const Chunk<E> c(n);
+  T x[E], v[G][E];
+  c.load(w, x);
+  load_group<T, E, G>(c, V, n, 0, cnt, v);
   if (cvec) {
-    for (int j = threadIdx.x; j <= it; j += NT) Acc<T>::put(cvec[j], cs + j * NC);
-    __syncthreads();
+    for (int q = threadIdx.x; q < cnt * NC; q += NL) cs[q] = cvec[q];
   } else {
-    sum_parts_multi(partC, nb, (it + 1) * NC, cs);
-  }
-  size_t b, e;
-  chunk_range(n, b, e);
-  double a0 = 0.0, a1 = 0.0;
-  size_t i = b + threadIdx.x;
-  for (; i + NT < e; i += 2 * NT) {
-    T x = w[i], x2 = w[i + NT];
-    for (int j = 0; j <= it; ++j) {
-      const T c = Acc<T>::get(cs + j * NC);
-      const T* vj = V + (size_t)j * n;
-      x = x - c * vj[i];
-      x2 = x2 - c * vj[i + NT];
+    for (int q = threadIdx.x >> 6; q < cnt * NC; q += NW) {
+      const double r = sum_parts(partC + (size_t)q * nb, nb);
+      if ((threadIdx.x & 63) == 0) cs[q] = r;
     }
-    w[i] = x;
-    w[i + NT] = x2;
-    a0 += abs2(x);
-    a1 += abs2(x2);
   }
-  for (; i < e; i += NT) {
-    T x = w[i];
-    for (int j = 0; j <= it; ++j) x = x - Acc<T>::get(cs + j * NC) * V[(size_t)j * n + i];
-    w[i] = x;
-    a0 += abs2(x);
-  }
-  const double v[1] = {a0 + a1};
-  write_parts<1>(v, 1, partN, 0, nb, sh);
+  __syncthreads();
+  sub_basis<T, E, G>(c, V, n, cnt, cs, x, v);
+  c.store(w, x);
+  const double s = block_sum(sum_abs2<T, E>(x), sh);
+  if (threadIdx.x == 0) partN[blockIdx.x] = s;
 }
 
 // out = sum_j y_j v_j; partN[blk] = |out|^2 over the chunk.
-template <class T>
-__global__ __launch_bounds__(NT) void k_ritz(T* __restrict__ out, const T* __restrict__ V, size_t n,
-                                            int niter, const double* y, double* __restrict__ partN) {
-  __shared__ double sh[NT / 64];
-  __shared__ double ys[128];
-  for (int j = threadIdx.x; j < niter; j += NT) ys[j] = y[j];
-  __syncthreads();
-  size_t b, e;
-  chunk_range(n, b, e);
-  double acc = 0.0;
-  for (size_t i = b + threadIdx.x; i < e; i += NT) {
-    T x = T(0);
-    for (int j = 0; j < niter; ++j) x = x + ys[j] * V[(size_t)j * n + i];
-    out[i] = x;
-    acc += abs2(x);
+template <class T, int E>
+__device__ inline double ritz_chunk(const Chunk<E>& c, const T* __restrict__ V, size_t n, int niter,
+                                    const double* ys, T (&x)[E]) {
+  constexpr int G = group<T, E>();
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = T(0);
+  for (int j0 = 0; j0 < niter; j0 += G) {
+    T v[G][E];
+    load_group<T, E, G>(c, V, n, j0, niter, v);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+      if (j0 + g < niter)
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] += ys[j0 + g] * v[g][e];
   }
-  const double v[1] = {acc};
-  write_parts<1>(v, 1, partN, 0, gridDim.x, sh);
+  return sum_abs2<T, E>(x);
+}
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_ritz(T* __restrict__ out, const T* __restrict__ V, size_t n,
+                                            int niter, const double* y, double* __restrict__ partN) {
+  __shared__ double sh[NW];
+  __shared__ double ys[128];
+  for (int j = threadIdx.x; j < niter; j += NL) ys[j] = y[j];
+  __syncthreads();
+  const Chunk<E> c(n);
+  T x[E];
+  const double s = block_sum(ritz_chunk<T, E>(c, V, n, niter, ys, x), sh);
+  c.store(out, x);
+  if (threadIdx.x == 0) partN[blockIdx.x] = s;
+}
+
+// ---------------------------------------------------------------------------
+// Vectors of at most LZ_ONE elements: one workgroup holds the vector, so an
+// iteration's four kernels (and the three at either end of a call) are one.
+// Such launches cost their latency, not their work (20 iterations with the
+// two-site operator, one workgroup against four kernels: n = 256 473 us against
+// 676, 1024 500 against 688).  Past LZ_ONE the basis through one CU takes what
+// the launches save (n = 2304 717 against 721, 6400 1138 against 782).
+// ---------------------------------------------------------------------------
+// v_0 = theta / |theta|, theta replaced by the stream when |theta| < thr.
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_one_start(T* theta, T* v0, size_t n, uint64_t seed,
+                                                 double thr, double* scal) {
+  __shared__ double sh[NW];
+  const Chunk<E> c(n);
+  T x[E];
+  c.load(theta, x);
+  double nrm = sqrt(block_sum(sum_abs2<T, E>(x), sh));
+  if (nrm < thr) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = c.in[e] ? rand_entry<T>(seed, c.idx[e], 1.0) : T(0);
+    c.store(theta, x);
+    nrm = sqrt(block_sum(sum_abs2<T, E>(x), sh));
+  }
+  const double s = inv_norm(nrm);
+  if (threadIdx.x == 0) {
+    put_norm(nrm, s, scal, nullptr, nullptr);
+    scal[2] = 1e30;
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = x[e] * s;
+  c.store(v0, x);
+}
+
+// One iteration behind w = H v_it: alpha[it], the three-term update, one
+// projection on the basis, beta[it] and v_{it+1} (if given).
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_one_step(const T* __restrict__ w, T* V, size_t n, int it,
+                                                double* alpha, double* beta, double* scal,
+                                                T* vnext) {
+  constexpr int NC = Acc<T>::N, G = group<T, E>();
+  __shared__ double sh[128 * NC * NW];
+  __shared__ double cs[128 * NC];
+  const int cnt = it + 1;
+  const Chunk<E> c(n);
+  T x[E], vi[E], vm[E], v[G][E];
+  c.load(w, x);
+  c.load(V + (size_t)it * n, vi);
+  c.load(V + (size_t)max(it - 1, 0) * n, vm);
+  load_group<T, E, G>(c, V, n, 0, cnt, v);
+  const double bm = it > 0 ? beta[it - 1] : 0.0;
+  double s = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) s += real(conj(vi[e]) * x[e]);
+  const double a = block_sum(s, sh);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    x[e] = x[e] - a * vi[e];
+    if (it > 0) x[e] = x[e] - bm * vm[e];
+  }
+  wave_dots<T, E, G>(c, V, n, cnt, x, v, sh);
+  load_group<T, E, G>(c, V, n, 0, cnt, v);
+  __syncthreads();
+  for (int q = threadIdx.x; q < cnt * NC; q += NL) {
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) r += sh[q * NW + i];
+    cs[q] = r;
+  }
+  __syncthreads();
+  sub_basis<T, E, G>(c, V, n, cnt, cs, x, v);
+  const double nrm = sqrt(block_sum(sum_abs2<T, E>(x), sh));
+  const double si = inv_norm(nrm);
+  if (threadIdx.x == 0) {
+    alpha[it] = a;
+    put_norm(nrm, si, scal, beta + it, nullptr);
+  }
+  if (!vnext) return;
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = x[e] * si;
+  c.store(vnext, x);
+}
+
+// out = V y / |V y|
+template <class T, int E>
+__global__ __launch_bounds__(NL) void k_one_ritz(T* __restrict__ out, const T* __restrict__ V,
+                                                size_t n, int niter, const double* y, double* scal,
+                                                double* host) {
+  __shared__ double sh[NW];
+  __shared__ double ys[128];
+  for (int j = threadIdx.x; j < niter; j += NL) ys[j] = y[j];
+  __syncthreads();
+  const Chunk<E> c(n);
+  T x[E];
+  const double nrm = sqrt(block_sum(ritz_chunk<T, E>(c, V, n, niter, ys, x), sh));
+  const double s = inv_norm(nrm);
+  if (threadIdx.x == 0) put_norm(nrm, s, scal, nullptr, host);
+#pragma unroll
+  for (int e = 0; e < E; ++e) x[e] = x[e] * s;
+  c.store(out, x);
 }
 
 // ---------------------------------------------------------------------------
 // Symmetric tridiagonal T(k): diagonal a[0..k), off-diagonal b[0..k-1).
 // ---------------------------------------------------------------------------
 
-__device__ inline int sturm_count(const double* a, const double* b2, int k, double x, double pivmin) {
-  double q = a[0] - x;
-  int c = q < 0.0;
-  for (int i = 1; i < k; ++i) {
-    if (fabs(q) < pivmin) q = -pivmin;
-    q = (a[i] - x) - b2[i - 1] / q;
-    c += q < 0.0;
-  }
-  return c;
-}
-
-// Lowest eigenvalue by 64-way multisection (one wave).
-__device__ double tri_lowest(const double* a, const double* b, int k, double* b2) {
-  // One wave: every lane holds the same bracket [lo, hi] (the same arithmetic
-  // on the same data), evaluates the Sturm count at one of 64 interior points
-  // per round, and a ballot gives the first point with a count >= 1.
+// Lowest eigenvalue by multisection (one wave): every lane holds the same
+// bracket [lo, hi] (the same arithmetic on the same data) and tests two of 128
+// interior points a round; ballots give the first point x at which T - x I is
+// not positive definite.  The test is the sign of the leading minors,
+// p_{i+1} = (a_i - x) p_i - b_{i-1}^2 p_{i-1}: one multiply-add of latency a
+// row where the recurrence of their ratios has a division, and as the ratios
+// exact for a matrix an eps away.  T is scaled by a power of two to entries
+// below 4 and the pair of minors every eight rows, so neither leaves the range.
+// A check of 7 to 19 rows takes 7 to 10 us (12 to 16 with divisions).
+__device__ double tri_lowest(const double* a, const double* b, int k, double* as /*[144]*/,
+                             double* b2 /*[144]*/) {
   const int t = threadIdx.x;
-  double lo = a[0], hi = a[0], mb = 0.0;
-  for (int i = 0; i < k; ++i) {
-    double r = (i > 0 ? fabs(b[i - 1]) : 0.0) + (i < k - 1 ? fabs(b[i]) : 0.0);
+  double lo = INFINITY, hi = -INFINITY, bad = 0.0;
+  for (int i = t; i < k; i += 64) {
+    const double r = (i > 0 ? fabs(b[i - 1]) : 0.0) + (i < k - 1 ? fabs(b[i]) : 0.0);
     lo = fmin(lo, a[i] - r);
     hi = fmax(hi, a[i] + r);
-    if (i < k - 1) mb = fmax(mb, b[i] * b[i]);
+    bad += 0.0 * a[i] + 0.0 * r;  // NaN for an infinite or NaN entry
   }
-  {
-    const double w = fmax(fabs(lo), fabs(hi));
-    lo -= 2.0 * DBL_EPSILON * w + DBL_MIN;
-    hi += 2.0 * DBL_EPSILON * w + DBL_MIN;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+    bad += __shfl_xor(bad, o, 64);
   }
-  const double pm = DBL_MIN * fmax(1.0, mb);
-  for (int i = t; i < k - 1; i += 64) b2[i] = b[i] * b[i];
+  if (!(bad == 0.0) || !(hi - lo < INFINITY)) return NAN;
+  const double w0 = fmax(fabs(lo), fabs(hi));
+  lo -= 2.0 * DBL_EPSILON * w0 + DBL_MIN;
+  hi += 2.0 * DBL_EPSILON * w0 + DBL_MIN;
+  const int ex = ilogb(fmax(w0, 1e-290));
+  // rows past k: a = 8 and b = 0 keep the sign of the minors
+  for (int i = t; i < 144; i += 64) {
+    as[i] = i < k ? ldexp(a[min(i, k - 1)], -ex) : 8.0;
+    const double bi = i > 0 && i < k ? ldexp(b[min(i, k - 1) - (i > 0)], -ex) : 0.0;
+    b2[i] = bi * bi;
+  }
   __syncthreads();
-  for (int round = 0; round < 24; ++round) {
+  lo = ldexp(lo, -ex);
+  hi = ldexp(hi, -ex);
+  for (int round = 0; round < 20; ++round) {
     const double w = fmax(fabs(lo), fabs(hi));
     if (hi - lo <= 2.0 * DBL_EPSILON * w + 4.0 * DBL_MIN) break;
-    const double x = lo + (hi - lo) * (double)(t + 1) / 65.0;
-    const unsigned long long m = __ballot(sturm_count(a, b2, k, x, pm) >= 1);
-    const int l = m ? __ffsll((long long)m) - 1 : 64;
-    const double nlo = (l == 0) ? lo : lo + (hi - lo) * (double)l / 65.0;
-    const double nhi = (l == 64) ? hi : lo + (hi - lo) * (double)(l + 1) / 65.0;
+    const double x0 = lo + (hi - lo) * (double)(t + 1) / 129.0;
+    const double x1 = lo + (hi - lo) * (double)(t + 65) / 129.0;
+    double p0 = 1.0, q0 = 0.0, p1 = 1.0, q1 = 0.0;
+    bool n0 = false, n1 = false;
+    double ca[8], cb[8];  // the next eight rows, read ahead of the chain
+#pragma unroll
+    for (int u = 0; u < 8; ++u) ca[u] = as[u], cb[u] = b2[u];
+    for (int i0 = 0; i0 < k; i0 += 8) {
+      double ra[8], rb[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        ra[u] = ca[u], rb[u] = cb[u];
+        ca[u] = as[i0 + 8 + u], cb[u] = b2[i0 + 8 + u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const double r0 = (ra[u] - x0) * p0 - rb[u] * q0, r1 = (ra[u] - x1) * p1 - rb[u] * q1;
+        q0 = p0, p0 = r0;
+        q1 = p1, p1 = r1;
+        n0 |= !(r0 > 0.0);
+        n1 |= !(r1 > 0.0);
+      }
+      const int e0 = __builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(q0)));
+      const int e1 = __builtin_amdgcn_frexp_exp(fmax(fabs(p1), fabs(q1)));
+      p0 = ldexp(p0, -e0), q0 = ldexp(q0, -e0);
+      p1 = ldexp(p1, -e1), q1 = ldexp(q1, -e1);
+    }
+    const unsigned long long m0 = __ballot(n0), m1 = __ballot(n1);
+    const int l = m0 ? __ffsll((long long)m0) - 1 : m1 ? 63 + __ffsll((long long)m1) : 128;
+    const double nlo = (l == 0) ? lo : lo + (hi - lo) * (double)l / 129.0;
+    const double nhi = (l == 128) ? hi : lo + (hi - lo) * (double)(l + 1) / 129.0;
     lo = nlo;
     hi = nhi;
   }
-  return 0.5 * (lo + hi);
+  return ldexp(0.5 * (lo + hi), ex);
 }
 
-// Eigenvector of T for eigenvalue lam by inverse iteration (thread 0).
-// Work arrays (5 x 128 doubles + 128 ints) live in LDS, passed by the caller.
+// Eigenvector of T for eigenvalue lam by inverse iteration (one wave): thread 0
+// factors T - lam I with partial pivoting and runs the two substitutions; the
+// wave inverts the pivots and normalises.  Work arrays in LDS.
+struct TriWork {
+  double d[128], du[128], dl[128], du2[128], x[128];
+  int piv[128];
+};
+__device__ inline double wave_max(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+  return v;
+}
 __device__ void tri_vector(const double* a, const double* b, int k, double lam, double* y,
-                           double* d, double* du, double* dl, double* du2, double* x, int* piv) {
-  if (k == 1) { y[0] = 1.0; return; }
+                           TriWork& s) {
+  const int t = threadIdx.x;
   double tnorm = 0.0;
-  for (int i = 0; i < k; ++i)
+  for (int i = t; i < k; i += 64) {
     tnorm = fmax(tnorm, fabs(a[i]) + (i > 0 ? fabs(b[i - 1]) : 0.0) + (i < k - 1 ? fabs(b[i]) : 0.0));
+    s.d[i] = a[i] - lam;
+    s.du[i] = s.dl[i] = i < k - 1 ? b[i] : 0.0;
+    s.du2[i] = 0.0;
+    s.x[i] = 1.0 + 0.25 * (double)i / (double)k;
+  }
+  tnorm = wave_max(tnorm);
   const double tiny = fmax(DBL_EPSILON * tnorm, DBL_MIN);
-  for (int i = 0; i < k; ++i) {
-    d[i] = a[i] - lam;
-    if (i < k - 1) { du[i] = b[i]; dl[i] = b[i]; }
-    du2[i] = 0.0;
-  }
-  for (int i = 0; i < k - 1; ++i) {
-    if (fabs(d[i]) >= fabs(dl[i])) {
-      if (fabs(d[i]) < tiny) d[i] = d[i] >= 0.0 ? tiny : -tiny;
-      double f = dl[i] / d[i];
-      dl[i] = f;
-      d[i + 1] -= f * du[i];
-      piv[i] = i;
-    } else {
-      double f = d[i] / dl[i];
-      d[i] = dl[i];
-      dl[i] = f;
-      double tmp = du[i];
-      du[i] = d[i + 1];
-      d[i + 1] = tmp - f * d[i + 1];
-      if (i < k - 2) {
-        du2[i] = du[i + 1];
-        du[i + 1] = -f * du[i + 1];
-      }
-      piv[i] = i + 1;
-    }
-  }
-  if (fabs(d[k - 1]) < tiny) d[k - 1] = d[k - 1] >= 0.0 ? tiny : -tiny;
-  for (int i = 0; i < k; ++i) x[i] = 1.0 + 0.25 * (double)i / (double)k;
-  for (int iter = 0; iter < 3; ++iter) {
+  __syncthreads();
+  if (t == 0) {
+    double di = s.d[0], ui = s.du[0];  // row i, as updated
     for (int i = 0; i < k - 1; ++i) {
-      if (piv[i] == i) {
-        x[i + 1] -= dl[i] * x[i];
+      const double li = s.dl[i], dn = s.d[i + 1], un = s.du[i + 1];
+      if (fabs(di) >= fabs(li)) {
+        if (fabs(di) < tiny) di = di >= 0.0 ? tiny : -tiny;
+        const double f = li / di;
+        s.d[i] = di;
+        s.du[i] = ui;
+        s.dl[i] = f;
+        s.piv[i] = 0;
+        di = dn - f * ui;
+        ui = un;
       } else {
-        double tmp = x[i];
-        x[i] = x[i + 1];
-        x[i + 1] = tmp - dl[i] * x[i];
+        const double f = di / li;
+        s.d[i] = li;
+        s.du[i] = dn;
+        s.du2[i] = un;
+        s.dl[i] = f;
+        s.piv[i] = 1;
+        di = ui - f * dn;
+        ui = -f * un;
       }
     }
-    x[k - 1] /= d[k - 1];
-    if (k > 1) x[k - 2] = (x[k - 2] - du[k - 2] * x[k - 1]) / d[k - 2];
-    for (int i = k - 3; i >= 0; --i) x[i] = (x[i] - du[i] * x[i + 1] - du2[i] * x[i + 2]) / d[i];
-    double s = 0.0, mx = 0.0;
-    for (int i = 0; i < k; ++i) s += x[i] * x[i], mx = fmax(mx, fabs(x[i]));
-    // rescale first to avoid overflow of the next solve
-    double inv = 1.0 / sqrt(s);
-    for (int i = 0; i < k; ++i) x[i] *= inv;
-    (void)mx;
+    s.d[k - 1] = fabs(di) < tiny ? (di >= 0.0 ? tiny : -tiny) : di;
   }
-  // deterministic sign: largest-magnitude component positive
-  int im = 0;
-  for (int i = 1; i < k; ++i)
-    if (fabs(x[i]) > fabs(x[im])) im = i;
-  double sg = x[im] < 0.0 ? -1.0 : 1.0;
-  for (int i = 0; i < k; ++i) y[i] = sg * x[i];
+  __syncthreads();
+  for (int i = t; i < k; i += 64) s.d[i] = 1.0 / s.d[i];
+  __syncthreads();
+  for (int iter = 0; iter < 3; ++iter) {
+    if (t == 0) {
+      double xi = s.x[0];
+#pragma unroll 4
+      for (int i = 0; i < k - 1; ++i) {
+        const double xn = s.x[i + 1], f = s.dl[i];
+        const bool p = s.piv[i] != 0;
+        const double top = p ? xn : xi, low = p ? xi : xn;
+        s.x[i] = top;
+        xi = low - f * top;
+      }
+      double x1 = xi * s.d[k - 1], x2 = 0.0;
+      s.x[k - 1] = x1;
+#pragma unroll 4
+      for (int i = k - 2; i >= 0; --i) {
+        const double v = ((s.x[i] - s.du2[i] * x2) - s.du[i] * x1) * s.d[i];
+        s.x[i] = v;
+        x2 = x1;
+        x1 = v;
+      }
+    }
+    __syncthreads();
+    // by the largest entry, then to unit length: no square leaves the range
+    double mx = 0.0, q = 0.0;
+    for (int i = t; i < k; i += 64) mx = fmax(mx, fabs(s.x[i]));
+    mx = wave_max(mx);
+    for (int i = t; i < k; i += 64) {
+      const double v = s.x[i] / mx;
+      q += v * v;
+    }
+    const double inv = 1.0 / sqrt(wave_sum_all(q));
+    for (int i = t; i < k; i += 64) s.x[i] = s.x[i] / mx * inv;
+    __syncthreads();
+  }
+  // deterministic sign: largest-magnitude component (the first of equals) positive
+  double mx = 0.0;
+  for (int i = t; i < k; i += 64) mx = fmax(mx, fabs(s.x[i]));
+  mx = wave_max(mx);
+  unsigned long long at = 0;
+  double sg = 1.0;
+  for (int i0 = 0; i0 < k && at == 0; i0 += 64) {
+    const double v = i0 + t < k ? s.x[i0 + t] : 0.0;
+    at = __ballot(i0 + t < k && fabs(v) == mx);
+    if (at) sg = __shfl(v, __ffsll((long long)at) - 1, 64) < 0.0 ? -1.0 : 1.0;
+  }
+  for (int i = t; i < k; i += 64) y[i] = sg * s.x[i];
 }
 
+// mode 0: convergence check (status[0] = stop, status[1] = niter; status may be
+// host memory); mode 1: scal[3] = lowest eigenvalue, y = its vector.
 __global__ __launch_bounds__(64) void k_tri(const double* alpha, const double* beta, int k, int mode,
                                            double beta_tol, double eig_tol, double eig_rel,
                                            double* scal, int* status, double* y) {
-  __shared__ double b2[128];
+  __shared__ double ts[144], b2[144];
   __shared__ double as[128], bs[128];  // the tridiagonal, read once from HBM
-  __shared__ int bidx;
-  __shared__ double wd[128], wdu[128], wdl[128], wdu2[128], wx[128];
-  __shared__ int wpiv[128];
+  __shared__ TriWork work;
   const int t = threadIdx.x;
   for (int i = t; i < k; i += 64) {
     as[i] = alpha[i];
-    bs[i] = beta[i];
+    bs[i] = mode == 0 || i < k - 1 ? beta[i] : 0.0;
   }
   __syncthreads();
-  alpha = as;
-  beta = bs;
   if (mode == 0) {  // check
-    if (t == 0) {
-      bidx = -1;
-      for (int j = 0; j < k; ++j)
-        if (beta[j] < beta_tol) { bidx = j; break; }
+    int bidx = -1;
+    for (int j0 = 0; j0 < k && bidx < 0; j0 += 64) {
+      const unsigned long long m = __ballot(j0 + t < k && bs[min(j0 + t, k - 1)] < beta_tol);
+      if (m) bidx = j0 + __ffsll((long long)m) - 1;
     }
-    __syncthreads();
     if (bidx >= 0) {
       if (t == 0) { status[0] = 1; status[1] = bidx + 1; }
       return;
     }
-    double lam = tri_lowest(alpha, beta, k, b2);
+    const double lam = k == 1 ? as[0] : tri_lowest(as, bs, k, ts, b2);
     if (t == 0) {
       scal[4] = lam;
-      double prev = scal[2];
-      if (fabs(lam - prev) < fmax(eig_tol, eig_rel * fabs(lam))) { status[0] = 1; status[1] = k; }
-      else { status[0] = 0; scal[2] = lam; }
+      const double prev = scal[2];
+      const bool stop = fabs(lam - prev) < fmax(eig_tol, eig_rel * fabs(lam));
+      status[0] = stop;
+      if (stop) status[1] = k;
+      else scal[2] = lam;
     }
   } else {  // final
-    double lam = (k == 1) ? alpha[0] : tri_lowest(alpha, beta, k, b2);
-    if (t == 0) {
-      scal[3] = lam;
-      tri_vector(alpha, beta, k, lam, y, wd, wdu, wdl, wdu2, wx, wpiv);
+    const double lam = (k == 1) ? as[0] : tri_lowest(as, bs, k, ts, b2);
+    if (t == 0) scal[3] = lam;
+    if (k == 1) {
+      if (t == 0) y[0] = 1.0;
+    } else {
+      tri_vector(as, bs, k, lam, y, work);
     }
   }
 }
 
-__global__ void k_lz_reset(double* scal, int* status) {
-  scal[2] = 1e30;
-  status[0] = 0;
-  status[1] = 0;
-}
-
 }  // namespace
 
-int lz_blocks(size_t n) {
-  // one workgroup per 1024 elements up to 1024 workgroups (C4, n = 2^20: the
-  // projections of iteration 9 take 28 us against 35 with 512 workgroups)
-  size_t nb = (n + 1023) / 1024;
-  if (nb < 1) nb = 1;
-  if (nb > 1024) nb = 1024;
-  return (int)nb;
-}
+namespace {
+constexpr size_t LZ_ONE = 2 * NL;
+// Elements a thread holds: 1 to 2^18, 2 to 2^19, then 4.
+int lz_elems(size_t n) { return n <= (size_t)256 * NL ? 1 : n <= (size_t)512 * NL ? 2 : 4; }
+bool lz_one(size_t n) { return n <= LZ_ONE; }
+}  // namespace
 
-size_t lz_part_doubles(int kmax, size_t n) { return (size_t)(2 * kmax + 2) * lz_blocks(n); }
+int lz_blocks(size_t n) { return std::max(1, (int)cdiv(n, (size_t)NL * lz_elems(n))); }
+
+size_t lz_part_doubles(int kmax, size_t n) {
+  // for every length up to n
+  const size_t nb = std::max<size_t>(lz_blocks(n), std::min<size_t>(256, cdiv(std::max<size_t>(n, 1), NL)));
+  return (2 * (size_t)kmax + 2) * nb;
+}
 
 void LzDev::alloc(int kmax_, size_t part_bytes_, size_t elem_bytes) {
   release();
@@ -484,7 +716,6 @@ void LzDev::alloc(int kmax_, size_t part_bytes_, size_t elem_bytes) {
   DMRG_HIP(hipMalloc(&beta, kmax * sizeof(double)));
   DMRG_HIP(hipMalloc(&y, kmax * sizeof(double)));
   DMRG_HIP(hipMalloc(&scal, 8 * sizeof(double)));
-  DMRG_HIP(hipMalloc(&status, 4 * sizeof(int)));
   DMRG_HIP(hipMalloc(&part, part_bytes));
   DMRG_HIP(hipMalloc(&cvec, kmax * elem_bytes));
   DMRG_HIP(hipMemset(alpha, 0, kmax * sizeof(double)));
@@ -492,10 +723,9 @@ void LzDev::alloc(int kmax_, size_t part_bytes_, size_t elem_bytes) {
 }
 
 void LzDev::release() {
-  for (void* p : {(void*)alpha, (void*)beta, (void*)y, (void*)scal, (void*)status, part, cvec})
+  for (void* p : {(void*)alpha, (void*)beta, (void*)y, (void*)scal, part, cvec})
     if (p) (void)hipFree(p);
   alpha = beta = y = scal = nullptr;
-  status = nullptr;
   part = cvec = nullptr;
 }
 
@@ -511,123 +741,120 @@ inline void need_parts(const LzDev& d, size_t n, int cnt) {
 }
 }  // namespace
 
-template <class T>
-void lz_norm(hipStream_t st, LzDev& d, const T* x, size_t n) {
-  const int nb = lz_blocks(n);
-  need_parts(d, n, 0);
-  hipLaunchKernelGGL(k_norm<T>, dim3(nb), dim3(NT), 0, st, x, n, partN(d, nb));
-  DMRG_LAUNCH_CHECK();
-}
+// Launch KERNEL<T, E> with the E of length n.
+#define DMRG_LZ(KERNEL, ...)                                                                   \
+  do {                                                                                         \
+    const dim3 g_(lz_blocks(n)), b_(NL);                                                       \
+    switch (lz_elems(n)) {                                                                     \
+      case 1: hipLaunchKernelGGL((KERNEL<T, 1>), g_, b_, 0, st, __VA_ARGS__); break;           \
+      case 2: hipLaunchKernelGGL((KERNEL<T, 2>), g_, b_, 0, st, __VA_ARGS__); break;           \
+      default: hipLaunchKernelGGL((KERNEL<T, 4>), g_, b_, 0, st, __VA_ARGS__);                 \
+    }                                                                                          \
+    DMRG_LAUNCH_CHECK();                                                                       \
+  } while (0)
+// The same with one workgroup, n <= LZ_ONE.
+#define DMRG_LZ_ONE(KERNEL, ...)                                                               \
+  do {                                                                                         \
+    const dim3 g_(1), b_(NL);                                                                  \
+    if (n <= NL) hipLaunchKernelGGL((KERNEL<T, 1>), g_, b_, 0, st, __VA_ARGS__);               \
+    else hipLaunchKernelGGL((KERNEL<T, 2>), g_, b_, 0, st, __VA_ARGS__);                       \
+    DMRG_LAUNCH_CHECK();                                                                       \
+  } while (0)
 
 template <class T>
-void lz_fill_if_small(hipStream_t st, LzDev& d, T* x, size_t n, uint64_t seed, double thr) {
+void lz_start(hipStream_t st, LzDev& d, T* theta, T* v0, size_t n, uint64_t seed, double thr) {
+  if (lz_one(n)) {
+    DMRG_LZ_ONE(k_one_start, theta, v0, n, seed, thr, d.scal);
+    return;
+  }
   const int nb = lz_blocks(n);
-  hipLaunchKernelGGL(k_fill_random<T>, dim3(std::min<size_t>(cdiv(n, NT), 2048)), dim3(NT), 0, st,
-                     x, n, seed, 0ull, 1.0, (const double*)partN(d, nb), nb, thr);
-  DMRG_LAUNCH_CHECK();
+  need_parts(d, n, 0);
+  DMRG_LZ(k_norm, theta, n, partN(d, nb), d.scal);
+  DMRG_LZ(k_fill_small, theta, n, seed, thr, (const double*)partN(d, nb), partA(d));
+  DMRG_LZ(k_scale, v0, (const T*)theta, n, (const double*)partA(d), nb, d.scal, (double*)nullptr,
+          (double*)nullptr);
 }
 
 template <class T>
 void fill_random(hipStream_t st, T* x, size_t n, uint64_t seed, uint64_t offset, double scale) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_fill_random<T>, dim3(std::min<size_t>(cdiv(n, NT), 2048)), dim3(NT), 0, st,
-                     x, n, seed, offset, scale, (const double*)nullptr, 0, 0.0);
+                     x, n, seed, offset, scale);
   DMRG_LAUNCH_CHECK();
 }
 
 template <class T>
-void lz_scale(hipStream_t st, LzDev& d, T* dst, const T* src, size_t n, double* beta_out) {
-  const int nb = lz_blocks(n);
-  hipLaunchKernelGGL(k_scale<T>, dim3(nb), dim3(NT), 0, st, dst, src, n,
-                     (const double*)partN(d, nb), nb, d.scal, beta_out);
-  DMRG_LAUNCH_CHECK();
-}
-
-template <class T>
-void lz_next(hipStream_t st, LzDev& d, T* vnext, const T* w, size_t n, int it) {
-  lz_scale<T>(st, d, vnext, w, n, d.beta + it);
-}
-
-template <class T>
-void lz_alpha(hipStream_t st, LzDev& d, const T* v, const T* w, size_t n, int it) {
-  (void)it;
-  const int nb = lz_blocks(n);
-  hipLaunchKernelGGL(k_alpha<T>, dim3(nb), dim3(NT), 0, st, v, w, n, partA(d));
-  DMRG_LAUNCH_CHECK();
-}
-
-void lz_alpha_value(hipStream_t st, LzDev& d, size_t n, int it) {
-  hipLaunchKernelGGL(k_alpha_value, dim3(1), dim3(NT), 0, st, (const double*)partA(d),
-                     lz_blocks(n), d.alpha, it);
-  DMRG_LAUNCH_CHECK();
-}
-
-template <class T>
-void lz_sub_dots(hipStream_t st, LzDev& d, T* w, const T* V, size_t n, int it) {
+void lz_step(hipStream_t st, LzDev& d, T* w, T* V, size_t n, int it, bool next) {
   DMRG_REQUIRE(it < d.kmax && it < 128, "lanczos: Krylov dimension exceeds 128");
-  need_parts(d, n, (it + 1) * Acc<T>::N);
+  const int cnt = (it + 1) * Acc<T>::N;
+  T* const vnext = next ? V + (size_t)(it + 1) * n : nullptr;
+  if (lz_one(n)) {
+    DMRG_LZ_ONE(k_one_step, (const T*)w, V, n, it, d.alpha, d.beta, d.scal, vnext);
+    return;
+  }
+  need_parts(d, n, cnt);
   const int nb = lz_blocks(n);
-  hipLaunchKernelGGL(k_sub_dots<T>, dim3(nb), dim3(NT), 0, st, w, V, n, it,
-                     (const double*)partA(d), d.alpha, (const double*)d.beta, partC(d, nb));
-  DMRG_LAUNCH_CHECK();
+  DMRG_LZ(k_alpha, (const T*)V + (size_t)it * n, (const T*)w, n, partA(d));
+  DMRG_LZ(k_sub_dots, w, (const T*)V, n, it, (const double*)partA(d), d.alpha,
+          (const double*)d.beta, partC(d, nb));
+  // every workgroup re-reduces the coefficients up to 256 partials each (n =
+  // 2^18, 20 iterations: 6.3 us a time against 5.6 and 4.2 for a kernel of
+  // its own); past that a wave per coefficient reduces them first
+  const double* cv = nullptr;
+  if (nb > 256) {
+    hipLaunchKernelGGL(k_coeffs, dim3(cnt), dim3(64), 0, st, (const double*)partC(d, nb), nb,
+                       (double*)d.cvec);
+    cv = (const double*)d.cvec;
+  }
+  DMRG_LZ(k_orth_norm, w, (const T*)V, n, it, (const double*)partC(d, nb), cv, partN(d, nb));
+  DMRG_LZ(k_scale, vnext, (const T*)w, n, (const double*)partN(d, nb), nb, d.scal, d.beta + it,
+          (double*)nullptr);
 }
 
 template <class T>
-void lz_orth_norm(hipStream_t st, LzDev& d, T* w, const T* V, size_t n, int it) {
-  const int nb = lz_blocks(n);
-  const int cnt = (it + 1) * Acc<T>::N;
-  // every workgroup re-reduces the coefficients while that stays small; past
-  // that one workgroup per coefficient reduces them first (C4, n = 2^20, 1024
-  // workgroups: 19 us against 24 at iteration 9, 30 against 43 at 19)
-  const T* cv = nullptr;
-  if ((size_t)cnt * nb > 1024) {
-    hipLaunchKernelGGL(k_coeffs, dim3(cnt), dim3(NT), 0, st, (const double*)partC(d, nb), nb,
-                       (double*)d.cvec);
-    cv = (const T*)d.cvec;
-  }
-  hipLaunchKernelGGL(k_orth_norm<T>, dim3(nb), dim3(NT), 0, st, w, V, n, it,
-                     (const double*)partC(d, nb), cv, partN(d, nb));
+void lz_dot(hipStream_t st, LzDev& d, const T* v, const T* w, size_t n) {
+  need_parts(d, n, 0);
+  DMRG_LZ(k_alpha, v, w, n, partA(d));
+  hipLaunchKernelGGL(k_alpha_value, dim3(1), dim3(64), 0, st, (const double*)partA(d),
+                     lz_blocks(n), d.alpha, 0);
   DMRG_LAUNCH_CHECK();
 }
 
 void lz_check(hipStream_t st, LzDev& d, int ncheck, double beta_tol, double eig_tol,
-              double eig_rel) {
+              double eig_rel, int* status) {
   DMRG_REQUIRE(ncheck <= 128, "lanczos: tridiagonal larger than 128");
   hipLaunchKernelGGL(k_tri, dim3(1), dim3(64), 0, st, d.alpha, d.beta, ncheck, 0, beta_tol, eig_tol,
-                     eig_rel, d.scal, d.status, d.y);
+                     eig_rel, d.scal, status, d.y);
   DMRG_LAUNCH_CHECK();
 }
 
 void lz_final(hipStream_t st, LzDev& d, int niter) {
   DMRG_REQUIRE(niter >= 1 && niter <= 128, "lanczos: bad Krylov dimension");
   hipLaunchKernelGGL(k_tri, dim3(1), dim3(64), 0, st, d.alpha, d.beta, niter, 1, 0.0, 0.0, 0.0,
-                     d.scal, d.status, d.y);
-  DMRG_LAUNCH_CHECK();
-}
-
-void lz_reset(hipStream_t st, LzDev& d) {
-  hipLaunchKernelGGL(k_lz_reset, dim3(1), dim3(1), 0, st, d.scal, d.status);
+                     d.scal, (int*)nullptr, d.y);
   DMRG_LAUNCH_CHECK();
 }
 
 template <class T>
-void lz_ritz(hipStream_t st, LzDev& d, T* out, const T* V, size_t n, int niter) {
+void lz_ritz(hipStream_t st, LzDev& d, T* out, const T* V, size_t n, int niter, double* host) {
   DMRG_REQUIRE(niter <= 128, "lanczos: Krylov dimension exceeds 128");
+  if (lz_one(n)) {
+    DMRG_LZ_ONE(k_one_ritz, out, V, n, niter, (const double*)d.y, d.scal, host);
+    return;
+  }
   const int nb = lz_blocks(n);
-  hipLaunchKernelGGL(k_ritz<T>, dim3(nb), dim3(NT), 0, st, out, V, n, niter, (const double*)d.y,
-                     partN(d, nb));
-  DMRG_LAUNCH_CHECK();
+  DMRG_LZ(k_ritz, out, V, n, niter, (const double*)d.y, partN(d, nb));
+  DMRG_LZ(k_scale, out, (const T*)out, n, (const double*)partN(d, nb), nb, d.scal,
+          (double*)nullptr, host);
 }
+#undef DMRG_LZ
+#undef DMRG_LZ_ONE
 
-#define DMRG_INST(T)                                                                        \
-  template void lz_norm<T>(hipStream_t, LzDev&, const T*, size_t);                          \
-  template void lz_fill_if_small<T>(hipStream_t, LzDev&, T*, size_t, uint64_t, double);     \
-  template void lz_scale<T>(hipStream_t, LzDev&, T*, const T*, size_t, double*);            \
-  template void lz_next<T>(hipStream_t, LzDev&, T*, const T*, size_t, int);                 \
-  template void lz_alpha<T>(hipStream_t, LzDev&, const T*, const T*, size_t, int);          \
-  template void lz_sub_dots<T>(hipStream_t, LzDev&, T*, const T*, size_t, int);             \
-  template void lz_orth_norm<T>(hipStream_t, LzDev&, T*, const T*, size_t, int);            \
-  template void lz_ritz<T>(hipStream_t, LzDev&, T*, const T*, size_t, int);                 \
+#define DMRG_INST(T)                                                                             \
+  template void lz_start<T>(hipStream_t, LzDev&, T*, T*, size_t, uint64_t, double);              \
+  template void lz_step<T>(hipStream_t, LzDev&, T*, T*, size_t, int, bool);                      \
+  template void lz_dot<T>(hipStream_t, LzDev&, const T*, const T*, size_t);                      \
+  template void lz_ritz<T>(hipStream_t, LzDev&, T*, const T*, size_t, int, double*);             \
   template void fill_random<T>(hipStream_t, T*, size_t, uint64_t, uint64_t, double);
 DMRG_INST(double)
 DMRG_INST(cdouble)
