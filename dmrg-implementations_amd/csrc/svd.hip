@@ -1286,20 +1286,24 @@ __global__ void k_identity(T* __restrict__ Q, int n) {
 }
 
 // Largest matrix whose panels fit the registers of one workgroup, and the
-// smallest one worth it (see jacobi).
+// smallest one of more than a single pair (splits of 40^2, 64^2, 100^2 kept to
+// half: 1200, 1420, 3100 us by sweeps alone, 770, 850, 1570 so).
 template <class T> constexpr int qr_max() { return is_cplx<T>::value ? 1536 : 2048; }
-constexpr int QR_MIN = 160;
+constexpr int QR_MIN = 64;
+// Smallest matrix for which first-order steps between cold sweeps cost less
+// than the sweep they save (equal from 64 to 140, 8.3 -> 7.3 ms at 512).
+constexpr int FO_MIN = 160;
 
 // A (Np x Np, ld Np) <- R, Q <- the unitary factor; work holds at least
-// 4 * 32 * Np + 32 * 32 values.
+// 128 Np values (64 Np for Np < 128), Tm 32 * 32.
 template <class T>
-void qr_factor(hipStream_t st, T* A, T* Q, T* work, int Np) {
+void qr_factor(hipStream_t st, T* A, T* Q, T* work, T* Tm, int Np) {
   const bool cx = is_cplx<T>::value;
   T* V = work;
-  T* U = V + (size_t)32 * Np;
-  T* W = U + (size_t)32 * Np;
-  T* Y = W + (size_t)32 * Np;
-  T* Tm = Y + (size_t)32 * Np;
+  const size_t panel = (size_t)(Np < 128 ? 16 : 32) * Np;
+  T* U = V + panel;
+  T* W = U + panel;
+  T* Y = W + panel;
   hipLaunchKernelGGL(k_identity<T>, dim3(std::min<size_t>(cdiv((size_t)Np * Np, 256), 4096)),
                      dim3(256), 0, st, Q, Np);
   for (int j0 = 0; j0 < Np;) {
@@ -1312,6 +1316,7 @@ void qr_factor(hipStream_t st, T* A, T* Q, T* work, int Np) {
                        V, Np, Tm);                                                              \
   } while (0)
     if (rows < 32) DMRG_QR(1, 1);
+    else if (Np < 128) DMRG_QR(2, 1);
     else if (rows <= 256) DMRG_QR(4, 2);
     else if (rows <= 512) DMRG_QR(8, 2);
     else if constexpr (!is_cplx<T>::value) {
@@ -1437,15 +1442,14 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     // the graded spectrum of a truncation to within a few sweeps of diagonal
     // (512^2, Schmidt values falling to 1e-6: 5 sweeps instead of 16; a bond
     // of a first DMRG sweep at chi = 128: 1 instead of 5).  A step costs about
-    // as much as one sweep of the round robin; below QR_MIN a sweep is a few
-    // rounds and costs less.
+    // as much as one sweep of the round robin at every size.
     for (int it = 0; it < 2; ++it) {
       hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np,
                          N, w.perm, nullptr);
       hipLaunchKernelGGL(k_permute<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], w.V[cur],
                          w.A[1 - cur], w.V[1 - cur], w.perm, Np);
       cur = 1 - cur;
-      qr_factor<T>(st, w.A[cur], w.W, w.Y, Np);
+      qr_factor<T>(st, w.A[cur], w.W, w.Y, w.Q, Np);
       // (R Q)^H: its upper triangle, which k_prep keeps, comes from the later,
       // smaller rows of R
       const GemmTile tl = gemm_pick_tile(Np, Np, Np, is_cplx<T>::value);
@@ -1460,7 +1464,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (last_off <= prm.tol * fro) last_off = accept_keep(w.A[cur], last_off);
     off_rel = last_off / fro;
     done = last_off <= prm.tol * fro;
-    near = last_off <= gate * fro;
+    near = Np >= FO_MIN && last_off <= gate * fro;
   }
   // Near the eigenbasis: first-order (all-pairs, GEMM-only) corrections.  They
   // run before any Jacobi sweep from a basis that was given, and between
@@ -1611,7 +1615,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (ka > 0) ++cnt.bip;
     if (ka > 0 && (++n_bip >= 4 || off > 0.1 * off_before)) bip_ok = false;
     sweeps = sw + 1;
-    if (!v_given) near = Np >= QR_MIN && off <= gate * fro;
+    if (!v_given) near = Np >= FO_MIN && off <= gate * fro;
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
   }

@@ -1,6 +1,6 @@
 """Eigen-solver and bond split without a warm start, across the sizes at which
-the QR iteration in front of the Jacobi sweeps starts (129), changes its panel
-kernel (rows 32, 256, 512, 1024) or ends (complex above 1536).
+the QR iteration in front of the Jacobi sweeps starts (33), changes its panel
+(order 96, rows 32, 256, 512, 1024), takes first-order steps (129) or ends (complex above 1536).
 
 Tolerances: the off-diagonal criterion and N eps |H| of rounding leave
 eigenvalues to 1e-12 |H| and residuals to 1e-11 sqrt(N) |H| (the bounds of the
@@ -25,7 +25,7 @@ def _spectrum(kind, N, rng):
     return rng.uniform(-3, 3, N)
 
 
-SIZES = ([(n, c, k) for n in (128, 129, 160, 161, 257, 511, 545) for c in (False, True)
+SIZES = ([(n, c, k) for n in (32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 257, 511, 545) for c in (False, True)
           for k in ("graded", "degenerate", "indefinite")]
          + [(1057, False, "graded"), (1057, False, "degenerate"), (1100, True, "graded"),
             (1536, True, "degenerate"), (1537, True, "graded"), (2048, False, "graded")])
