@@ -729,7 +729,6 @@ void Engine<T>::warm_alloc() {
   const size_t tsz = (size_t)chi * chi;
   for (T** p : {&wT[0], &wT[1], &wZ0, &wZ1, &wP, &wTmp}) dmalloc((void**)p, tsz * sizeof(T));
   dmalloc((void**)&wXw, capN * capN * sizeof(T));
-  dmalloc((void**)&wDev, (size_t)kPolarMaxIter * kPolarParts * sizeof(double));
   DMRG_HIP(hipHostMalloc((void**)&wHost, (size_t)kPolarMaxIter * kPolarParts * sizeof(double),
                          hipHostMallocDefault));
   warm_on = true;
@@ -748,8 +747,6 @@ void Engine<T>::warm_free() {
     f(*p);
     *p = nullptr;
   }
-  f(wDev);
-  wDev = nullptr;
   if (wHost) (void)hipHostFree(wHost);
   wHost = nullptr;
   warm_on = false;
@@ -773,7 +770,7 @@ const T* Engine<T>::warm_basis(int site, char dir) {
   // any T with singular values in (0, 1] has a polar factor; the basis it
   // gives is exact, and close to the new eigenbasis where the block changed
   // little, so accept every convergent start
-  if (!polar_unitary<T>(s_main, wT[wCur], cb, wZ0, wZ1, wP, wDev, wHost, 1.01, &Z)) return nullptr;
+  if (!polar_unitary<T>(s_main, wT[wCur], cb, wZ0, wZ1, wP, wHost, 1.01, &Z)) return nullptr;
   if (dir == 'R') warm_basis_left<T>(s_main, Z, cb, d, wX[wi][site], wXw);
   else warm_basis_right<T>(s_main, Z, cb, d, wX[wi][site], wXw);
   return wXw;

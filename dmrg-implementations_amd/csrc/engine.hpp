@@ -279,7 +279,6 @@ class Engine {
   std::vector<int> wAL[2], wAR[2];  // its bond dimensions (0: none)
   T* wT[2] = {nullptr, nullptr};   // running block overlap (ping-pong)
   T *wZ0 = nullptr, *wZ1 = nullptr, *wP = nullptr, *wTmp = nullptr, *wXw = nullptr;
-  double* wDev = nullptr;
   double* wHost = nullptr;  // pinned read-back of the polar iteration's deviation
   int wTr = 0, wTc = 0, wCur = 0;
   int* h_status = nullptr;

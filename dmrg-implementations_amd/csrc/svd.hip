@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_norms_part(const T* __restrict__ A, int
 // scal[0] = |rho|_F, scal[2] = trace(rho) from nb partials (one workgroup,
 // fixed order).
 __global__ __launch_bounds__(256) void k_norms_fin(const double* __restrict__ red, int nb,
-                                                   double* scal) {
+                                                   double* scal, double* host) {
   __shared__ double s1[256], s2[256];
   const int t = threadIdx.x;
   s1[t] = t < nb ? red[t] : 0.0;
@@ -147,7 +147,10 @@ __global__ __launch_bounds__(256) void k_norms_fin(const double* __restrict__ re
     if (t < o) { s1[t] += s1[t + o]; s2[t] += s2[t + o]; }
     __syncthreads();
   }
-  if (t == 0) { scal[0] = sqrt(s1[0]); scal[2] = s2[0]; }
+  if (t == 0) {
+    *host = scal[0] = sqrt(s1[0]);
+    scal[2] = s2[0];
+  }
 }
 
 // rank[i] = position of diagonal entry i in the stable descending order of
@@ -838,7 +841,8 @@ __global__ __launch_bounds__(256) void k_vecnorm(const T* __restrict__ Y, int ld
 // basis of the kept space).
 __global__ __launch_bounds__(256) void k_rank(const double* __restrict__ sigma,
                                               const double* __restrict__ gdiag, int k,
-                                              double cutoff, double rel, double* scal, int* newk) {
+                                              double cutoff, double rel, const double* scal,
+                                              double* disc, int* newk) {
   __shared__ int first[256];
   __shared__ double part[256];
   const int t = threadIdx.x;
@@ -864,7 +868,7 @@ __global__ __launch_bounds__(256) void k_rank(const double* __restrict__ sigma,
     __syncthreads();
   }
   if (t == 0) {
-    scal[1] = fmax(scal[2] - part[0], 0.0);
+    *disc = fmax(scal[2] - part[0], 0.0);
     *newk = nk;
   }
 }
@@ -1375,13 +1379,25 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   {
     const int nbr = (int)std::min<size_t>(NRED, std::max<size_t>(1, cdiv(tot, 4096)));
     hipLaunchKernelGGL(k_norms_part<T>, dim3(nbr), dim3(256), 0, st, w.A[0], N, Np, w.red);
-    hipLaunchKernelGGL(k_norms_fin, dim3(1), dim3(256), 0, st, (const double*)w.red, nbr, w.scal);
+    hipLaunchKernelGGL(k_norms_fin, dim3(1), dim3(256), 0, st, (const double*)w.red, nbr,
+                       w.scal, w.host + NRED + 2);
   }
+  // What the host reads the kernels write to pinned memory: NRED workgroup
+  // maxima, the largest and the keep-th largest diagonal entry, |rho|_F.
+  double* const hp = w.host;
+  double* const kk = w.host + NRED;
+  auto measure = [&](const T* M) {
+    if (keep > 0)
+      hipLaunchKernelGGL(k_rank_diag<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, M, N, Np, keep,
+                         w.rank, kk);
+    hipLaunchKernelGGL(k_offmax<T>, dim3(NRED), dim3(256), 0, st, M, N, Np,
+                       keep > 0 ? (const int*)w.rank : nullptr, keep, hp);
+    DMRG_LAUNCH_CHECK();
+  };
+  if (v_given) measure(w.A[0]);  // read by the first of the first-order steps
   DMRG_LAUNCH_CHECK();
-  double* const hs = w.host;  // pinned: the copy engine writes it directly
-  DMRG_HIP(hipMemcpyAsync(hs, w.scal, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
   DMRG_HIP(hipStreamSynchronize(st));
-  const double fro = hs[0];
+  const double fro = w.host[NRED + 2];
   if (!(fro == fro) || std::isinf(fro)) throw Error(ST_NONFINITE, "svd: non-finite matrix entries");
   const double rot_tol = 0.125 * prm.tol;
   // One inner sweep per block pair: a second one before the pairs meet other
@@ -1400,20 +1416,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     return cur;
   }
   double key_hi = 0.0, key_keep = 0.0;  // largest and keep-th largest diagonal entry
-  double* const offpart = w.red + 2 * NRED;  // per-workgroup maxima of k_offmax
-  auto offmax = [&](const T* M) {
-    if (keep > 0)
-      hipLaunchKernelGGL(k_rank_diag<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, M, N, Np, keep,
-                         w.rank, w.red);
-    hipLaunchKernelGGL(k_offmax<T>, dim3(NRED), dim3(256), 0, st, M, N, Np,
-                       keep > 0 ? (const int*)w.rank : nullptr, keep, offpart);
-    DMRG_LAUNCH_CHECK();
-    double* const hp = w.host;         // NRED workgroup maxima
-    double* const kk = w.host + NRED;  // largest and keep-th largest diagonal entry
-    DMRG_HIP(hipMemcpyAsync(hp, offpart, NRED * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (keep > 0)
-      DMRG_HIP(hipMemcpyAsync(kk, w.red, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-    DMRG_HIP(hipStreamSynchronize(st));
+  auto read_measure = [&] {
     if (keep > 0) {
       key_hi = kk[0];
       key_keep = kk[1];
@@ -1422,6 +1425,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     for (int b = 0; b < NRED; ++b) o = std::max(o, hp[b]);
     if (std::isinf(o) || !(o == o)) throw Error(ST_NONFINITE, "svd: non-finite matrix entries");
     return o;
+  };
+  auto offmax = [&](const T* M) {
+    measure(M);
+    DMRG_HIP(hipStreamSynchronize(st));
+    return read_measure();
   };
   // subspace convergence reached: accept it, or switch to full convergence
   // when the cutoff reaches into the kept group (returns the full off-norm).
@@ -1469,7 +1477,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // Near the eigenbasis: first-order (all-pairs, GEMM-only) corrections.  They
   // run before any Jacobi sweep from a basis that was given, and between
   // sweeps from one that was not, once the measure is below the gate.
-  // `known`: the measure of w.A[0] when it has been taken already.
+  // `known`: the measure of w.A[0].
   auto first_order = [&](double known) {
     // A pair is corrected when its gap exceeds sep |A_ij| (the first-order step then
     // leaves O(|A_ij|/sep)); the subspace criterion tolerates the rougher sep.
@@ -1481,11 +1489,8 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     double sep = keep > 0 || !v_given ? 1e2 : 1e4;
     const int max_steps = keep > 0 || !v_given ? 5 : 2;
     for (int it = 0; it <= max_steps && !done; ++it) {
-      double o = known;
-      if (it > 0 || known < 0.0) {
-        o = offmax(w.A[0]);
-        if (o <= prm.tol * fro) o = accept_keep(w.A[0], o);
-      }
+      double o = it > 0 ? offmax(w.A[0]) : known;
+      if (o <= prm.tol * fro) o = accept_keep(w.A[0], o);
       const double prev = last_off;
       last_off = o;
       off_rel = o / fro;
@@ -1507,7 +1512,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       // do not certify, the reading before step 4 decides (<= 1e-8 to take
       // it, else Jacobi takes over with A and V unchanged).
       T* freeb[4] = {w.A[1], w.V[1], w.W, w.Y};  // Y holds E
-      double* const nspart = w.red + 2 * NRED;  // free while no offmax is pending
+      double* const nspart = w.host;  // free while no measure is pending
       T* Z = w.Y;
       T* P = freeb[0];
       T* Zn = freeb[1];
@@ -1517,11 +1522,9 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       DMRG_LAUNCH_CHECK();
       gemm<T>(st, OP_N, OP_N, Np, Np, Np, T(1), Z, Np, P, Np, T(0), Zn, Np, tl);
       std::swap(Z, Zn);
-      double* const dp = w.host;
-      DMRG_HIP(hipMemcpyAsync(dp, nspart, NRED * sizeof(double), hipMemcpyDeviceToHost, st));
       DMRG_HIP(hipStreamSynchronize(st));
       double d2 = 0.0;
-      for (int b = 0; b < NRED; ++b) d2 += dp[b];
+      for (int b = 0; b < NRED; ++b) d2 += nspart[b];
       if (!(d2 == d2)) break;  // non-finite generator: Jacobi
       double dl = std::sqrt(d2);  // bound on the deviation before step `last`
       int last = 0;
@@ -1540,10 +1543,9 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
         gemm<T>(st, OP_N, OP_N, Np, Np, Np, T(1), Z, Np, P, Np, T(0), Zn, Np, tl);
         std::swap(Z, Zn);
         if (check) {
-          DMRG_HIP(hipMemcpyAsync(dp, nspart, NRED * sizeof(double), hipMemcpyDeviceToHost, st));
           DMRG_HIP(hipStreamSynchronize(st));
           double c2 = 0.0;
-          for (int b = 0; b < NRED; ++b) c2 += dp[b];
+          for (int b = 0; b < NRED; ++b) c2 += nspart[b];
           unitary = c2 <= 1e-16;  // |Q^H Q - I|_F <= 1e-8 before this step (false for NaN)
         }
       }
@@ -1582,7 +1584,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
         std::swap(w.V[0], w.V[1]);
         cur = 0;
       }
-      first_order(v_given ? -1.0 : last_off);
+      first_order(v_given ? read_measure() : last_off);
       if (done) break;
     }
     // sort the diagonal, permute rho and V into the other buffer
@@ -1649,7 +1651,6 @@ void SvdWork<T>::alloc(int cap_n) {
   DMRG_HIP(hipMalloc(&sigma, cap * sizeof(double)));
   DMRG_HIP(hipMalloc(&resid, cap * sizeof(double)));
   DMRG_HIP(hipMalloc(&scal, 4 * sizeof(double)));
-  DMRG_HIP(hipMalloc(&newk, sizeof(int)));
   // every device-to-host read of the solver lands in pinned memory, so no
   // copy goes through the runtime's pageable staging path
   DMRG_HIP(hipHostMalloc((void**)&host, (2 * (size_t)cap + 2 * NRED + 16) * sizeof(double),
@@ -1664,7 +1665,7 @@ void SvdWork<T>::release() {
     if (V[i]) (void)hipFree(V[i]);
     A[i] = V[i] = nullptr;
   }
-  void* ps[] = {Y, W, Q, qflag, perm, rank, gdiag, red, sigma, resid, scal, newk};
+  void* ps[] = {Y, W, Q, qflag, perm, rank, gdiag, red, sigma, resid, scal};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   if (host) (void)hipHostFree(host);
@@ -1682,7 +1683,6 @@ void SvdWork<T>::release() {
   sigma = nullptr;
   resid = nullptr;
   scal = nullptr;
-  newk = nullptr;
   cap = 0;
 }
 
@@ -1787,10 +1787,9 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
     }
   }
   hipLaunchKernelGGL(k_rank, dim3(1), dim3(256), 0, st, (const double*)w.sigma,
-                     (const double*)w.gdiag, k, cutoff, rel_cutoff, w.scal, w.newk);
+                     (const double*)w.gdiag, k, cutoff, rel_cutoff, (const double*)w.scal,
+                     w.host, w.host_i);
   DMRG_LAUNCH_CHECK();
-  DMRG_HIP(hipMemcpyAsync(w.host_i, w.newk, sizeof(int), hipMemcpyDeviceToHost, st));
-  DMRG_HIP(hipMemcpyAsync(w.host, w.scal + 1, sizeof(double), hipMemcpyDeviceToHost, st));
   DMRG_HIP(hipStreamSynchronize(st));
   const int nk = w.host_i[0];
   const double disc = w.host[0];

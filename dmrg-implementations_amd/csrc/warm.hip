@@ -146,13 +146,13 @@ void overlap_right_step(hipStream_t st, const T* Tin, int r, int c, const T* Bol
 }
 
 template <class T>
-bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, double* dev,
-                   double* hp, double start_tol, T** Zout) {
+bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, double* hp,
+                   double start_tol, T** Zout) {
   const bool cx = is_cplx<T>::value;
   copy_dev<T>(st, Z0, Tin, (size_t)n * n);
   T* Z = Z0;
   T* Zn = Z1;
-  // dev[it*kPolarParts + blk]: workgroup maxima of |Z_it^H Z_it - I|; the host
+  // hp[it*kPolarParts + blk] (written by the kernels): workgroup maxima of |Z_it^H Z_it - I|; the host
   // reduces them after the first step and after steps 9, 11, 13, ... from the
   // fixed bound (which needs 13), or K-2, K, K+2, ... from a Gershgorin bound
   // that needs K steps to reach 1 (steps past convergence keep Z unitary
@@ -169,10 +169,8 @@ bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, doub
     gemm_herm<T>(st, OP_H, OP_N, n, n, T(1), Z, n, Z, n, P, n, gemm_pick_tile(n, n, n, cx));
     if (it == 0) {
       double* const gp = hp + 2 * (size_t)kPolarParts;  // past slots 0 and 1 of the read-back
-      hipLaunchKernelGGL(k_gersh<T>, dim3(kPolarParts), dim3(256), 0, st, (const T*)P, n, dev);
+      hipLaunchKernelGGL(k_gersh<T>, dim3(kPolarParts), dim3(256), 0, st, (const T*)P, n, gp);
       DMRG_LAUNCH_CHECK();
-      DMRG_HIP(hipMemcpyAsync(gp, dev, 3 * (size_t)kPolarParts * sizeof(double),
-                              hipMemcpyDeviceToHost, st));
       DMRG_HIP(hipStreamSynchronize(st));
       double gmin = INFINITY, h = 0.0;
       for (int b = 0; b < kPolarParts; ++b) {
@@ -194,12 +192,9 @@ bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, doub
     const double a = l < 1.0 ? std::sqrt(3.0 / (1.0 + l + l * l)) : 1.0;
     l = std::min(1.0, 0.5 * a * l * (3.0 - a * a * l * l));
     hipLaunchKernelGGL(k_ns_prep<T>, dim3(kPolarParts), dim3(256), 0, st, P, n, a,
-                       it == 0 ? nullptr : dev + (size_t)it * kPolarParts);
+                       it == 0 ? nullptr : hp + (size_t)it * kPolarParts);
     DMRG_LAUNCH_CHECK();
     if (it > 0 && ((it >= first_check && (it - first_check) % 2 == 0) || it == kPolarMaxIter - 1)) {
-      DMRG_HIP(hipMemcpyAsync(hp + (size_t)seen * kPolarParts, dev + (size_t)seen * kPolarParts,
-                              (size_t)(it + 1 - seen) * kPolarParts * sizeof(double),
-                              hipMemcpyDeviceToHost, st));
       DMRG_HIP(hipStreamSynchronize(st));
       for (int j = seen; j <= it; ++j) {
         double h = 0.0;
@@ -247,8 +242,8 @@ void warm_basis_right(hipStream_t st, const T* Z, int cR, int d, const T* X, T* 
                                      int, int, T*, T*);                                         \
   template void overlap_right_step<T>(hipStream_t, const T*, int, int, const T*, int, const T*, \
                                       int, int, T*, T*);                                        \
-  template bool polar_unitary<T>(hipStream_t, const T*, int, T*, T*, T*, double*, double*,      \
-                                 double, T**);                                                  \
+  template bool polar_unitary<T>(hipStream_t, const T*, int, T*, T*, T*, double*, double,    \
+                                 T**);                                                          \
   template void warm_basis_left<T>(hipStream_t, const T*, int, int, const T*, T*);               \
   template void warm_basis_right<T>(hipStream_t, const T*, int, int, const T*, T*);
 DMRG_WARM_INST(double)
