@@ -887,12 +887,22 @@ __global__ void k_copy_rows(const T* __restrict__ Y, int ldy, int nk, int n, T* 
 // First-order eigenvector correction of a nearly diagonal Hermitian A
 // (Np x Np, real part of the diagonal = lambda): the generator E with
 // E_ij = A_ij / (lambda_j - lambda_i) for pairs the perturbation resolves
-// (|lambda_j - lambda_i| > sep |A_ij|), 0 otherwise (left to Jacobi) and on
-// the diagonal.  E is exactly anti-Hermitian (A is Hermitian and the test is
-// symmetric), so I + E is unitary up to O(|E|^2).  One workgroup per column.
+// (|lambda_j - lambda_i| > sep |A_ij|), 0 otherwise (left to Jacobi), on the
+// diagonal and for couplings at the level of rounding: up to thr, which the
+// sweeps leave alone too, and up to thr_cross between the kept group and the
+// rest (rank on either side of keep).  Between the eigenvalues of the
+// discarded group those are noise over noise, up to 1/sep each: with them
+// |E^2| is 0.1 to 0.5 instead of 1e-4, and a step cuts the measure by sep
+// instead of squaring it (N = 1024 of an FP32 engine: two steps and a sweep a
+// split, now one or two steps; sweep of 24 sites at chi = 512 85 -> 67 ms, of
+// 32 at chi = 256 54 -> 50).  Skipping the cross couplings up to thr as well
+// costs the next Lanczos call 4 % more products.  E is exactly anti-Hermitian
+// (A is Hermitian and the test is symmetric), so I + E is unitary up to
+// O(|E|^2).  One workgroup per column.
 template <class T>
 __global__ __launch_bounds__(256) void k_oa_q(const T* __restrict__ A, T* __restrict__ Q, int N,
-                                              int Np, double sep) {
+                                              int Np, double sep, double thr, double thr_cross,
+                                              const int* __restrict__ rank, int keep) {
   const int c = blockIdx.x;
   const double lc = real(A[c + (size_t)c * Np]);
   for (int r = threadIdx.x; r < Np; r += 256) {
@@ -901,7 +911,10 @@ __global__ __launch_bounds__(256) void k_oa_q(const T* __restrict__ A, T* __rest
     if (r != c && r < N && c < N) {
       const T a = A[e];
       const double g = lc - real(A[r + (size_t)r * Np]);
-      if (fabs(g) > sep * sqrt(abs2(a))) q = a * (1.0 / g);
+      const double m = sqrt(abs2(a));
+      const bool cross = keep > 0 && (rank[r] < keep) != (rank[c] < keep);
+      const bool noise = m <= (cross ? thr_cross : thr);
+      if (!noise && fabs(g) > sep * m) q = a * (1.0 / g);
     }
     Q[e] = q;
   }
@@ -1479,15 +1492,14 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // sweeps from one that was not, once the measure is below the gate.
   // `known`: the measure of w.A[0].
   auto first_order = [&](double known) {
-    // A pair is corrected when its gap exceeds sep |A_ij| (the first-order step then
-    // leaves O(|A_ij|/sep)); the subspace criterion tolerates the rougher sep.
-    // Steps go on while each one cuts the measure at least tenfold.  Pairs
-    // near the cut whose gap is only 30-100 times their coupling stall the
-    // step at sep = 1e2; the subspace criterion then retries with sep = 30
-    // (first-order error |A_ij|/30 per step) before handing over to Jacobi.
+    // A pair is corrected when its gap exceeds sep |A_ij| (the first-order step
+    // then leaves O(|A_ij|/sep)).  Steps go on while each one cuts the measure
+    // at least tenfold.  Pairs whose gap is only 30-100 times their coupling
+    // stall the step at sep = 1e2: it is tried with sep = 30 (first-order error
+    // |A_ij|/30 per step) before the block goes to Jacobi.
     const GemmTile tl = gemm_pick_tile(Np, Np, Np, is_cplx<T>::value);
-    double sep = keep > 0 || !v_given ? 1e2 : 1e4;
-    const int max_steps = keep > 0 || !v_given ? 5 : 2;
+    double sep = 1e2;
+    const int max_steps = 5;
     for (int it = 0; it <= max_steps && !done; ++it) {
       double o = it > 0 ? offmax(w.A[0]) : known;
       if (o <= prm.tol * fro) o = accept_keep(w.A[0], o);
@@ -1497,10 +1509,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       if (o <= prm.tol * fro) { done = true; break; }
       if (it == max_steps || o > gate * fro) break;  // not perturbative: Jacobi
       if (it > 0 && o > 0.1 * prev) {                // stalled (near-degenerate pairs)
-        if (keep > 0 && sep > 30.0) sep = 30.0;
+        if (sep > 30.0) sep = 30.0;
         else break;                                  // Jacobi
       }
-      hipLaunchKernelGGL(k_oa_q<T>, dim3(Np), dim3(256), 0, st, (const T*)w.A[0], w.Y, N, Np, sep);
+      hipLaunchKernelGGL(k_oa_q<T>, dim3(Np), dim3(256), 0, st, (const T*)w.A[0], w.Y, N, Np, sep,
+                         rot_tol * fro, 0.01 * prm.tol * fro, (const int*)w.rank, keep);
       // The unitary factor Q2 of I + E by Newton-Schulz, Q <- Q (3I - Q^H Q)/2
       // from Q_0 = I + E.  Every eigenvalue x of Q^H Q - I goes to
       // -x^2 (3 - x)/4, so the Frobenius deviation delta = |Q^H Q - I|_F obeys
