@@ -39,7 +39,8 @@ void heff2_apply(hipStream_t st, const T* Lenv, const T* Renv, const T* WW, cons
   if (!fused) {
     if constexpr (std::is_same<T, float>::value) {
       if (sc.split_bf16) {
-        gemm_f32_split_bf16(st, OP_T, OP_N, D * cL, dd * cR, cL, Lenv, cL, theta, cL, sc.X, D * cL);
+        gemm_f32_split_bf16(st, OP_T, OP_N, D * cL, dd * cR, cL, Lenv, cL, theta, cL, sc.X, D * cL,
+                            sc.Y, need);
       } else {
         gemm<T>(st, OP_T, OP_N, D * cL, dd * cR, cL, one, Lenv, cL, theta, cL, zero, sc.X, D * cL,
                 pickT<T>(D * cL, dd * cR, cL));
@@ -52,17 +53,17 @@ void heff2_apply(hipStream_t st, const T* Lenv, const T* Renv, const T* WW, cons
     View2 vy{{cL, 1, (long long)cL * dd}, {dd, (long long)cL, (long long)cL * dd * cR}};
     mpo_step<T>(st, cL * cR, dd * D, D * dd, sc.X, vx, WW, sc.Y, vy);
   }
-  // out[(a' + cL ss'), b'] = sum_{(b, n)} Y * R[(b + cR n), b']
+  // out[(a' + cL ss'), b'] = sum_{(b, n)} Y * R[(b + cR n), b'].  X is free
+  // again here: it serves as the split-K workspace (`need` of it, whatever its
+  // capacity, so that the slicing depends on the shape alone)
   bool done = false;
   if constexpr (std::is_same<T, float>::value) {
     if (sc.split_bf16) {
       gemm_f32_split_bf16(st, OP_N, OP_N, cL * dd, cR, D * cR, sc.Y, cL * dd, Renv, cR * D, out,
-                          cL * dd);
+                          cL * dd, sc.X, need);
       done = true;
     }
   }
-  // X is free again here: it serves as the split-K workspace (`need` of it,
-  // whatever its capacity, so that the slicing depends on the shape alone)
   if (!done)
     done = gemm_splitk<T>(st, OP_N, OP_N, cL * dd, cR, D * cR, sc.Y, cL * dd, Renv, cR * D, out,
                           cL * dd, sc.X, need);

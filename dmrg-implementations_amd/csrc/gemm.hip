@@ -881,76 +881,72 @@ __device__ inline void split3(float x, unsigned short& h, unsigned short& m, uns
   memcpy(&l, &bl, 2);
 }
 
+// blockIdx.z is the slice of Kc values of k (a multiple of BK); its product goes
+// to C + z zstride.  The loads have no branch and run two k-tiles ahead: row
+// indices past the operand are clamped (those results are not stored), a chunk
+// past the last whole k-tile is the last one again, and the remainder of K is a
+// tile of its own behind the loop.  A branch around a load makes every wait of
+// the loop a wait for all of them: 1556 x 451 x 2255 with odd leading
+// dimensions took 124 us with checked scalar loads one tile ahead on 200
+// workgroups, 52 + 6 us in four slices now (1945 x 1804 x 389: 72 -> 40).
+struct __attribute__((packed, aligned(4))) F4u {
+  float v[4];
+};
 template <bool KFA, bool KFB>
-__global__ __launch_bounds__(256) void k_gemm_bf3(int M, int N, int K, const float* __restrict__ A,
-                                                  long long lda, const float* __restrict__ B,
-                                                  long long ldb, float* __restrict__ C,
-                                                  long long ldc) {
-  constexpr int BM = 64, BN = 64, NL = BM * BF_BK / 256;  // 8 elements of A and of B per thread
+__global__ __launch_bounds__(256) void k_gemm_bf3(int M, int N, int K, int Kc,
+                                                  const float* __restrict__ A, long long lda,
+                                                  const float* __restrict__ B, long long ldb,
+                                                  float* __restrict__ C, long long ldc,
+                                                  long long zstride) {
+  constexpr int BM = 64, BN = 64;  // 8 elements of A and of B per thread
   __shared__ __attribute__((aligned(16))) unsigned short As[2][3][BM][BF_LD];
   __shared__ __attribute__((aligned(16))) unsigned short Bs[2][3][BN][BF_LD];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  float ra[NL], rb[NL];
-  // k-fast operand: thread t holds the 8 consecutive k 8 (t%4) .. +7 of row
-  // t/4 (two 16-byte loads; one 16-byte LDS store per bf16 plane).  m-fast
-  // operand: row t%64 at k = t/64 + 4r, stored element by element.
-  auto load_op = [&](bool kfast, const float* __restrict__ X, long long ld, int rows0, int nrows,
-                     int k0, float* r) {
+  const int kb = blockIdx.z * Kc, ke = min(K, kb + Kc);
+  C += blockIdx.z * zstride;
+  // Thread t holds 8 consecutive k of one row (one 16-byte LDS store per bf16
+  // plane): k-fast operand row t/4, k = 8 (t%4) (two 16-byte loads); m-fast
+  // operand row t%64, k = 8 (t/64) (eight loads, each of 64 rows).
+  const int rowA = KFA ? t >> 2 : lane, kqA = KFA ? (t & 3) * 8 : wave * 8;
+  const int rowB = KFB ? t >> 2 : lane, kqB = KFB ? (t & 3) * 8 : wave * 8;
+  const int ga = min(m0 + rowA, M - 1), gb = min(n0 + rowB, N - 1);
+  const float* const pA = KFA ? A + ga * lda + kqA : A + ga + kqA * lda;
+  const float* const pB = KFB ? B + gb * ldb + kqB : B + gb + kqB * ldb;
+  auto load_op = [](bool kfast, const float* __restrict__ X, long long ld, int k0, float (&r)[8]) {
     if (kfast) {
-      const int row = t >> 2, kq = (t & 3) * 8;
-      const int g = rows0 + row, gk = k0 + kq;
-      const float* src = X + gk + (long long)g * ld;
-      if (g < nrows && gk + 8 <= K && (ld & 3) == 0 && ((uintptr_t)X & 15) == 0) {
-        const float4 a = reinterpret_cast<const float4*>(src)[0];
-        const float4 b = reinterpret_cast<const float4*>(src)[1];
-        r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
-        r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
-      } else {
+      const F4u u = *reinterpret_cast<const F4u*>(X + k0);
+      const F4u v = *reinterpret_cast<const F4u*>(X + k0 + 4);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) r[q] = (g < nrows && gk + q < K) ? src[q] : 0.f;
-      }
+      for (int q = 0; q < 4; ++q) r[q] = u.v[q], r[q + 4] = v.v[q];
     } else {
 #pragma unroll
-      for (int q = 0; q < NL; ++q) {
-        const int g = rows0 + (t & 63), gk = k0 + (t >> 6) + 4 * q;
-        r[q] = (g < nrows && gk < K) ? X[g + (long long)gk * ld] : 0.f;
-      }
+      for (int q = 0; q < 8; ++q) r[q] = X[(long long)(k0 + q) * ld];
     }
   };
-  auto load = [&](int k0) {
-    load_op(KFA, A, lda, m0, M, k0, ra);
-    load_op(KFB, B, ldb, n0, N, k0, rb);
-  };
-  auto store_op = [&](bool kfast, unsigned short (*S)[BM][BF_LD], const float* r) {
-    if (kfast) {
-      const int row = t >> 2, kq = (t & 3) * 8;
-      unsigned short h[8], mi[8], lo[8];
+  // the remainder: k0 + q + kq < ke only
+  auto load_tail = [&](bool kfast, const float* __restrict__ X, long long ld, int k0, int kq,
+                       float (&r)[8]) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) split3(r[q], h[q], mi[q], lo[q]);
-      uint4 v;
-      memcpy(&v, h, 16);
-      *reinterpret_cast<uint4*>(&S[0][row][kq]) = v;
-      memcpy(&v, mi, 16);
-      *reinterpret_cast<uint4*>(&S[1][row][kq]) = v;
-      memcpy(&v, lo, 16);
-      *reinterpret_cast<uint4*>(&S[2][row][kq]) = v;
-    } else {
-#pragma unroll
-      for (int q = 0; q < NL; ++q) {
-        const int row = t & 63, k = (t >> 6) + 4 * q;
-        unsigned short h, mi, lo;
-        split3(r[q], h, mi, lo);
-        S[0][row][k] = h;
-        S[1][row][k] = mi;
-        S[2][row][k] = lo;
-      }
+    for (int q = 0; q < 8; ++q) {
+      const bool in = k0 + kq + q < ke;
+      const int k = in ? k0 + q : ke - 1 - kq;
+      const float v = X[kfast ? (long long)k : (long long)k * ld];
+      r[q] = in ? v : 0.f;
     }
   };
-  auto store = [&](int buf) {
-    store_op(KFA, As[buf], ra);
-    store_op(KFB, Bs[buf], rb);
+  auto store_op = [](unsigned short (*S)[BM][BF_LD], int row, int kq, const float (&r)[8]) {
+    unsigned short h[8], mi[8], lo[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) split3(r[q], h[q], mi[q], lo[q]);
+    uint4 v;
+    memcpy(&v, h, 16);
+    *reinterpret_cast<uint4*>(&S[0][row][kq]) = v;
+    memcpy(&v, mi, 16);
+    *reinterpret_cast<uint4*>(&S[1][row][kq]) = v;
+    memcpy(&v, lo, 16);
+    *reinterpret_cast<uint4*>(&S[2][row][kq]) = v;
   };
   f4_t acc_hh[2][2], acc_x[2][2];
 #pragma unroll
@@ -958,13 +954,7 @@ __global__ __launch_bounds__(256) void k_gemm_bf3(int M, int N, int K, const flo
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc_hh[i][j] = acc_x[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
   const int li = lane & 15, lg = lane >> 4;
-  const int nk = (K + BF_BK - 1) / BF_BK;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kt & 1;
-    if (kt + 1 < nk) load((kt + 1) * BF_BK);
+  auto compute = [&](int buf) {
     bf8_t af[2][3], bfr[2][3];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -986,8 +976,47 @@ __global__ __launch_bounds__(256) void k_gemm_bf3(int M, int N, int K, const flo
         x = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[j][1], af[i][0], x, 0, 0, 0);
         acc_x[i][j] = x;
       }
-    if (kt + 1 < nk) store(buf ^ 1);
+  };
+  const int nf = (ke - kb) / BF_BK;  // whole k-tiles
+  if (nf > 0) {
+    float ra[2][8], rb[2][8];
+    auto load = [&](int kt, int s) {
+      const int k0 = kb + min(kt, nf - 1) * BF_BK;
+      load_op(KFA, pA, lda, k0, ra[s]);
+      load_op(KFB, pB, ldb, k0, rb[s]);
+    };
+    auto store = [&](int s) {
+      store_op(As[s], rowA, kqA, ra[s]);
+      store_op(Bs[s], rowB, kqB, rb[s]);
+    };
+    load(0, 0);
+    load(1, 1);
+    store(0);
+    load(2, 0);
     __syncthreads();
+    // two tiles a pass, so that registers and buffers have fixed indices
+    for (int kt = 0; kt + 1 < nf; kt += 2) {
+      compute(0);
+      store(1);
+      load(kt + 3, 1);
+      __syncthreads();
+      compute(1);
+      store(0);
+      load(kt + 4, 0);
+      __syncthreads();
+    }
+    if (nf & 1) compute(0);
+  }
+  const int kt0 = kb + nf * BF_BK;
+  if (kt0 < ke) {
+    float xa[8], xb[8];
+    load_tail(KFA, pA, lda, kt0, kqA, xa);
+    load_tail(KFB, pB, ldb, kt0, kqB, xb);
+    __syncthreads();  // the last whole tile has been read
+    store_op(As[0], rowA, kqA, xa);
+    store_op(Bs[0], rowB, kqB, xb);
+    __syncthreads();
+    compute(0);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -1001,25 +1030,6 @@ __global__ __launch_bounds__(256) void k_gemm_bf3(int M, int N, int K, const flo
       }
 }
 }  // namespace
-
-void gemm_f32_split_bf16(hipStream_t st, int opA, int opB, int M, int N, int K, const float* A,
-                         int lda, const float* B, int ldb, float* C, int ldc) {
-  DMRG_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_bf16x3: negative size");
-  DMRG_REQUIRE(opA >= 0 && opA <= 3 && opB >= 0 && opB <= 3, "gemm_bf16x3: bad op");
-  if (M == 0 || N == 0) return;
-  // op(A) (m, k): transposed storage is k-fast; op(B) (k, n): plain storage is k-fast
-  const bool kfa = op_trans(opA), kfb = !op_trans(opB);
-  const dim3 grid(cdiv(M, 64), cdiv(N, 64));
-#define DMRG_BF3(KA_, KB_) \
-  hipLaunchKernelGGL((k_gemm_bf3<KA_, KB_>), grid, dim3(256), 0, st, M, N, K, A, (long long)lda, B, \
-                     (long long)ldb, C, (long long)ldc)
-  if (kfa && kfb) DMRG_BF3(true, true);
-  else if (kfa) DMRG_BF3(true, false);
-  else if (kfb) DMRG_BF3(false, true);
-  else DMRG_BF3(false, false);
-#undef DMRG_BF3
-  DMRG_LAUNCH_CHECK();
-}
 
 namespace {
 // C[i] = sum_{z<S} W[i + z*stride] for i < M*N over an M x N block (ld ldc);
@@ -1096,6 +1106,43 @@ bool splitk_impl(hipStream_t st, int opA, int opB, int M, int N, int K, const T*
   return true;
 }
 }  // namespace
+
+void gemm_f32_split_bf16(hipStream_t st, int opA, int opB, int M, int N, int K, const float* A,
+                         int lda, const float* B, int ldb, float* C, int ldc, float* ws,
+                         size_t ws_elems) {
+  DMRG_REQUIRE(M >= 0 && N >= 0 && K >= 0, "gemm_bf16x3: negative size");
+  DMRG_REQUIRE(opA >= 0 && opA <= 3 && opB >= 0 && opB <= 3, "gemm_bf16x3: bad op");
+  if (M == 0 || N == 0) return;
+  // op(A) (m, k): transposed storage is k-fast; op(B) (k, n): plain storage is k-fast
+  const bool kfa = op_trans(opA), kfb = !op_trans(opB);
+  // Slices of k where the tiles leave the chip short of two workgroups a CU
+  // (what its LDS holds), each of eight k-tiles or more.
+  const int nkt = (int)cdiv(K, BF_BK);
+  const long long tiles = (long long)cdiv(M, 64) * cdiv(N, 64);
+  int S = 1;
+  if (ws)
+    while (S < 16 && tiles * S < 768 && nkt >= 8 * (S + 1) && (size_t)(S + 1) * M * N <= ws_elems)
+      ++S;
+  const int Kc = std::max(1, (int)cdiv(nkt, S)) * BF_BK;
+  S = std::max(1, (int)cdiv(K, Kc));  // no empty slice
+  const dim3 grid(cdiv(M, 64), cdiv(N, 64), S);
+  float* const out = S > 1 ? ws : C;
+  const long long ldo = S > 1 ? M : ldc, zs = S > 1 ? (long long)M * N : 0;
+#define DMRG_BF3(KA_, KB_)                                                                        \
+  hipLaunchKernelGGL((k_gemm_bf3<KA_, KB_>), grid, dim3(256), 0, st, M, N, K, Kc, A,              \
+                     (long long)lda, B, (long long)ldb, out, ldo, zs)
+  if (kfa && kfb) DMRG_BF3(true, true);
+  else if (kfa) DMRG_BF3(true, false);
+  else if (kfb) DMRG_BF3(false, true);
+  else DMRG_BF3(false, false);
+#undef DMRG_BF3
+  if (S > 1)
+    hipLaunchKernelGGL((k_splitk_sum<float, float>),
+                       dim3((unsigned)std::min<long long>(cdiv((size_t)M * N, 256), 4096)),
+                       dim3(256), 0, st, (const float*)ws, S, (long long)M * N, M, N, C, ldc,
+                       (const double*)nullptr, (const double*)nullptr);
+  DMRG_LAUNCH_CHECK();
+}
 
 template <class T>
 bool gemm_splitk(hipStream_t st, int opA, int opB, int M, int N, int K, const T* A, int lda,

@@ -82,9 +82,12 @@ bool gemm_nn_splitk_to_f64(hipStream_t st, int M, int N, int K, const float* A, 
 // FP32 C (M x N, ldc) = op(A) op(B) with split-BF16 products: each operand as
 // three bf16 terms, the six leading cross products on the bf16 MFMA with FP32
 // accumulation (FP32-class accuracy).  op: OP_N or OP_T (conjugation is a
-// no-op for real data); alpha = 1, beta = 0.
+// no-op for real data); alpha = 1, beta = 0.  With a workspace ws (ws_elems
+// elements) a product whose tiles leave the chip idle is cut along K and the
+// slices summed in a fixed order.
 void gemm_f32_split_bf16(hipStream_t st, int opA, int opB, int M, int N, int K, const float* A,
-                         int lda, const float* B, int ldb, float* C, int ldc);
+                         int lda, const float* B, int ldb, float* C, int ldc, float* ws = nullptr,
+                         size_t ws_elems = 0);
 
 // C = op(A) op(B) (alpha 1, beta 0) split along K into slices computed into the
 // workspace ws (ws_elems elements) and summed in a fixed order: for products
