@@ -770,7 +770,15 @@ const T* Engine<T>::warm_basis(int site, char dir) {
   // any T with singular values in (0, 1] has a polar factor; the basis it
   // gives is exact, and close to the new eigenbasis where the block changed
   // little, so accept every convergent start
-  if (!polar_unitary<T>(s_main, wT[wCur], cb, wZ0, wZ1, wP, wHost, 1.01, &Z)) return nullptr;
+  bool singular = false;
+  if (!polar_unitary<T>(s_main, wT[wCur], cb, wZ0, wZ1, wP, wHost, 1.01, &Z, &singular)) {
+    // Kept spaces that differ by a vector have no polar factor; at a cut among
+    // Schmidt values of rounding size that is so in every sweep (chi = 512,
+    // FP32: one or two of 46 splits, 10 ms each from a cold start and less than
+    // 1 ms from this basis).
+    Z = wZ0;
+    if (!singular || !qr_unitary<T>(s_main, svdw, wT[wCur], cb, Z)) return nullptr;
+  }
   if (dir == 'R') warm_basis_left<T>(s_main, Z, cb, d, wX[wi][site], wXw);
   else warm_basis_right<T>(s_main, Z, cb, d, wX[wi][site], wXw);
   return wXw;

@@ -1302,6 +1302,19 @@ __global__ void k_identity(T* __restrict__ Q, int n) {
     Q[e] = T(mod32(e, n) == div32(e, n) ? 1.0 : 0.0);
 }
 
+// out(:, j) = Q(:, j) R(j, j) / |R(j, j)| (Q(:, j) where R(j, j) = 0).
+template <class T>
+__global__ void k_qr_phase(const T* __restrict__ Q, const T* __restrict__ R, int n,
+                           T* __restrict__ out) {
+  const size_t tot = (size_t)n * n;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
+       e += (size_t)gridDim.x * blockDim.x) {
+    const T r = R[(size_t)div32(e, n) * (n + 1)];
+    const double a = sqrt(abs2(r));
+    out[e] = a > 0.0 ? Q[e] * (r * (1.0 / a)) : Q[e];
+  }
+}
+
 // Largest matrix whose panels fit the registers of one workgroup, and the
 // smallest one of more than a single pair (splits of 40^2, 64^2, 100^2 kept to
 // half: 1200, 1420, 3100 us by sweeps alone, 770, 850, 1570 so).
@@ -1310,6 +1323,9 @@ constexpr int QR_MIN = 64;
 // Smallest matrix for which first-order steps between cold sweeps cost less
 // than the sweep they save (equal from 64 to 140, 8.3 -> 7.3 ms at 512).
 constexpr int FO_MIN = 160;
+// Stalling sweeps go back to QR steps above this measure (below it the pairs left
+// are few, and the first-order steps and a sweep or two end it).
+constexpr double QR_GATE = 1e-9;
 
 // A (Np x Np, ld Np) <- R, Q <- the unitary factor; work holds at least
 // 128 Np values (64 Np for Np < 128), Tm 32 * 32.
@@ -1407,7 +1423,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
                        keep > 0 ? (const int*)w.rank : nullptr, keep, hp);
     DMRG_LAUNCH_CHECK();
   };
-  if (v_given) measure(w.A[0]);  // read by the first of the first-order steps
+  if (v_given) measure(w.A[0]);  // read behind the one synchronisation
   DMRG_LAUNCH_CHECK();
   DMRG_HIP(hipStreamSynchronize(st));
   const double fro = w.host[NRED + 2];
@@ -1456,14 +1472,14 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   bool done = false;
   double last_off = INFINITY;  // latest convergence measure (criterion in force)
   const double gate = keep > 0 ? 1e-4 : 1e-6;  // measure below which first-order steps are tried
-  bool near = v_given;                          // try them before the next sweep
-  if (!v_given && Np >= QR_MIN && Np <= qr_max<T>()) {
-    // No basis given: two steps of orthogonal iteration, Q R = rho with the
-    // columns in descending order of the diagonal, then R Q = Q^H rho Q, bring
-    // the graded spectrum of a truncation to within a few sweeps of diagonal
-    // (512^2, Schmidt values falling to 1e-6: 5 sweeps instead of 16; a bond
-    // of a first DMRG sweep at chi = 128: 1 instead of 5).  A step costs about
-    // as much as one sweep of the round robin at every size.
+  if (v_given) last_off = read_measure();
+  // Two steps of orthogonal iteration, Q R = rho with the columns in descending
+  // order of the diagonal, then R Q = Q^H rho Q, bring the graded spectrum of a
+  // truncation to within a few sweeps of diagonal (512^2, Schmidt values
+  // falling to 1e-6: 5 sweeps instead of 16; a bond of a first DMRG sweep at
+  // chi = 128: 1 instead of 5).  A step costs about as much as one sweep of the
+  // round robin at every size.
+  auto qr_steps = [&] {
     for (int it = 0; it < 2; ++it) {
       hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np,
                          N, w.perm, nullptr);
@@ -1474,7 +1490,8 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       // (R Q)^H: its upper triangle, which k_prep keeps, comes from the later,
       // smaller rows of R
       const GemmTile tl = gemm_pick_tile(Np, Np, Np, is_cplx<T>::value);
-      gemm<T>(st, OP_H, OP_H, Np, Np, Np, T(1), w.W, Np, w.A[cur], Np, T(0), w.A[1 - cur], Np, tl);
+      gemm<T>(st, OP_H, OP_H, Np, Np, Np, T(1), w.W, Np, w.A[cur], Np, T(0),
+              w.A[1 - cur], Np, tl);
       gemm<T>(st, OP_N, OP_N, Np, Np, Np, T(1), w.V[cur], Np, w.W, Np, T(0), w.V[1 - cur], Np, tl);
       cur = 1 - cur;
       hipLaunchKernelGGL(k_prep<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], w.V[cur], N, Np,
@@ -1485,6 +1502,16 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (last_off <= prm.tol * fro) last_off = accept_keep(w.A[cur], last_off);
     off_rel = last_off / fro;
     done = last_off <= prm.tol * fro;
+  };
+  const bool qr_ok = Np >= QR_MIN && Np <= qr_max<T>();
+  // Far from the eigenbasis: no basis given, or one whose measure is above the
+  // gate, as in the second sweep of a run, or sweeps that stall (9 sweeps of a
+  // 512^2 block before; splits of the first four sweeps of 32 sites at chi = 256
+  // 450 -> 300 ms).
+  const bool far = !v_given || (qr_ok && last_off > gate * fro);
+  bool near = !far;  // try first-order steps before the next sweep
+  if (far && qr_ok) {
+    qr_steps();
     near = Np >= FO_MIN && last_off <= gate * fro;
   }
   // Near the eigenbasis: first-order (all-pairs, GEMM-only) corrections.  They
@@ -1586,9 +1613,10 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       ++cnt.oa;
     }
   };
-  int fo_left = v_given ? 1 : 2;  // stages of first-order steps left to try
+  int fo_left = far ? 2 : 1;  // stages of first-order steps left to try
   bool bip_ok = true;  // bipartite sweeps allowed (revoked once one stalls)
   int n_bip = 0;
+  bool qr_left = qr_ok;
   for (int sw = 0; sw < prm.max_sweeps && !done; ++sw) {
     if (near && fo_left > 0) {
       --fo_left;
@@ -1597,7 +1625,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
         std::swap(w.V[0], w.V[1]);
         cur = 0;
       }
-      first_order(v_given ? read_measure() : last_off);
+      first_order(last_off);
       if (done) break;
     }
     // sort the diagonal, permute rho and V into the other buffer
@@ -1630,9 +1658,14 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (ka > 0) ++cnt.bip;
     if (ka > 0 && (++n_bip >= 4 || off > 0.1 * off_before)) bip_ok = false;
     sweeps = sw + 1;
-    if (!v_given) near = Np >= FO_MIN && off <= gate * fro;
+    if (far) near = Np >= FO_MIN && off <= gate * fro;
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
+    // a graded block again: sweeps that stall this far out take five to nine
+    if (!far && qr_left && off > 0.1 * off_before && off > QR_GATE * fro) {
+      qr_left = false;
+      qr_steps();
+    }
   }
   if (!done) throw Error(ST_SOLVER_NO_CONV, "svd: Jacobi eigen-solver did not converge");
   hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np, N, w.perm,
@@ -1833,6 +1866,19 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
 }
 
 template <class T>
+bool qr_unitary(hipStream_t st, SvdWork<T>& w, const T* M, int n, T* out) {
+  if (n % JP != 0 || n > qr_max<T>() || n > w.cap ||
+      (size_t)(n < 128 ? 64 : 128) * n > (size_t)w.cap * w.cap)
+    return false;
+  copy_dev<T>(st, w.A[0], M, (size_t)n * n);
+  qr_factor<T>(st, w.A[0], w.W, w.Y, w.Q, n);
+  hipLaunchKernelGGL(k_qr_phase<T>, dim3(grid_for((size_t)n * n)), dim3(256), 0, st,
+                     (const T*)w.W, (const T*)w.A[0], n, out);
+  DMRG_LAUNCH_CHECK();
+  return true;
+}
+
+template <class T>
 int heig(hipStream_t st, SvdWork<T>& w, const T* H, int N, int ldh, double* evals, T* evecs,
          int lde, const SvdParams& prm) {
   DMRG_REQUIRE(N > 0 && ldh >= N && lde >= N, "heig: bad shape");
@@ -1975,6 +2021,8 @@ template SvdResult rsvd_split<cdouble>(hipStream_t, SvdWork<cdouble>&, RsvdWork<
                                        const cdouble*, int, int, int, int, double, double, bool,
                                        cdouble*, int, cdouble*, const SvdParams&, int, int,
                                        uint64_t);
+template bool qr_unitary<double>(hipStream_t, SvdWork<double>&, const double*, int, double*);
+template bool qr_unitary<cdouble>(hipStream_t, SvdWork<cdouble>&, const cdouble*, int, cdouble*);
 template int heig<double>(hipStream_t, SvdWork<double>&, const double*, int, int, double*, double*,
                           int, const SvdParams&);
 template int heig<cdouble>(hipStream_t, SvdWork<cdouble>&, const cdouble*, int, int, double*,

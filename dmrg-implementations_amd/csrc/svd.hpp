@@ -101,6 +101,14 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
                     double* sigma_out, const SvdParams& prm, const T* warm = nullptr,
                     T* basis_out = nullptr);
 
+// out = the unitary factor Q of M = Q R with a positive diagonal of R (M and
+// out n x n, ld n): close to M where M is close to unitary, and unitary also
+// where M is singular.  Uses w's buffers.  Returns false (and does nothing)
+// unless n is a multiple of 32 that the workspace and one workgroup's panel
+// hold.
+template <class T>
+bool qr_unitary(hipStream_t st, SvdWork<T>& w, const T* M, int n, T* out);
+
 // Work space of rsvd_split: sketch, bases and the projected matrix, each
 // cap_len x cap_r, plus Gram-Schmidt scratch.
 template <class T>

@@ -147,7 +147,7 @@ void overlap_right_step(hipStream_t st, const T* Tin, int r, int c, const T* Bol
 
 template <class T>
 bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, double* hp,
-                   double start_tol, T** Zout) {
+                   double start_tol, T** Zout, bool* singular) {
   const bool cx = is_cplx<T>::value;
   copy_dev<T>(st, Z0, Tin, (size_t)n * n);
   T* Z = Z0;
@@ -205,7 +205,11 @@ bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, doub
         // a zero singular value never converges: give up when the start is
         // too far or the deviation is still O(1) after 24 steps (from
         // s = 1e-5 the scaled iteration needs about 24)
-        if (!(h == h) || (j >= 24 && h > 0.5)) return false;
+        if (!(h == h)) return false;
+        if (j >= 24 && h > 0.5) {
+          *singular = std::isfinite(h);
+          return false;
+        }
         if (h <= 1e-14) {
           *Zout = Z;
           return true;
@@ -243,7 +247,7 @@ void warm_basis_right(hipStream_t st, const T* Z, int cR, int d, const T* X, T* 
   template void overlap_right_step<T>(hipStream_t, const T*, int, int, const T*, int, const T*, \
                                       int, int, T*, T*);                                        \
   template bool polar_unitary<T>(hipStream_t, const T*, int, T*, T*, T*, double*, double,    \
-                                 T**);                                                          \
+                                 T**, bool*);                                                          \
   template void warm_basis_left<T>(hipStream_t, const T*, int, int, const T*, T*);               \
   template void warm_basis_right<T>(hipStream_t, const T*, int, int, const T*, T*);
 DMRG_WARM_INST(double)

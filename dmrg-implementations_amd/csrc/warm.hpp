@@ -44,7 +44,7 @@ constexpr double kPolarL0 = 3e-4;  // initial lower bound of the smallest singul
 // about (3/2) a per step, so the bound is a guess that costs steps when it is
 // wrong, never convergence.  Returns false (and leaves *Zout undefined) when
 // max|T^H T - I| > start_tol, when the iteration stalls (a singular value
-// near 0) or when it does not reach max|Z^H Z - I| <= 1e-14 in kPolarMaxIter
+// near 0; then *singular is set) or when it does not reach max|Z^H Z - I| <= 1e-14 in kPolarMaxIter
 // steps.  When Gershgorin's discs of Z^H Z at the first step leave out 0,
 // the square root of their lower end replaces kPolarL0 as the start bound.
 // Z0, Z1, P are n x n work buffers; hp holds kPolarMaxIter * kPolarParts pinned
@@ -52,7 +52,8 @@ constexpr double kPolarL0 = 3e-4;  // initial lower bound of the smallest singul
 // step, then every second step from two steps before the bound reaches 1
 // (from step 9 with the fixed bound).
 template <class T>
-bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, double* hp, double start_tol, T** Zout);
+bool polar_unitary(hipStream_t st, const T* Tin, int n, T* Z0, T* Z1, T* P, double* hp,
+                   double start_tol, T** Zout, bool* singular);
 
 // Left side: out[(a + cL s), j] = sum_a' conj(Z[a', a]) X[(a' + cL s), j],
 // N = cL d columns (ld N).
