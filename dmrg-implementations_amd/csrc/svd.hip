@@ -1506,9 +1506,15 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   const bool qr_ok = Np >= QR_MIN && Np <= qr_max<T>();
   // Far from the eigenbasis: no basis given, or one whose measure is above the
   // gate, as in the second sweep of a run, or sweeps that stall (9 sweeps of a
-  // 512^2 block before; splits of the first four sweeps of 32 sites at chi = 256
-  // 450 -> 300 ms).
-  const bool far = !v_given || (qr_ok && last_off > gate * fro);
+  // 512^2 block before).  A given basis goes through the QR steps only where
+  // the keep-th eigenvalue is above rounding and the cutoff: they resolve
+  // directions of rounding size that the sweeps leave mixed, and where those
+  // are kept they would fall under the cutoff and shrink the bond.
+  auto clear_cut = [&] {
+    return keep > 0 && key_keep > std::max(prm.tol * fro, 1e4 * std::max(cut_abs * cut_abs,
+                                                                         cut_rel * cut_rel * key_hi));
+  };
+  const bool far = !v_given || (qr_ok && last_off > gate * fro && clear_cut());
   bool near = !far;  // try first-order steps before the next sweep
   if (far && qr_ok) {
     qr_steps();
@@ -1662,7 +1668,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
     // a graded block again: sweeps that stall this far out take five to nine
-    if (!far && qr_left && off > 0.1 * off_before && off > QR_GATE * fro) {
+    if (!far && qr_left && clear_cut() && off > 0.1 * off_before && off > QR_GATE * fro) {
       qr_left = false;
       qr_steps();
     }

@@ -34,3 +34,17 @@ def test_warm_ends_like_cold(dmrg_amd, cplx, chi):
         eng.close()
     assert abs(E[1][-1] - E[0][-1]) < 1e-8 * abs(E[0][-1])
     assert all(abs(n - 1) < 1e-10 for n in norm.values())
+
+
+@pytest.mark.parametrize("seed", [31, 34])
+def test_full_rank_bonds_keep_their_size(dmrg_amd, seed):
+    """Bonds that are not truncated keep every vector: their smallest Schmidt
+    values are of rounding size, and a warm split must not resolve them below
+    the cutoff where the sweeps leave them mixed with the rest."""
+    L, chi = 32, 256
+    Ws = models.heisenberg_mpo(L)
+    with dmrg_amd.DMRG(L, 2, chi, 5, tol=0.0, krylov_max=20) as eng:
+        eng.set_mpo(Ws)
+        eng.initialize_mps_random(seed=seed, scale=0.1)
+        eng.run(4)
+        assert list(eng.bond_dims()) == [min(2 ** i, 2 ** (L - i), chi) for i in range(L + 1)]
