@@ -102,6 +102,16 @@ __global__ void k_prep(T* __restrict__ A, T* __restrict__ V, int N, int Np, int 
   }
 }
 
+__device__ inline double ldexp_v(double a, int e) { return ldexp(a, e); }
+__device__ inline cdouble ldexp_v(cdouble a, int e) { return cdouble(ldexp(a.x, e), ldexp(a.y, e)); }
+// A <- 2^e A (tot entries), *trace <- 2^e *trace (if given).
+template <class T>
+__global__ void k_scale_pow2(T* __restrict__ A, size_t tot, int e, double* trace) {
+  const size_t i0 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (trace && i0 == 0) *trace = ldexp(*trace, e);
+  for (size_t i = i0; i < tot; i += (size_t)gridDim.x * blockDim.x) A[i] = ldexp_v(A[i], e);
+}
+
 // V (Np x Np) = the caller's N x N basis X (ld N), identity on the padding.
 template <class T>
 __global__ void k_set_basis(T* __restrict__ V, const T* __restrict__ X, int N, int Np) {
@@ -1405,12 +1415,13 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   const size_t tot = (size_t)Np * Np;
   hipLaunchKernelGGL(k_prep<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[0], w.V[0], N, Np,
                      v_given ? 0 : 1);
-  {
+  auto norms = [&] {
     const int nbr = (int)std::min<size_t>(NRED, std::max<size_t>(1, cdiv(tot, 4096)));
     hipLaunchKernelGGL(k_norms_part<T>, dim3(nbr), dim3(256), 0, st, w.A[0], N, Np, w.red);
     hipLaunchKernelGGL(k_norms_fin, dim3(1), dim3(256), 0, st, (const double*)w.red, nbr,
                        w.scal, w.host + NRED + 2);
-  }
+  };
+  norms();
   // What the host reads the kernels write to pinned memory: NRED workgroup
   // maxima, the largest and the keep-th largest diagonal entry, |rho|_F.
   double* const hp = w.host;
@@ -1426,8 +1437,24 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   if (v_given) measure(w.A[0]);  // read behind the one synchronisation
   DMRG_LAUNCH_CHECK();
   DMRG_HIP(hipStreamSynchronize(st));
-  const double fro = w.host[NRED + 2];
+  double fro = w.host[NRED + 2];
   if (!(fro == fro) || std::isinf(fro)) throw Error(ST_NONFINITE, "svd: non-finite matrix entries");
+  // The panel reflections, the rotations and the measures square entries down
+  // to rounding size: those of a norm far from one would leave the range of a
+  // double (|rho|_F = 1e-140: the reflections dropped columns that count).  The
+  // iteration then works on 2^e rho, which is exact.
+  int e2 = 0;
+  if (fro != 0.0 && (fro < 0x1p-300 || fro > 0x1p+300)) {
+    e2 = -std::ilogb(fro);
+    hipLaunchKernelGGL(k_scale_pow2<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[0], tot, e2,
+                       (double*)nullptr);
+    norms();
+    if (v_given) measure(w.A[0]);
+    DMRG_LAUNCH_CHECK();
+    DMRG_HIP(hipStreamSynchronize(st));
+    fro = w.host[NRED + 2];
+  }
+  const double cut2 = std::ldexp(cut_abs * cut_abs, e2);  // the cutoff in units of the scaled rho
   const double rot_tol = 0.125 * prm.tol;
   // One inner sweep per block pair: a second one before the pairs meet other
   // blocks saves one outer sweep in fourteen and costs as much again (256^2,
@@ -1464,7 +1491,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // when the cutoff reaches into the kept group (returns the full off-norm).
   auto accept_keep = [&](const T* M, double o) {
     if (keep == 0) return o;
-    const double floor = 1e4 * std::max(cut_abs * cut_abs, cut_rel * cut_rel * key_hi);
+    const double floor = 1e4 * std::max(cut2, cut_rel * cut_rel * key_hi);
     if (key_keep >= floor) return o;
     keep = 0;
     return offmax(M);
@@ -1511,8 +1538,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // directions of rounding size that the sweeps leave mixed, and where those
   // are kept they would fall under the cutoff and shrink the bond.
   auto clear_cut = [&] {
-    return keep > 0 && key_keep > std::max(prm.tol * fro, 1e4 * std::max(cut_abs * cut_abs,
-                                                                         cut_rel * cut_rel * key_hi));
+    return keep > 0 && key_keep > std::max(prm.tol * fro, 1e4 * std::max(cut2, cut_rel * cut_rel * key_hi));
   };
   const bool far = !v_given || (qr_ok && last_off > gate * fro && clear_cut());
   bool near = !far;  // try first-order steps before the next sweep
@@ -1674,6 +1700,9 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     }
   }
   if (!done) throw Error(ST_SOLVER_NO_CONV, "svd: Jacobi eigen-solver did not converge");
+  if (e2 != 0)
+    hipLaunchKernelGGL(k_scale_pow2<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], tot, -e2,
+                       w.scal + 2);
   hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np, N, w.perm,
                      nullptr);
   DMRG_LAUNCH_CHECK();
