@@ -25,6 +25,14 @@ constexpr int JP = 2 * JB;   // order of one pair sub-problem
 constexpr int LDP = JP + 1;  // LDS column stride (padding)
 constexpr int NT = 256;      // threads of the pair kernels
 constexpr int SORT_MAX = 2048;
+// A kept group that reaches diagonal entries of rho below TAIL |rho|_F does not
+// go through the QR steps (see jacobi).  Bonds shrank in 7 of 450 runs of single-
+// site chains of 18 to 22 sites at chi = 256 without this rule, in one with
+// 1e-16, in none with 1e-17 or 1e-15; a chain of 32 sites at chi = 256 without
+// warm starts takes 0.46, 0.47, 0.57 and 0.76 s for three sweeps without it and
+// with 1e-17, 1e-16 and 1e-15, and 1.05 s by sweeps alone.  The largest of these:
+// it is next to the tolerance of the sweeps, which is what leaves the tail mixed.
+constexpr double TAIL = 1e-15;
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
@@ -205,6 +213,20 @@ __global__ __launch_bounds__(256) void k_rank_diag(const T* __restrict__ A, int 
       }
     }
   }
+}
+
+// *host = number of diagonal entries above both `thr` and TAIL |rho|_F (one wave).
+template <class T>
+__global__ __launch_bounds__(64) void k_count_diag(const T* __restrict__ A, int N, int Np, double thr,
+                                                   const double* __restrict__ scal, double* host) {
+  thr = fmax(thr, TAIL * scal[0]);
+  int a = 0;
+  for (int i0 = 0; i0 < N; i0 += 64) {
+    const int i = i0 + threadIdx.x;
+    const double d = i < N ? real(A[i + (size_t)i * Np]) : -INFINITY;
+    a += __popcll(__ballot(d > thr));
+  }
+  if (threadIdx.x == 0) *host = a;
 }
 
 // Stable descending sort of n <= 2048 keys -> perm (and the sorted keys).
@@ -848,11 +870,12 @@ __global__ __launch_bounds__(256) void k_vecnorm(const T* __restrict__ Y, int ld
 // Truncation rank (scalar_traits.h:497-505 semantics, plus the optional
 // relative cutoff) and discarded weight trace - sum_{j<nk} |product vector j|^2
 // (the weight the kept orthonormal vectors carry, exact for any orthonormal
-// basis of the kept space).
+// basis of the kept space).  host[0] = discarded weight, host[1], host[2] =
+// the last kept and the first sigma.
 __global__ __launch_bounds__(256) void k_rank(const double* __restrict__ sigma,
                                               const double* __restrict__ gdiag, int k,
                                               double cutoff, double rel, const double* scal,
-                                              double* disc, int* newk) {
+                                              double* host, int* newk) {
   __shared__ int first[256];
   __shared__ double part[256];
   const int t = threadIdx.x;
@@ -878,7 +901,9 @@ __global__ __launch_bounds__(256) void k_rank(const double* __restrict__ sigma,
     __syncthreads();
   }
   if (t == 0) {
-    *disc = fmax(scal[2] - part[0], 0.0);
+    host[0] = fmax(scal[2] - part[0], 0.0);
+    host[1] = sigma[nk - 1];
+    host[2] = sigma[0];
     *newk = nk;
   }
 }
@@ -1401,14 +1426,17 @@ void qr_factor(hipStream_t st, T* A, T* Q, T* work, T* Tm, int Np) {
 // within a factor 1e4 of max(cut_abs^2, cut_rel^2 * largest) -- the cutoff
 // may then drop kept vectors, which needs them resolved -- the iteration goes
 // on to full convergence.
+// rank > 0: the number of vectors that the caller keeps unless the cutoff drops
+// some.
 struct JacobiCount {
   int sweeps = 0, bip = 0, oa = 0;
+  bool qr = false;  // QR steps were taken
 };
 
 template <class T>
 int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, JacobiCount& cnt,
            double& off_rel, bool v_given = false, int keep = 0, double cut_abs = 0.0,
-           double cut_rel = 0.0) {
+           double cut_rel = 0.0, int rank = 0) {
   int& sweeps = cnt.sweeps;
   const int nb = Np / JB;
   const int np = nb / 2;
@@ -1435,6 +1463,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     DMRG_LAUNCH_CHECK();
   };
   if (v_given) measure(w.A[0]);  // read behind the one synchronisation
+  double* const above = w.host + NRED + 3;
+  const bool check = prm.qr && rank > 0 && !v_given && Np >= QR_MIN;
+  if (check)
+    hipLaunchKernelGGL(k_count_diag<T>, dim3(1), dim3(64), 0, st, (const T*)w.A[0], N, Np,
+                       1e4 * cut_abs * cut_abs, (const double*)w.scal, above);
   DMRG_LAUNCH_CHECK();
   DMRG_HIP(hipStreamSynchronize(st));
   double fro = w.host[NRED + 2];
@@ -1456,11 +1489,19 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   }
   const double cut2 = std::ldexp(cut_abs * cut_abs, e2);  // the cutoff in units of the scaled rho
   const double rot_tol = 0.125 * prm.tol;
+  // Where the spectrum falls through the resolution of rho (tol |rho|_F) and on
+  // towards the cutoff, a cold split is the sweeps' alone.  They leave the
+  // directions below that resolution mixed with the rest, so none falls under
+  // the cutoff; the QR steps keep the small entries of a graded rho and take
+  // them apart, and bonds that are not truncated would shrink (256 -> 247 at the
+  // bond of 8 sites of a chain of 32 at chi = 256), at once or in a later sweep.
+  // The diagonal of rho tells: what is not graded is mixed by rounding anyway.
+  const bool qr = prm.qr && !(check && *above < rank);
   // One inner sweep per block pair: a second one before the pairs meet other
   // blocks saves one outer sweep in fourteen and costs as much again (256^2,
   // Schmidt values falling to 1e-6: 14 sweeps of 31 inner rounds against 13 of
   // 62).  A matrix of a single pair is diagonalised in place.
-  const int inner_max = (nb == 2) ? 64 : 1;
+  const int inner_max = (nb == 2) ? 64 : qr ? 1 : 2;
   const int noff = np * (np - 1) / 2, nvt = (Np / JP) * np;
   int cur = 0;
   sweeps = 0;
@@ -1507,6 +1548,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // chi = 128: 1 instead of 5).  A step costs about as much as one sweep of the
   // round robin at every size.
   auto qr_steps = [&] {
+    cnt.qr = true;
     for (int it = 0; it < 2; ++it) {
       hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np,
                          N, w.perm, nullptr);
@@ -1530,7 +1572,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     off_rel = last_off / fro;
     done = last_off <= prm.tol * fro;
   };
-  const bool qr_ok = Np >= QR_MIN && Np <= qr_max<T>();
+  const bool qr_ok = qr && Np >= QR_MIN && Np <= qr_max<T>();
   // Far from the eigenbasis: no basis given, or one whose measure is above the
   // gate, as in the second sweep of a run, or sweeps that stall (9 sweeps of a
   // 512^2 block before).  A given basis goes through the QR steps only where
@@ -1645,7 +1687,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       ++cnt.oa;
     }
   };
-  int fo_left = far ? 2 : 1;  // stages of first-order steps left to try
+  int fo_left = far ? (qr ? 2 : 0) : 1;  // stages of first-order steps left to try
   bool bip_ok = true;  // bipartite sweeps allowed (revoked once one stalls)
   int n_bip = 0;
   bool qr_left = qr_ok;
@@ -1690,7 +1732,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (ka > 0) ++cnt.bip;
     if (ka > 0 && (++n_bip >= 4 || off > 0.1 * off_before)) bip_ok = false;
     sweeps = sw + 1;
-    if (far) near = Np >= FO_MIN && off <= gate * fro;
+    if (far) near = qr && Np >= FO_MIN && off <= gate * fro;
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
     // a graded block again: sweeps that stall this far out take five to nine
@@ -1808,7 +1850,7 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
   const int keep = (prm.subspace && k < N) ? k : 0;
   JacobiCount jc;
   const int cur = jacobi<T>(st, w, N, Np, prm, jc, res.off, warm != nullptr, keep, cutoff,
-                            rel_cutoff);
+                            rel_cutoff, k);
   res.sweeps = jc.sweeps;
   res.bip_sweeps = jc.bip;
   res.oa_steps = jc.oa;
@@ -1873,18 +1915,28 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
   DMRG_LAUNCH_CHECK();
   DMRG_HIP(hipStreamSynchronize(st));
   const int nk = w.host_i[0];
-  const double disc = w.host[0];
+  const double disc = w.host[0], last = w.host[1], first = w.host[2];
+  auto again = [&](const SvdParams& p2) {
+    SvdResult r2 = svd_split<T>(st, w, A, m, n, lda, kmax, cutoff, rel_cutoff, scale_left, left,
+                                ldl, right, sigma_out, p2, warm, basis_out);
+    r2.sweeps += res.sweeps;
+    r2.bip_sweeps += res.bip_sweeps;
+    r2.oa_steps += res.oa_steps;
+    return r2;
+  };
+  if (jc.qr && nk < k && last * last < 100.0 * prm.tol * first * first) {
+    // the rank ends among Schmidt values below the resolution of rho, not in a
+    // gap: the number of them is the sweeps' (see jacobi)
+    SvdParams sweeps_only = prm;
+    sweeps_only.qr = false;
+    return again(sweeps_only);
+  }
   if (keep > 0 && nk < k) {
     // the cutoff cuts inside the kept group, whose vectors are not resolved:
     // redo the split with every pair converged
     SvdParams full = prm;
     full.subspace = false;
-    SvdResult r2 = svd_split<T>(st, w, A, m, n, lda, kmax, cutoff, rel_cutoff, scale_left, left,
-                                ldl, right, sigma_out, full, warm, basis_out);
-    r2.sweeps += res.sweeps;
-    r2.bip_sweeps += res.bip_sweeps;
-    r2.oa_steps += res.oa_steps;
-    return r2;
+    return again(full);
   }
   res.nk = nk;
   res.discarded = disc;

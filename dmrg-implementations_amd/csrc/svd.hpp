@@ -47,10 +47,10 @@ struct SvdWork {
   int* perm = nullptr;           // sort permutation
   int* rank = nullptr;           // inverse of perm (position of each index)
   double* gdiag = nullptr;       // squared norms of the k product vectors
-  double* red = nullptr;         // reduction partials / small results (1024 doubles)
+  double* red = nullptr;         // partials of |rho|_F^2 and of the trace
   double* sigma = nullptr;       // singular values in output order
   double* resid = nullptr;       // first-pass QR residuals
-  double* scal = nullptr;        // [0] |rho|_F, [1] discarded weight, [2] trace(rho)
+  double* scal = nullptr;        // [0] |rho|_F, [2] trace(rho)
   double* host = nullptr;  // pinned host staging of every read-back (2 cap + 2*256 + 16 doubles)
   int* host_i = nullptr;   // pinned host staging of the kept rank
   int cap = 0;  // largest supported rho dimension (multiple of 32)
@@ -69,6 +69,7 @@ struct SvdParams {
   // product vectors after projecting out the earlier ones.  Falls back to
   // full convergence when the cutoff keeps fewer than k vectors.
   bool subspace = false;
+  bool qr = true;  // QR steps ahead of the sweeps where they serve
 };
 
 struct SvdResult {
