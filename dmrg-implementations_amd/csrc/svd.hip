@@ -1464,7 +1464,10 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   };
   if (v_given) measure(w.A[0]);  // read behind the one synchronisation
   double* const above = w.host + NRED + 3;
-  const bool check = prm.qr && rank > 0 && !v_given && Np >= QR_MIN;
+  const bool cold = prm.qr && !v_given && Np >= QR_MIN, check = cold && rank > 0;
+  if (cold)  // all pairs: the diagonal need not be the spectrum yet
+    hipLaunchKernelGGL(k_offmax<T>, dim3(NRED), dim3(256), 0, st, (const T*)w.A[0], N, Np,
+                       (const int*)nullptr, 0, hp);
   if (check)
     hipLaunchKernelGGL(k_count_diag<T>, dim3(1), dim3(64), 0, st, (const T*)w.A[0], N, Np,
                        1e4 * cut_abs * cut_abs, (const double*)w.scal, above);
@@ -1476,9 +1479,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // to rounding size: those of a norm far from one would leave the range of a
   // double (|rho|_F = 1e-140: the reflections dropped columns that count).  The
   // iteration then works on 2^e rho, which is exact.
+  double off0 = cold ? *std::max_element(hp, hp + NRED) / fro : INFINITY;
   int e2 = 0;
   if (fro != 0.0 && (fro < 0x1p-300 || fro > 0x1p+300)) {
     e2 = -std::ilogb(fro);
+    off0 = INFINITY;  // measured out of range
     hipLaunchKernelGGL(k_scale_pow2<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[0], tot, e2,
                        (double*)nullptr);
     norms();
@@ -1496,7 +1501,9 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // them apart, and bonds that are not truncated would shrink (256 -> 247 at the
   // bond of 8 sites of a chain of 32 at chi = 256), at once or in a later sweep.
   // The diagonal of rho tells: what is not graded is mixed by rounding anyway.
-  const bool qr = prm.qr && !(check && *above < rank);
+  // And one next to diagonal needs a sweep or two (a matrix of equal Schmidt
+  // values, 512^2: 0.5 ms; 2.4 ms with QR steps).
+  const bool qr = prm.qr && !(check && *above < rank) && off0 > QR_GATE;
   // One inner sweep per block pair: a second one before the pairs meet other
   // blocks saves one outer sweep in fourteen and costs as much again (256^2,
   // Schmidt values falling to 1e-6: 14 sweeps of 31 inner rounds against 13 of
@@ -1537,7 +1544,8 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     keep = 0;
     return offmax(M);
   };
-  bool done = false;
+  bool done = off0 <= rot_tol;  // a sweep would rotate nothing
+  if (done) off_rel = off0;
   double last_off = INFINITY;  // latest convergence measure (criterion in force)
   const double gate = keep > 0 ? 1e-4 : 1e-6;  // measure below which first-order steps are tried
   if (v_given) last_off = read_measure();
