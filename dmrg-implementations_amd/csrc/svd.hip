@@ -1503,12 +1503,18 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // The diagonal of rho tells: what is not graded is mixed by rounding anyway.
   // And one next to diagonal needs a sweep or two (a matrix of equal Schmidt
   // values, 512^2: 0.5 ms; 2.4 ms with QR steps).
-  const bool qr = prm.qr && !(check && *above < rank) && off0 > QR_GATE;
+  // Nor does the eigen-solver (rank 0) take them: a general Hermitian matrix is
+  // not graded (40^2 to 512^2: sweeps alone 0.73 to 0.99 of the time).
+  const bool qr = prm.qr && rank > 0 && !(check && *above < rank) && off0 > QR_GATE;
+  // It shares the other two measures of a cold split, one inner sweep per block
+  // pair and first-order steps between the sweeps, where those pay (from
+  // FO_MIN: 512^2 0.70 to 0.90 of the time; 40^2, 64^2 of low rank: 1.2).
+  const bool lean = qr || (cold && rank == 0 && Np >= FO_MIN && off0 > QR_GATE);
   // One inner sweep per block pair: a second one before the pairs meet other
   // blocks saves one outer sweep in fourteen and costs as much again (256^2,
   // Schmidt values falling to 1e-6: 14 sweeps of 31 inner rounds against 13 of
   // 62).  A matrix of a single pair is diagonalised in place.
-  const int inner_max = (nb == 2) ? 64 : qr ? 1 : 2;
+  const int inner_max = (nb == 2) ? 64 : lean ? 1 : 2;
   const int noff = np * (np - 1) / 2, nvt = (Np / JP) * np;
   int cur = 0;
   sweeps = 0;
@@ -1554,10 +1560,14 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // truncation to within a few sweeps of diagonal (512^2, Schmidt values
   // falling to 1e-6: 5 sweeps instead of 16; a bond of a first DMRG sweep at
   // chi = 128: 1 instead of 5).  A step costs about as much as one sweep of the
-  // round robin at every size.
+  // round robin at every size.  Of blocks up to 64 it is two, and the first step
+  // does most of it (64^2, Schmidt values falling to 1e-6 and those of a random
+  // tensor: 1460 and 1050 us by sweeps alone, 840 and 1130 with two steps, 840 and
+  // 1050 with one).
+  const int steps = v_given || Np > 64 ? 2 : 1;
   auto qr_steps = [&] {
     cnt.qr = true;
-    for (int it = 0; it < 2; ++it) {
+    for (int it = 0; it < steps; ++it) {
       hipLaunchKernelGGL(k_sort<T>, dim3(cdiv(Np, 16)), dim3(256), 0, st, w.A[cur], Np, nullptr, Np,
                          N, w.perm, nullptr);
       hipLaunchKernelGGL(k_permute<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[cur], w.V[cur],
@@ -1695,7 +1705,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
       ++cnt.oa;
     }
   };
-  int fo_left = far ? (qr ? 2 : 0) : 1;  // stages of first-order steps left to try
+  int fo_left = far ? (lean ? 2 : 0) : 1;  // stages of first-order steps left to try
   bool bip_ok = true;  // bipartite sweeps allowed (revoked once one stalls)
   int n_bip = 0;
   bool qr_left = qr_ok;
@@ -1740,7 +1750,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     if (ka > 0) ++cnt.bip;
     if (ka > 0 && (++n_bip >= 4 || off > 0.1 * off_before)) bip_ok = false;
     sweeps = sw + 1;
-    if (far) near = qr && Np >= FO_MIN && off <= gate * fro;
+    if (far) near = lean && Np >= FO_MIN && off <= gate * fro;
     off_rel = off / fro;
     if (off <= prm.tol * fro) { done = true; break; }
     // a graded block again: sweeps that stall this far out take five to nine
