@@ -43,6 +43,12 @@ __device__ inline double sum_parts(const double* __restrict__ part, int nb) {
   return wave_sum_all(s);
 }
 
+// A sum that the consuming kernel forms with sum_parts: n partials at p.
+struct Parts {
+  const double* p;
+  int n;
+};
+
 // Sum of v over the workgroup, in every thread (sh: NW values, free on return).
 __device__ inline double block_sum(double v, double* sh) {
   v = wave_sum_all(v);
@@ -184,10 +190,10 @@ __global__ __launch_bounds__(NT) void k_fill_random(T* x, size_t n, uint64_t see
 // result.
 template <class T, int E>
 __global__ __launch_bounds__(NL) void k_fill_small(T* x, size_t n, uint64_t seed, double thr,
-                                                  const double* __restrict__ partN,
+                                                  const double* __restrict__ partN, Parts sumN,
                                                   double* __restrict__ partO) {
   __shared__ double sh[NW];
-  if (!(sqrt(sum_parts(partN, gridDim.x)) < thr)) {
+  if (!(sqrt(sum_parts(sumN.p, sumN.n)) < thr)) {
     if (threadIdx.x == 0) partO[blockIdx.x] = partN[blockIdx.x];
     return;
   }
@@ -215,12 +221,12 @@ __device__ inline double inv_norm(double nrm) { return (nrm > 1e-300) ? 1.0 / nr
 // nrm = sqrt(sum partN); dst = src / nrm (if dst given; zero if nrm <= 1e-300).
 template <class T, int E>
 __global__ __launch_bounds__(NL) void k_scale(T* dst, const T* src, size_t n,
-                                             const double* __restrict__ partN, int nbp,
-                                             double* scal, double* beta_out, double* host) {
+                                             Parts sumN, double* scal, double* beta_out,
+                                             double* host) {
   const Chunk<E> c(n);
   T v[E];
   c.load(src, v);
-  const double nrm = sqrt(sum_parts(partN, nbp));
+  const double nrm = sqrt(sum_parts(sumN.p, sumN.n));
   const double s = inv_norm(nrm);
   if (blockIdx.x == 0 && threadIdx.x == 0) put_norm(nrm, s, scal, beta_out, host);
   if (!dst) return;
@@ -245,13 +251,6 @@ __global__ __launch_bounds__(NL) void k_alpha(const T* __restrict__ v, const T* 
   if (threadIdx.x == 0) partA[blockIdx.x] = s;
 }
 
-// out[it] = sum partA (one wave).
-__global__ __launch_bounds__(64) void k_alpha_value(const double* __restrict__ partA, int nbp,
-                                                    double* alpha, int it) {
-  const double a = sum_parts(partA, nbp);
-  if (threadIdx.x == 0) alpha[it] = a;
-}
-
 // alpha[it] = sum partA;  w -= alpha v_it + beta[it-1] v_{it-1};
 // partC[(j*NC + c)*nb + blk] = component c of <v_j, w> over the chunk, j <= it.
 // One pass over the basis, bound by the L2 and the Infinity Cache; every load
@@ -260,8 +259,8 @@ __global__ __launch_bounds__(64) void k_alpha_value(const double* __restrict__ p
 // through LDS per group of eight vectors before).
 template <class T, int E>
 __global__ __launch_bounds__(NL) void k_sub_dots(T* __restrict__ w, const T* __restrict__ V,
-                                                size_t n, int it, const double* __restrict__ partA,
-                                                double* alpha, const double* beta,
+                                                size_t n, int it, Parts sumA, double* alpha,
+                                                const double* beta,
                                                 double* __restrict__ partC) {
   constexpr int NC = Acc<T>::N, G = group<T, E>();
   __shared__ double sh[128 * NC * NW];
@@ -272,7 +271,7 @@ __global__ __launch_bounds__(NL) void k_sub_dots(T* __restrict__ w, const T* __r
   c.load(V + (size_t)it * n, vi);
   c.load(V + (size_t)max(it - 1, 0) * n, vm);
   load_group<T, E, G>(c, V, n, 0, cnt, v);
-  const double a = sum_parts(partA, nb);
+  const double a = sum_parts(sumA.p, sumA.n);
   const double bm = it > 0 ? beta[it - 1] : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) alpha[it] = a;
 #pragma unroll
@@ -291,11 +290,21 @@ __global__ __launch_bounds__(NL) void k_sub_dots(T* __restrict__ w, const T* __r
   }
 }
 
-// cvec[g] = sum_b partC[g*nb + b] (doubles; one wave per g, fixed order).
-__global__ __launch_bounds__(64) void k_coeffs(const double* __restrict__ partC, int nb,
-                                               double* __restrict__ cvec) {
-  const double s = sum_parts(partC + (size_t)blockIdx.x * nb, nb);
-  if (threadIdx.x == 0) cvec[blockIdx.x] = s;
+// out[g] = sum_b part[g*nb + b] (one workgroup of NTH threads per g, fixed order).
+template <int NTH>
+__global__ __launch_bounds__(NTH) void k_totals(const double* __restrict__ part, int nb,
+                                                double* __restrict__ out) {
+  const double* const p = part + (size_t)blockIdx.x * nb;
+  double s;
+  if constexpr (NTH == 64) {
+    s = sum_parts(p, nb);
+  } else {
+    __shared__ double sh[NW];
+    s = 0.0;
+    for (int b = threadIdx.x; b < nb; b += NTH) s += p[b];
+    s = block_sum(s, sh);
+  }
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // w -= sum_j c_j v_j (c from cvec, or re-reduced from partC when cvec is null);
@@ -695,6 +704,12 @@ __global__ __launch_bounds__(64) void k_tri(const double* alpha, const double* b
 
 namespace {
 constexpr size_t LZ_ONE = 2 * NL;
+// Every wave of a consuming kernel reads all partials of a sum, n / 4096 of them
+// past 2^19 elements: work that grows with n^2.  Past LZ_PARTS a launch reduces
+// them first (12 iterations, n = 2^21, 2^22, 2^23, 2^24, and 4 at 2^26: 2.79, 5.48,
+// 14.6, 36.8 and 112 ms without, 2.78, 5.21, 13.6, 32.2 and 82 with 512; 256 and
+// 1024 within 1 % of that but for 5.40 at 2^22 with 1024).
+constexpr int LZ_PARTS = 512;
 // Elements a thread holds: 1 to 2^18, 2 to 2^19, then 4.
 int lz_elems(size_t n) { return n <= (size_t)256 * NL ? 1 : n <= (size_t)512 * NL ? 2 : 4; }
 bool lz_one(size_t n) { return n <= LZ_ONE; }
@@ -739,6 +754,21 @@ inline void need_parts(const LzDev& d, size_t n, int cnt) {
   const size_t need = (size_t)(cnt + 2) * lz_blocks(n) * sizeof(double);
   DMRG_REQUIRE(need <= d.part_bytes, "lanczos: partial buffer too small");
 }
+
+void totals(hipStream_t st, const double* part, int nb, int count, double* out) {
+  if (nb <= LZ_PARTS)
+    hipLaunchKernelGGL(k_totals<64>, dim3(count), dim3(64), 0, st, part, nb, out);
+  else
+    hipLaunchKernelGGL(k_totals<NL>, dim3(count), dim3(NL), 0, st, part, nb, out);
+  DMRG_LAUNCH_CHECK();
+}
+// The sum of nb partials as every wave of the next kernel reads it: the partials
+// themselves up to LZ_PARTS, past that one value (kept in `slot`).
+Parts sum_of(hipStream_t st, const double* part, int nb, double* slot) {
+  if (nb <= LZ_PARTS) return {part, nb};
+  totals(st, part, nb, 1, slot);
+  return {slot, 1};
+}
 }  // namespace
 
 // Launch KERNEL<T, E> with the E of length n.
@@ -770,9 +800,10 @@ void lz_start(hipStream_t st, LzDev& d, T* theta, T* v0, size_t n, uint64_t seed
   const int nb = lz_blocks(n);
   need_parts(d, n, 0);
   DMRG_LZ(k_norm, theta, n, partN(d, nb), d.scal);
-  DMRG_LZ(k_fill_small, theta, n, seed, thr, (const double*)partN(d, nb), partA(d));
-  DMRG_LZ(k_scale, v0, (const T*)theta, n, (const double*)partA(d), nb, d.scal, (double*)nullptr,
-          (double*)nullptr);
+  const Parts first = sum_of(st, partN(d, nb), nb, d.scal + 5);
+  DMRG_LZ(k_fill_small, theta, n, seed, thr, (const double*)partN(d, nb), first, partA(d));
+  const Parts nrm = sum_of(st, partA(d), nb, d.scal + 5);
+  DMRG_LZ(k_scale, v0, (const T*)theta, n, nrm, d.scal, (double*)nullptr, (double*)nullptr);
 }
 
 template <class T>
@@ -795,29 +826,26 @@ void lz_step(hipStream_t st, LzDev& d, T* w, T* V, size_t n, int it, bool next) 
   need_parts(d, n, cnt);
   const int nb = lz_blocks(n);
   DMRG_LZ(k_alpha, (const T*)V + (size_t)it * n, (const T*)w, n, partA(d));
-  DMRG_LZ(k_sub_dots, w, (const T*)V, n, it, (const double*)partA(d), d.alpha,
-          (const double*)d.beta, partC(d, nb));
+  const Parts al = sum_of(st, partA(d), nb, d.scal + 5);
+  DMRG_LZ(k_sub_dots, w, (const T*)V, n, it, al, d.alpha, (const double*)d.beta, partC(d, nb));
   // every workgroup re-reduces the coefficients up to 256 partials each (n =
   // 2^18, 20 iterations: 6.3 us a time against 5.6 and 4.2 for a kernel of
   // its own); past that a wave per coefficient reduces them first
   const double* cv = nullptr;
   if (nb > 256) {
-    hipLaunchKernelGGL(k_coeffs, dim3(cnt), dim3(64), 0, st, (const double*)partC(d, nb), nb,
-                       (double*)d.cvec);
+    totals(st, partC(d, nb), nb, cnt, (double*)d.cvec);
     cv = (const double*)d.cvec;
   }
   DMRG_LZ(k_orth_norm, w, (const T*)V, n, it, (const double*)partC(d, nb), cv, partN(d, nb));
-  DMRG_LZ(k_scale, vnext, (const T*)w, n, (const double*)partN(d, nb), nb, d.scal, d.beta + it,
-          (double*)nullptr);
+  const Parts nrm = sum_of(st, partN(d, nb), nb, d.scal + 5);
+  DMRG_LZ(k_scale, vnext, (const T*)w, n, nrm, d.scal, d.beta + it, (double*)nullptr);
 }
 
 template <class T>
 void lz_dot(hipStream_t st, LzDev& d, const T* v, const T* w, size_t n) {
   need_parts(d, n, 0);
   DMRG_LZ(k_alpha, v, w, n, partA(d));
-  hipLaunchKernelGGL(k_alpha_value, dim3(1), dim3(64), 0, st, (const double*)partA(d),
-                     lz_blocks(n), d.alpha, 0);
-  DMRG_LAUNCH_CHECK();
+  totals(st, partA(d), lz_blocks(n), 1, d.alpha);
 }
 
 void lz_check(hipStream_t st, LzDev& d, int ncheck, double beta_tol, double eig_tol,
@@ -844,8 +872,8 @@ void lz_ritz(hipStream_t st, LzDev& d, T* out, const T* V, size_t n, int niter, 
   }
   const int nb = lz_blocks(n);
   DMRG_LZ(k_ritz, out, V, n, niter, (const double*)d.y, partN(d, nb));
-  DMRG_LZ(k_scale, out, (const T*)out, n, (const double*)partN(d, nb), nb, d.scal,
-          (double*)nullptr, host);
+  const Parts nrm = sum_of(st, partN(d, nb), nb, d.scal + 5);
+  DMRG_LZ(k_scale, out, (const T*)out, n, nrm, d.scal, (double*)nullptr, host);
 }
 #undef DMRG_LZ
 #undef DMRG_LZ_ONE

@@ -17,7 +17,7 @@ struct LzDev {
   double* alpha = nullptr;     // [kmax]
   double* beta = nullptr;      // [kmax]
   double* y = nullptr;         // [kmax] Ritz coefficients
-  double* scal = nullptr;      // [8]: 0 norm, 1 inv, 2 prev_energy, 3 energy, 4 check value
+  double* scal = nullptr;      // [8]: 0 norm, 1 inv, 2 prev_energy, 3 energy, 4 check value, 5 sum of partials
   void* part = nullptr;        // partial sums (bytes), lz_part_doubles(kmax, n) doubles
   void* cvec = nullptr;        // [kmax] projection coefficients (T)
   int kmax = 0;
