@@ -61,30 +61,36 @@ __device__ inline double block_sum(double v, double* sh) {
   return r;
 }
 
-// The thread's elements of x (zero, and an index inside the vector, past n).
+// The thread's elements of x (zero, and an index inside the vector, past n):
+// base + off[e], the base uniform over the workgroup.
 template <int E>
 struct Chunk {
-  unsigned idx[E];  // every vector has fewer than 2^32 elements
+  size_t base;
+  unsigned off[E];
   bool in[E];
-  __device__ explicit Chunk(size_t n) {
+  __device__ explicit Chunk(size_t n) : base((size_t)blockIdx.x * (E * NL)) {
+    const size_t left = n - base;  // at least one element for every workgroup
+    const unsigned cnt = left < E * NL ? (unsigned)left : E * NL;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const unsigned i = (blockIdx.x * E + e) * NL + threadIdx.x;
-      in[e] = i < (unsigned)n;
-      idx[e] = in[e] ? i : (unsigned)n - 1;
+      const unsigned i = e * NL + threadIdx.x;
+      in[e] = i < cnt;
+      off[e] = in[e] ? i : cnt - 1;
     }
   }
   template <class T> __device__ void load(const T* __restrict__ x, T (&v)[E]) const {
+    x += base;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const T u = x[idx[e]];
+      const T u = x[off[e]];
       v[e] = in[e] ? u : T(0);
     }
   }
   template <class T> __device__ void store(T* __restrict__ x, const T (&v)[E]) const {
+    x += base;
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      if (in[e]) x[idx[e]] = v[e];
+      if (in[e]) x[off[e]] = v[e];
   }
 };
 template <class T, int E> __device__ inline double sum_abs2(const T (&v)[E]) {
@@ -200,7 +206,7 @@ __global__ __launch_bounds__(NL) void k_fill_small(T* x, size_t n, uint64_t seed
   const Chunk<E> c(n);
   T v[E];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = c.in[e] ? rand_entry<T>(seed, c.idx[e], 1.0) : T(0);
+  for (int e = 0; e < E; ++e) v[e] = c.in[e] ? rand_entry<T>(seed, c.base + c.off[e], 1.0) : T(0);
   c.store(x, v);
   const double s = block_sum(sum_abs2<T, E>(v), sh);
   if (threadIdx.x == 0) partO[blockIdx.x] = s;
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(NL) void k_one_start(T* theta, T* v0, size_t n, uin
   double nrm = sqrt(block_sum(sum_abs2<T, E>(x), sh));
   if (nrm < thr) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = c.in[e] ? rand_entry<T>(seed, c.idx[e], 1.0) : T(0);
+    for (int e = 0; e < E; ++e) x[e] = c.in[e] ? rand_entry<T>(seed, c.base + c.off[e], 1.0) : T(0);
     c.store(theta, x);
     nrm = sqrt(block_sum(sum_abs2<T, E>(x), sh));
   }
