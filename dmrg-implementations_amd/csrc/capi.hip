@@ -449,7 +449,12 @@ struct dmrg_ctx {
   CtxF32 f;  // the FP32 matvec of the mixed modes
   int* h_status = nullptr;
   double* h_scal = nullptr;
+  // the last call that used the context's buffers: on the default stream, on a
+  // created one (then `used` was recorded behind it), or none
+  enum { NONE, DEFAULT, CREATED } last = NONE;
+  hipEvent_t used = nullptr;
   ~dmrg_ctx() {
+    if (used) (void)hipEventDestroy(used);
     if (h_status) (void)hipHostFree(h_status);
     if (h_scal) (void)hipHostFree(h_scal);
   }
@@ -470,6 +475,38 @@ void by_dtype(int dtype, F&& f) {
 // Every op runs on its context's device, whichever thread calls it.
 void use(const dmrg_ctx* c) { DMRG_HIP(hipSetDevice(c->device)); }
 
+// A call that uses the context's buffers, on the context's device: ordered on
+// `st` behind the previous one, whichever stream that was given.  Calls on the
+// default stream alone record and wait for nothing; one on a created stream
+// records an event (the stream may be gone when the next call comes).  Under
+// capture the order of graphs is the caller's.
+class CtxCall {
+ public:
+  CtxCall(dmrg_ctx* c, void* stream) : c_(c), st_((hipStream_t)stream) {
+    use(c);
+    if (st_) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      DMRG_HIP(hipStreamIsCapturing(st_, &cs));
+      captured_ = cs != hipStreamCaptureStatusNone;
+    }
+    if (captured_) return;
+    if (c->last == dmrg_ctx::DEFAULT && st_) DMRG_HIP(hipEventRecord(c->used, nullptr));
+    if (c->last == dmrg_ctx::CREATED || (c->last == dmrg_ctx::DEFAULT && st_))
+      DMRG_HIP(hipStreamWaitEvent(st_, c->used, 0));
+  }
+  ~CtxCall() {
+    if (captured_) return;
+    c_->last = st_ ? dmrg_ctx::CREATED : dmrg_ctx::DEFAULT;
+    if (st_ && hipEventRecord(c_->used, st_) != hipSuccess) (void)hipDeviceSynchronize();
+  }
+  CtxCall(const CtxCall&) = delete;
+
+ private:
+  dmrg_ctx* c_;
+  hipStream_t st_;
+  bool captured_ = false;
+};
+
 }  // namespace
 
 extern "C" {
@@ -483,6 +520,7 @@ int dmrg_ctx_create(int device, dmrg_ctx_handle* out) {
     c->device = device;
     DMRG_HIP(hipHostMalloc((void**)&c->h_status, 4 * sizeof(int), hipHostMallocDefault));
     DMRG_HIP(hipHostMalloc((void**)&c->h_scal, 8 * sizeof(double), hipHostMallocDefault));
+    DMRG_HIP(hipEventCreateWithFlags(&c->used, hipEventDisableTiming));
     *out = c.release();
   });
 }
@@ -497,7 +535,7 @@ int dmrg_op_heff2(dmrg_ctx_handle c, void* stream, int dtype, int cL, int cR, in
                   void* out) {
   if (!c || !L || !R || !W1 || !W2 || !theta || !out) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(cL >= 1 && cR >= 1 && d >= 1 && D >= 1, "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -521,7 +559,7 @@ int dmrg_op_heff2_f32(dmrg_ctx_handle c, void* stream, int prec, int cL, int cR,
                       const float* theta, float* out) {
   if (!c || !L || !R || !W1 || !W2 || !theta || !out) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(cL >= 1 && cR >= 1 && d >= 1 && D >= 1, "bad shape");
     DMRG_REQUIRE(prec == DMRG_PREC_FP32 || prec == DMRG_PREC_BF16X3, "prec must be FP32 or BF16X3");
     hipStream_t st = (hipStream_t)stream;
@@ -539,7 +577,7 @@ int dmrg_op_heff1(dmrg_ctx_handle c, void* stream, int dtype, int cL, int cR, in
                   const void* L, const void* R, const void* W, const void* theta, void* out) {
   if (!c || !L || !R || !W || !theta || !out) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(cL >= 1 && cR >= 1 && d >= 1 && D >= 1, "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -555,7 +593,7 @@ int dmrg_op_env_left(dmrg_ctx_handle c, void* stream, int dtype, int ci, int co,
                      const void* L, const void* A, const void* W, void* Lnew) {
   if (!c || !L || !A || !W || !Lnew) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(ci >= 1 && co >= 1 && d >= 1 && D >= 1, "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -578,7 +616,7 @@ int dmrg_op_env_right(dmrg_ctx_handle c, void* stream, int dtype, int ci, int co
                       const void* R, const void* A, const void* W, void* Rnew) {
   if (!c || !R || !A || !W || !Rnew) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(ci >= 1 && co >= 1 && d >= 1 && D >= 1, "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -597,7 +635,7 @@ int dmrg_op_svd_split(dmrg_ctx_handle c, void* stream, int dtype, int m, int n, 
                       void* right, double* sigma, int* nk_out) {
   if (!c || !M || !left || !right || !nk_out) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(m >= 1 && n >= 1 && k >= 1 && k <= std::min(m, n), "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -619,7 +657,7 @@ int dmrg_op_rsvd_split(dmrg_ctx_handle c, void* stream, int dtype, int m, int n,
                        void* right, int* nk_out) {
   if (!c || !M || !left || !right || !nk_out) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(m >= 1 && n >= 1 && k >= 1 && k <= std::min(m, n), "bad shape");
     DMRG_REQUIRE(oversample >= 0 && power >= 0 && power <= 8, "bad oversample / power");
     by_dtype(dtype, [&](auto tag) {
@@ -642,7 +680,7 @@ int dmrg_op_heig(dmrg_ctx_handle c, void* stream, int dtype, int N, const void* 
                  void* evecs, int* sweeps_out) {
   if (!c || !H || !evals || !evecs) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(N >= 1 && N <= 2048, "bad shape");
     by_dtype(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -660,7 +698,7 @@ int dmrg_op_tridiag_lowest(dmrg_ctx_handle c, int k, const double* alpha, const 
                            double* lam, double* y) {
   if (!c || !alpha || !lam || !y || (k > 1 && !beta)) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, nullptr);
     DMRG_REQUIRE(k >= 1 && k <= 128, "k must be in [1, 128]");
     auto& x = c->r;
     x.need_lz(128, 1);
@@ -680,7 +718,7 @@ int dmrg_op_lanczos2(dmrg_ctx_handle c, void* stream, int dtype, int cL, int cR,
                      int krylov_max, int site, double* energy, int* niter) {
   if (!c || !L || !R || !W1 || !W2 || !theta || !energy) return fail(DMRG_ERR_BAD_ARG, "NULL argument");
   return guard([&] {
-    use(c);
+    const CtxCall call(c, stream);
     DMRG_REQUIRE(cL >= 1 && cR >= 1 && d >= 1 && D >= 1, "bad shape");
     DMRG_REQUIRE(krylov_max >= 1 && krylov_max <= 128, "krylov_max must be in [1, 128]");
     by_dtype(dtype, [&](auto tag) {

@@ -249,6 +249,18 @@ const char* dmrg_last_error(void);
  * roofline bench).  Each replaces one library-call sequence of the reference
  * and runs on the given HIP stream (0 = default stream); `ctx` owns scratch
  * and names the device, which each call makes current on its thread.
+ *
+ * Stream order: a call returns once its work is on the stream, unless it gives
+ * the host a value (a kept rank, an energy).  Every operand, the MPO tensors
+ * among them, is read on that stream and stays valid and unchanged until the
+ * stream has run the call; writes from other streams are ordered by events, as
+ * with any kernel.  A context's scratch serves one call at a time: each call
+ * waits on the device for the context's previous one, whichever stream that ran
+ * on, so one context may be used on several streams, from one host thread at a
+ * time.  Work that is to overlap takes a context per stream.  Under stream
+ * capture a call neither waits nor is waited for: the order of a graph's launches
+ * with other calls on its context is the caller's, and the scratch has to be
+ * large enough beforehand (one call of that size outside the capture).
  * ---------------------------------------------------------------------- */
 typedef struct dmrg_ctx* dmrg_ctx_handle;
 /* Create / destroy an op-level context.  No reference counterpart: the
