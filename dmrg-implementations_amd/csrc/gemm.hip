@@ -602,6 +602,14 @@ void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K
   const bool ta = op_trans(opA), tb = op_trans(opB);
   bool ca = op_conj(opA), cb = op_conj(opB);
   if (!is_cplx<T>::value) ca = cb = false;
+  constexpr int MAX_COLS = 65535 * 32;  // grid.y of the narrowest tile
+  if (N > MAX_COLS && !herm) {
+    for (int n0 = 0; n0 < N; n0 += MAX_COLS)
+      dispatch<T>(st, opA, opB, tl, M, std::min(MAX_COLS, N - n0), K, Kc, slices, alpha, A, lda,
+                  B + (tb ? (long long)n0 : (long long)n0 * ldb), ldb, beta,
+                  C + (long long)n0 * ldc, ldc, sC, 0);
+    return;
+  }
 #define DMRG_P4(TA_, TB_, CA_, CB_) \
   launch<T, CA_, CB_, TA_, !TB_>(st, tl, M, N, K, Kc, slices, alpha, A, lda, B, ldb, beta, C, ldc, sC, herm)
   if (!ca && !cb) {
@@ -632,15 +640,16 @@ void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K
 }
 
 // ---------------------------------------------------------------------------
-// Tile autotuner.  When enabled (gemm_autotune), the first non-batched call
-// of each (scalar type, ops, M, N, K, Hermitian) shape times the 32x32, 64x32
-// (not for a Hermitian product) and 64x64 tiles on the caller's stream, with the device otherwise idle (one warm-up each, then
-// four interleaved rounds of one launch each into a scratch output, keeping
-// each tile's fastest), and keeps the fastest for the rest of the process --
-// the caller's tile unless the other is at least 3 % faster; later calls of
-// that shape use it.  Both tiles sum over k in the same order, so tuning
-// never changes a result: runs are bit-reproducible across processes.  A call made while its stream is being captured
-// into a graph uses the caller's tile and records nothing.
+// Tile autotuner.  When enabled (gemm_autotune), the first call of each (scalar
+// type, ops, M, N, K, Hermitian) shape times the 32x32, 64x32 (not for a
+// Hermitian product) and 64x64 tiles on the caller's stream, with the device
+// otherwise idle (one warm-up each, then four interleaved rounds of one launch
+// each into a scratch output, keeping each tile's fastest), and keeps the
+// fastest for the rest of the process -- the caller's tile unless another is at
+// least 3 % faster; later calls of that shape use it.  All tiles sum over k in
+// the same order, so tuning never changes a result: runs are bit-reproducible
+// across processes.  A call made while its stream is being captured into a
+// graph uses the caller's tile and records nothing.
 // ---------------------------------------------------------------------------
 struct TuneKey {
   int dt, opA, opB, M, N, K, herm;
@@ -677,8 +686,6 @@ template <class T> constexpr int dt_code() { return is_cplx<T>::value ? 1 : (std
 template <class T>
 GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K,
                     const T* A, int lda, const T* B, int ldb, int herm) {
-  // Every tile accumulates k in the same sequence, so the choice never changes
-  // a result.
   const TuneKey key{dt_code<T>(), opA, opB, M, N, K, herm};
   std::lock_guard<std::mutex> lk(g_tune_mu);
   auto it = g_tune.find(key);
