@@ -343,6 +343,11 @@ struct TileLoop {
   }
 };
 
+// 8 or 16 bytes at any multiple of 4.
+template <int BYTES> struct RawOf;
+template <> struct RawOf<16> { typedef unsigned type __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct RawOf<8> { typedef unsigned type __attribute__((ext_vector_type(2), aligned(4))); };
+
 // C = alpha op(A) op(B) + beta C (plain operands).  Block z of the grid takes
 // the k-slice [z Kc, z Kc + Kc) into C + z sC.  herm: a Hermitian product
 // (M == N, BM == BN, beta == 0): only tiles on and above the diagonal are
@@ -365,9 +370,11 @@ __global__ __launch_bounds__(256) void k_tile(int M, int N, int K, int Kc, T alp
   C += blockIdx.z * sC;
   const int li = lane & 15, lk = lane >> 4;
   const bool use_beta = !(real(beta) == 0.0 && imag(beta) == 0.0);
-  // lane -> row of C, register r -> column lk + 4r (f64) or 4 lk + r (f32)
+  // lane -> RW consecutive rows of C (the MFMA blocks of one group, see row_of),
+  // register r -> column lk + 4r (f64) or 4 lk + r (f32)
+  constexpr int RW = KFA ? 1 : TL::RVA;
 #pragma unroll
-  for (int i = 0; i < FM; ++i)
+  for (int i = 0; i < FM; i += RW)
 #pragma unroll
     for (int n = 0; n < FN; ++n)
 #pragma unroll
@@ -376,14 +383,41 @@ __global__ __launch_bounds__(256) void k_tile(int M, int N, int K, int Kc, T alp
         const int gn = n0 + wn * 16 * FN +
                        TL::row_of(KFB, TL::RVB, n, GT<T>::G1 ? lk + 4 * r : 4 * lk + r);
         if (gm < M && gn < N) {
-          T v;
-          if constexpr (TL::P == 1) v = T(acc[0][i][n][r]);
-          else v = make_scalar<T>(acc[0][i][n][r], acc[1][i][n][r]);
-          v = alpha * v;
+          T v[RW];
+#pragma unroll
+          for (int q = 0; q < RW; ++q) {
+            if constexpr (TL::P == 1) v[q] = T(acc[0][i + q][n][r]);
+            else v[q] = make_scalar<T>(acc[0][i + q][n][r], acc[1][i + q][n][r]);
+            v[q] = alpha * v[q];
+          }
           const long long idx = gm + (long long)gn * ldc;
-          if (use_beta) v = v + beta * C[idx];
-          C[idx] = v;
-          if (herm && blockIdx.x != blockIdx.y) C[gn + (long long)gm * ldc] = conj_v(v);
+          if constexpr (RW == 1) {
+            if (use_beta) v[0] = v[0] + beta * C[idx];
+            C[idx] = v[0];
+          } else if (gm + RW <= M) {  // one access for the RW rows
+            using R = typename RawOf<RW * sizeof(T)>::type;
+            R u;
+            if (use_beta) {
+              T old[RW];
+              u = *reinterpret_cast<const R*>(C + idx);
+              __builtin_memcpy(old, &u, sizeof(old));
+#pragma unroll
+              for (int q = 0; q < RW; ++q) v[q] = v[q] + beta * old[q];
+            }
+            __builtin_memcpy(&u, v, sizeof(v));
+            *reinterpret_cast<R*>(C + idx) = u;
+          } else {
+#pragma unroll
+            for (int q = 0; q < RW; ++q)
+              if (gm + q < M) {
+                if (use_beta) v[q] = v[q] + beta * C[idx + q];
+                C[idx + q] = v[q];
+              }
+          }
+          if (herm && blockIdx.x != blockIdx.y)
+#pragma unroll
+            for (int q = 0; q < RW; ++q)
+              if (gm + q < M) C[gn + (long long)(gm + q) * ldc] = conj_v(v[q]);
         }
       }
 }
