@@ -1505,7 +1505,10 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // values, 512^2: 0.5 ms; 2.4 ms with QR steps).
   // Nor does the eigen-solver (rank 0) take them: a general Hermitian matrix is
   // not graded (40^2 to 512^2: sweeps alone 0.73 to 0.99 of the time).
-  const bool qr = prm.qr && rank > 0 && !(check && *above < rank) && off0 > QR_GATE;
+  // Past the size of a panel splits are the sweeps' alone too (complex 1600^2 with
+  // one inner sweep: of low rank and of steep spectra 1.08 and 1.09 of the time).
+  const bool qr = prm.qr && rank > 0 && Np <= qr_max<T>() && !(check && *above < rank) &&
+                  off0 > QR_GATE;
   // It shares the other two measures of a cold split, one inner sweep per block
   // pair and first-order steps between the sweeps, where those pay (from
   // FO_MIN: 512^2 0.70 to 0.90 of the time; 40^2, 64^2 of low rank: 1.2).
@@ -1590,7 +1593,7 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
     off_rel = last_off / fro;
     done = last_off <= prm.tol * fro;
   };
-  const bool qr_ok = qr && Np >= QR_MIN && Np <= qr_max<T>();
+  const bool qr_ok = qr && Np >= QR_MIN;
   // Far from the eigenbasis: no basis given, or one whose measure is above the
   // gate, as in the second sweep of a run, or sweeps that stall (9 sweeps of a
   // 512^2 block before).  A given basis goes through the QR steps only where
