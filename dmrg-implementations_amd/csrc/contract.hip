@@ -39,8 +39,8 @@ void heff2_apply(hipStream_t st, const T* Lenv, const T* Renv, const T* WW, cons
   if (!fused) {
     if constexpr (std::is_same<T, float>::value) {
       if (sc.split_bf16) {
-        gemm_f32_split_bf16(st, OP_T, OP_N, D * cL, dd * cR, cL, Lenv, cL, theta, cL, sc.X, D * cL,
-                            sc.Y, need);
+        // no slices here: this product is as large as the free workspace
+        gemm_f32_split_bf16(st, OP_T, OP_N, D * cL, dd * cR, cL, Lenv, cL, theta, cL, sc.X, D * cL);
       } else {
         gemm<T>(st, OP_T, OP_N, D * cL, dd * cR, cL, one, Lenv, cL, theta, cL, zero, sc.X, D * cL,
                 pickT<T>(D * cL, dd * cR, cL));

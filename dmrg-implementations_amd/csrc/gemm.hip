@@ -18,9 +18,11 @@
 //    another: fragments of the next half tile are read while the present half
 //    multiplies, also across the barrier (one per tile).
 // Measured against the loop it replaces (element-wise LDS rows, loads under a
-// branch, which made every wait a wait for all loads): FP64 2048x512x2560
-// 120 -> 106 us, four k-slices 98 -> 88, 1024^3 50 -> 44, 512^3 10.9 -> 9.3;
-// FP32 2560x2048x512 69 -> 55, 2048x512x2560 87 -> 59 (two k-slices 69 -> 51).
+// branch, which made every wait a wait for all loads), us a call back to back:
+// FP64 1024^3 48.4 -> 40.4 (A and B plain), 46.5 -> 37.9 (A transposed), 49.3 ->
+// 41.1 (B transposed), 512^3 10.1 -> 9.0, 2048 x 512 x 2560 114 -> 94, 2560 x 2048 x
+// 512 with A transposed 95 -> 85; FP32 the last two 83 -> 54 and 66 -> 51; complex
+// 512^3 32.0 -> 21.2.
 #include "gemm.hpp"
 
 #include <type_traits>
@@ -1161,8 +1163,11 @@ void gemm_f32_split_bf16(hipStream_t st, int opA, int opB, int M, int N, int K, 
   if (M == 0 || N == 0) return;
   // op(A) (m, k): transposed storage is k-fast; op(B) (k, n): plain storage is k-fast
   const bool kfa = op_trans(opA), kfb = !op_trans(opB);
-  // Slices of k where the tiles leave the chip short of two workgroups a CU
-  // (what its LDS holds), each of eight k-tiles or more.
+  // Slices of k, each of eight k-tiles or more, up to three workgroups a CU: two
+  // are resident (LDS), and a grid just past that ends in a nearly empty wave
+  // (out-step at 768 x 768, D = 5, 576 tiles: matvec 386 us unsliced, 354 with two
+  // slices; limits of 256 to 1024 workgroups are within 8 % of one another at
+  // fourteen other shapes, in either direction).
   const int nkt = (int)cdiv(K, BF_BK);
   const long long tiles = (long long)cdiv(M, 64) * cdiv(N, 64);
   int S = 1;
