@@ -678,14 +678,14 @@ void dispatch(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N, int K
 // ---------------------------------------------------------------------------
 // Tile autotuner.  When enabled (gemm_autotune), the first call of each (scalar
 // type, ops, M, N, K, Hermitian) shape times the 32x32, 64x32 (not for a
-// Hermitian product) and 64x64 tiles on the caller's stream, with the device
-// otherwise idle (one warm-up each, then four interleaved rounds of one launch
-// each into a scratch output, keeping each tile's fastest), and keeps the
-// fastest for the rest of the process -- the caller's tile unless another is at
-// least 3 % faster; later calls of that shape use it.  All tiles sum over k in
-// the same order, so tuning never changes a result: runs are bit-reproducible
-// across processes.  A call made while its stream is being captured into a
-// graph uses the caller's tile and records nothing.
+// Hermitian product) and 64x64 tiles on the caller's stream, drained first (one
+// warm-up each, then four interleaved rounds of one launch each into a scratch
+// output, keeping each tile's fastest), and keeps the fastest for the rest of the
+// process -- the caller's tile unless another is at least 3 % faster; later calls
+// of that shape use it.  All tiles sum over k in the same order, so tuning never
+// changes a result: runs are bit-reproducible across processes.  A call made
+// while its stream is being captured into a graph uses the caller's tile and
+// records nothing.
 // ---------------------------------------------------------------------------
 struct TuneKey {
   int dt, opA, opB, M, N, K, herm;
@@ -751,9 +751,9 @@ GemmTile tuned_tile(hipStream_t st, int opA, int opB, GemmTile tl, int M, int N,
   GemmTile best = tl;
   float best_ms = 1e30f;
   try {
-    // Time on an idle device: other streams' work (the environment updates
-    // that overlap a bond) would otherwise bias whichever candidate it meets.
-    DMRG_HIP(hipDeviceSynchronize());
+    // Not the device: draining that is refused while any thread captures a
+    // stream of it, and breaks the capture.
+    DMRG_HIP(hipStreamSynchronize(st));
     for (int c = 0; c < NC; ++c)  // warm-up: code and operands into the caches
       dispatch<T>(st, opA, opB, cand[c], M, N, K, K, 1, T(1), A, lda, B, ldb, T(0), Cs, M, 0, herm);
     // Rounds interleave the candidates, and each keeps its fastest launch,

@@ -101,9 +101,10 @@ bool gemm_splitk(hipStream_t st, int opA, int opB, int M, int N, int K, const T*
 GemmTile gemm_pick_tile(int M, int N, int K, bool complex_);
 
 // Process-wide tile autotuner of gemm / gemm_herm: when on, the first call of
-// each shape (scalar type, ops, M, N, K) times the tiles on the caller's
-// stream and keeps the fastest for the rest of the process (the tile argument is then only the fallback of calls made during graph
-// capture).  gemm_autotune_entries() counts the shapes tuned so far.
+// each shape (scalar type, ops, M, N, K) times the tiles on the caller's stream
+// and keeps the fastest for the rest of the process (the tile argument is then
+// only the fallback of calls made during graph capture).
+// gemm_autotune_entries() counts the shapes tuned so far.
 void gemm_autotune(bool on);
 int gemm_autotune_entries();
 
