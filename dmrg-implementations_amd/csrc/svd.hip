@@ -26,12 +26,13 @@ constexpr int LDP = JP + 1;  // LDS column stride (padding)
 constexpr int NT = 256;      // threads of the pair kernels
 constexpr int SORT_MAX = 2048;
 // A kept group that reaches diagonal entries of rho below TAIL |rho|_F does not
-// go through the QR steps (see jacobi).  Bonds shrank in 7 of 450 runs of single-
-// site chains of 18 to 22 sites at chi = 256 without this rule, in one with
-// 1e-16, in none with 1e-17 or 1e-15; a chain of 32 sites at chi = 256 without
-// warm starts takes 0.46, 0.47, 0.57 and 0.76 s for three sweeps without it and
-// with 1e-17, 1e-16 and 1e-15, and 1.05 s by sweeps alone.  The largest of these:
-// it is next to the tolerance of the sweeps, which is what leaves the tail mixed.
+// go through the QR steps (see jacobi).  Without this rule 3 of 80 runs of chains
+// of 18 to 32 sites at chi = 200 and 256 lost vectors of a bond that is not
+// truncated; of 450 runs one with 1e-16, none with 1e-17 or 1e-15.  A chain of 32
+// sites at chi = 256 without warm starts takes 0.46, 0.47, 0.57 and 0.76 s for three
+// sweeps without it and with 1e-17, 1e-16 and 1e-15, and 1.05 s by sweeps alone.
+// The largest of these: it is next to the tolerance of the sweeps, which is what
+// leaves the tail mixed.
 constexpr double TAIL = 1e-15;
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
