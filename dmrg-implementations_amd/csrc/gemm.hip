@@ -822,12 +822,12 @@ namespace {
 // lower clock that their operand traffic leaves.  Complex k-tiles hold the same
 // bytes and twice the MFMAs; their 64x64 tile pays from two workgroups a CU on
 // (2048 x 2048 x 1024: 486 us, 514 with 32x32; 1024 x 1024 x 1024 137 and 135, x 32
-// 13.0 and 12.0), the 64x32 one hardly anywhere (640 x 640 x 1024: 79 us, 72 with
-// 32x32; 1152 x 1152 x 1024 194 and 196): at this price it is never taken.
+// 13.0 and 12.0), the 64x32 one too (640 x 640 x 1024: 79 us, 72 with 32x32; 1152 x
+// 1152 x 1024 194 and 196; first step of the matvec at 256, d = 5: 602 us in all, 606).
 double tile_cycles(const GemmTile& t, int w, bool cplx) {
   if (cplx) {
     if (t.bm == 32) return 640.0 * w;
-    return t.bn == 32 ? 1320.0 * w : std::max(2620.0, 2360.0 * w);
+    return t.bn == 32 ? std::max(1320.0, 1200.0 * w) : std::max(2620.0, 2360.0 * w);
   }
   if (t.bm == 32) return std::max(430.0, 332.0 * w);
   if (t.bn == 32) return std::max(620.0, 610.0 * w);
