@@ -216,11 +216,12 @@ __global__ __launch_bounds__(256) void k_rank_diag(const T* __restrict__ A, int 
   }
 }
 
-// *host = number of diagonal entries above both `thr` and TAIL |rho|_F (one wave).
+// *host = number of diagonal entries above both `thr` and rel |rho|_F (one wave).
 template <class T>
 __global__ __launch_bounds__(64) void k_count_diag(const T* __restrict__ A, int N, int Np, double thr,
-                                                   const double* __restrict__ scal, double* host) {
-  thr = fmax(thr, TAIL * scal[0]);
+                                                   double rel, const double* __restrict__ scal,
+                                                   double* host) {
+  thr = fmax(thr, rel * scal[0]);
   int a = 0;
   for (int i0 = 0; i0 < N; i0 += 64) {
     const int i = i0 + threadIdx.x;
@@ -1434,6 +1435,12 @@ struct JacobiCount {
   bool qr = false;  // QR steps were taken
 };
 
+// Whether the cutoff on Schmidt values lies below what tol * scale resolves of
+// their squares (scale: |rho|_F or the largest square).
+inline bool cut_below_resolution(double cut2, double cut_rel, double scale, double tol) {
+  return std::max(cut2, cut_rel * cut_rel * scale) < tol * scale;
+}
+
 template <class T>
 int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, JacobiCount& cnt,
            double& off_rel, bool v_given = false, int keep = 0, double cut_abs = 0.0,
@@ -1471,7 +1478,8 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
                        (const int*)nullptr, 0, hp);
   if (check)
     hipLaunchKernelGGL(k_count_diag<T>, dim3(1), dim3(64), 0, st, (const T*)w.A[0], N, Np,
-                       1e4 * cut_abs * cut_abs, (const double*)w.scal, above);
+                       1e4 * cut_abs * cut_abs, std::max(TAIL, 1e4 * cut_rel * cut_rel),
+                       (const double*)w.scal, above);
   DMRG_LAUNCH_CHECK();
   DMRG_HIP(hipStreamSynchronize(st));
   double fro = w.host[NRED + 2];
@@ -1502,14 +1510,18 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // them apart, and bonds that are not truncated would shrink (256 -> 247 at the
   // bond of 8 sites of a chain of 32 at chi = 256), at once or in a later sweep.
   // The diagonal of rho tells: what is not graded is mixed by rounding anyway.
+  // The same holds for a larger cutoff that reaches into the kept group, as long as
+  // it is below that resolution (single-site chains of 16 sites, chi = 64, cutoffs
+  // 1e-9 and 1e-10: 19 and 3 vectors a run fewer than the full bonds with QR steps, 2
+  // and 0.4 by sweeps alone); from 1e-7 on the two agree (127 both).
+  const bool tail = check && *above < rank && cut_below_resolution(cut2, cut_rel, fro, prm.tol);
   // And one next to diagonal needs a sweep or two (a matrix of equal Schmidt
   // values, 512^2: 0.5 ms; 2.4 ms with QR steps).
   // Nor does the eigen-solver (rank 0) take them: a general Hermitian matrix is
   // not graded (40^2 to 512^2: sweeps alone 0.73 to 0.99 of the time).
   // Past the size of a panel splits are the sweeps' alone too (complex 1600^2 with
   // one inner sweep: of low rank and of steep spectra 1.08 and 1.09 of the time).
-  const bool qr = prm.qr && rank > 0 && Np <= qr_max<T>() && !(check && *above < rank) &&
-                  off0 > QR_GATE;
+  const bool qr = prm.qr && rank > 0 && Np <= qr_max<T>() && !tail && off0 > QR_GATE;
   // It shares the other two measures of a cold split, one inner sweep per block
   // pair and first-order steps between the sweeps, where those pay (from
   // FO_MIN: 512^2 0.70 to 0.90 of the time; 40^2, 64^2 of low rank: 1.2).
@@ -1946,7 +1958,8 @@ SvdResult svd_split(hipStream_t st, SvdWork<T>& w, const T* A, int m, int n, int
     r2.oa_steps += res.oa_steps;
     return r2;
   };
-  if (jc.qr && nk < k && last * last < 100.0 * prm.tol * first * first) {
+  if (jc.qr && nk < k && last * last < 100.0 * prm.tol * first * first &&
+      cut_below_resolution(cutoff * cutoff, rel_cutoff, first * first, prm.tol)) {
     // the rank ends among Schmidt values below the resolution of rho, not in a
     // gap: the number of them is the sweeps' (see jacobi)
     SvdParams sweeps_only = prm;

@@ -22,6 +22,17 @@ def test_full_rank_bonds_keep_their_size(dmrg_amd, seed):
         assert list(eng.bond_dims()) == [min(2 ** i, 2 ** (L - i), chi) for i in range(L + 1)]
 
 
+@pytest.mark.parametrize("seed", [0, 1, 2])
+def test_single_site_bonds_with_a_cutoff(dmrg_amd, seed):
+    """Single-site splits start cold every time and cannot grow a bond again."""
+    L, chi = 16, 64
+    with dmrg_amd.DMRG(L, 2, chi, 5, tol=0.0, krylov_max=20, variant=dmrg_amd.SINGLE_SITE, svd_cutoff=1e-10) as eng:
+        eng.set_mpo(models.heisenberg_mpo(L))
+        eng.initialize_mps_random(seed=seed, scale=0.1)
+        eng.run(2)
+        assert list(eng.bond_dims()) == [min(2 ** i, 2 ** (L - i), chi) for i in range(L + 1)]
+
+
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("left", [False, True])
 @pytest.mark.parametrize("m,n,r", [(40, 50, 7), (130, 100, 30), (300, 260, 64)])
