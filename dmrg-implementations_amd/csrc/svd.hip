@@ -167,8 +167,8 @@ __global__ __launch_bounds__(256) void k_norms_fin(const double* __restrict__ re
     __syncthreads();
   }
   if (t == 0) {
-    *host = scal[0] = sqrt(s1[0]);
-    scal[2] = s2[0];
+    host[0] = scal[0] = sqrt(s1[0]);
+    host[2] = scal[2] = s2[0];
   }
 }
 
@@ -1363,6 +1363,10 @@ constexpr int FO_MIN = 160;
 // Stalling sweeps go back to QR steps above this measure (below it the pairs left
 // are few, and the first-order steps and a sweep or two end it).
 constexpr double QR_GATE = 1e-9;
+// Limits of the eigen-solver's QR steps (see jacobi): of 160^2 with 1/24 of the
+// eigenvalues not zero they cost as much as they save, and of Gram matrices of N and
+// 2 N random vectors (0.5 and 0.67) they take 0.98 and 1.08 of the time.
+constexpr double EIG_LO = 0.04, EIG_HI = 0.6;
 
 // A (Np x Np, ld Np) <- R, Q <- the unitary factor; work holds at least
 // 128 Np values (64 Np for Np < 128), Tm 32 * 32.
@@ -1473,9 +1477,11 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   if (v_given) measure(w.A[0]);  // read behind the one synchronisation
   double* const above = w.host + NRED + 3;
   const bool cold = prm.qr && !v_given && Np >= QR_MIN, check = cold && rank > 0;
-  if (cold)  // all pairs: the diagonal need not be the spectrum yet
+  auto couplings = [&] {  // all pairs: the diagonal need not be the spectrum yet
     hipLaunchKernelGGL(k_offmax<T>, dim3(NRED), dim3(256), 0, st, (const T*)w.A[0], N, Np,
                        (const int*)nullptr, 0, hp);
+  };
+  if (cold) couplings();
   if (check)
     hipLaunchKernelGGL(k_count_diag<T>, dim3(1), dim3(64), 0, st, (const T*)w.A[0], N, Np,
                        1e4 * cut_abs * cut_abs, std::max(TAIL, 1e4 * cut_rel * cut_rel),
@@ -1488,19 +1494,19 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // to rounding size: those of a norm far from one would leave the range of a
   // double (|rho|_F = 1e-140: the reflections dropped columns that count).  The
   // iteration then works on 2^e rho, which is exact.
-  double off0 = cold ? *std::max_element(hp, hp + NRED) / fro : INFINITY;
   int e2 = 0;
   if (fro != 0.0 && (fro < 0x1p-300 || fro > 0x1p+300)) {
     e2 = -std::ilogb(fro);
-    off0 = INFINITY;  // measured out of range
     hipLaunchKernelGGL(k_scale_pow2<T>, dim3(grid_for(tot)), dim3(256), 0, st, w.A[0], tot, e2,
                        (double*)nullptr);
     norms();
     if (v_given) measure(w.A[0]);
+    if (cold) couplings();
     DMRG_LAUNCH_CHECK();
     DMRG_HIP(hipStreamSynchronize(st));
     fro = w.host[NRED + 2];
   }
+  const double off0 = cold ? *std::max_element(hp, hp + NRED) / fro : INFINITY;
   const double cut2 = std::ldexp(cut_abs * cut_abs, e2);  // the cutoff in units of the scaled rho
   const double rot_tol = 0.125 * prm.tol;
   // Where the spectrum falls through the resolution of rho (tol |rho|_F) and on
@@ -1517,11 +1523,20 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   const bool tail = check && *above < rank && cut_below_resolution(cut2, cut_rel, fro, prm.tol);
   // And one next to diagonal needs a sweep or two (a matrix of equal Schmidt
   // values, 512^2: 0.5 ms; 2.4 ms with QR steps).
-  // Nor does the eigen-solver (rank 0) take them: a general Hermitian matrix is
-  // not graded (40^2 to 512^2: sweeps alone 0.73 to 0.99 of the time).
+  // The eigen-solver (rank 0) takes them for what looks like a density matrix:
+  // where the part of the spectrum that carries a positive semidefinite matrix,
+  // trace^2 / (N |rho|_F^2), is between EIG_LO and EIG_HI.  With them, by sweeps alone:
+  // 256^2, eigenvalues falling to 1e-6 and 1e-12 3.3 and 6.1, 3.2 and 8.9 ms, 1/8
+  // and 1/4 of them not zero 1.9 and 4.5, 1.1 and 5.1 ms.  Outside they cost more than
+  // they save (evenly spread over both signs 4.9 and 4.1, rank one 1.0 and 0.4 ms; 1/32
+  // not zero 0.7 to 1.3 of the time), as for blocks below FO_MIN and what is next
+  // to diagonal (couplings of 1e-3: 4.3 and 1.3 ms).  Well-conditioned kernel matrices
+  // lose: exp(-|i - j| / 10) 5.0 and 3.4 ms.
   // Past the size of a panel splits are the sweeps' alone too (complex 1600^2 with
   // one inner sweep: of low rank and of steep spectra 1.08 and 1.09 of the time).
-  const bool qr = prm.qr && rank > 0 && Np <= qr_max<T>() && !tail && off0 > QR_GATE;
+  const double tr = w.host[NRED + 4] / fro, part = tr > 0.0 ? tr * tr / N : 0.0;
+  const bool dense = Np >= FO_MIN && off0 * Np > 1.0 && part > EIG_LO && part < EIG_HI;
+  const bool qr = prm.qr && (rank > 0 || dense) && Np <= qr_max<T>() && !tail && off0 > QR_GATE;
   // It shares the other two measures of a cold split, one inner sweep per block
   // pair and first-order steps between the sweeps, where those pay (from
   // FO_MIN: 512^2 0.70 to 0.90 of the time; 40^2, 64^2 of low rank: 1.2).
