@@ -1368,6 +1368,10 @@ constexpr double QR_GATE = 1e-9;
 // eigenvalues not zero they cost as much as they save, and of Gram matrices of N and
 // 2 N random vectors (0.5 and 0.67) they take 0.98 and 1.08 of the time.
 constexpr double EIG_LO = 0.04, EIG_HI = 0.6;
+// And their smallest order: eigenvalues falling to 1e-6 and 1e-12 take 0.46 to 0.54
+// and 0.39 of the time with them at 112 and 128, 0.6 to 0.7 and 0.45 from 64 to 96,
+// kernel matrices and low rank above a flat background 1.0 to 1.25 and 1.1 to 1.45.
+constexpr int EIG_MIN = 128;
 
 // A (Np x Np, ld Np) <- R, Q <- the unitary factor; work holds at least
 // 128 Np values (64 Np for Np < 128), Tm 32 * 32.
@@ -1530,13 +1534,13 @@ int jacobi(hipStream_t st, SvdWork<T>& w, int N, int Np, const SvdParams& prm, J
   // 256^2, eigenvalues falling to 1e-6 and 1e-12 3.3 and 6.1, 3.2 and 8.9 ms, 1/8
   // and 1/4 of them not zero 1.9 and 4.5, 1.1 and 5.1 ms.  Outside they cost more than
   // they save (evenly spread over both signs 4.9 and 4.1, rank one 1.0 and 0.4 ms; 1/32
-  // not zero 0.7 to 1.3 of the time), as for blocks below FO_MIN and what is next
+  // not zero 0.7 to 1.3 of the time), as for blocks below EIG_MIN and what is next
   // to diagonal (couplings of 1e-3: 4.3 and 1.3 ms).  Well-conditioned kernel matrices
   // lose: exp(-|i - j| / 10) 5.0 and 3.4 ms.
   // Past the size of a panel splits are the sweeps' alone too (complex 1600^2 with
   // one inner sweep: of low rank and of steep spectra 1.08 and 1.09 of the time).
   const double tr = w.host[NRED + 4] / fro, part = tr > 0.0 ? tr * tr / N : 0.0;
-  const bool dense = Np >= FO_MIN && off0 * Np > 1.0 && part > EIG_LO && part < EIG_HI;
+  const bool dense = Np >= EIG_MIN && off0 * Np > 1.0 && part > EIG_LO && part < EIG_HI;
   const bool qr = prm.qr && (rank > 0 || dense) && Np <= qr_max<T>() && !tail && off0 > QR_GATE;
   // It shares the other two measures of a cold split, one inner sweep per block
   // pair and first-order steps between the sweeps, where those pay (from

@@ -1,7 +1,7 @@
-"""Eigen-solves on either side of the limits that choose their path: order 128
-and 129 (first-order steps and QR steps from a padded order of 160), the part of
-the spectrum that carries a positive semidefinite matrix (1/25 to 3/5 of it:
-QR steps), and spectra with many zeros (two inner sweeps a block pair).
+"""Eigen-solves on either side of the limits that choose their path: order 96 and
+97 (QR steps from a padded order of 128), 128 and 129 (first-order steps from
+160), the part of the spectrum that carries a positive semidefinite matrix (1/25
+to 3/5 of it: QR steps), and spectra with many zeros (two inner sweeps a block pair).
 
 The iteration stops once every coupling is below 1e-14 |H|_F, so an eigenvalue is
 within (N - 1) 1e-14 |H|_F of its row sum's centre, plus the rounding of some 20
@@ -34,7 +34,7 @@ def spectrum(kind, n):
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("kind", ["graded", "part-below", "part-above-low", "part-below-high", "part-above-high",
                                   "signs", "negative", "one"])
-@pytest.mark.parametrize("n", [128, 129, 160, 161, 330])
+@pytest.mark.parametrize("n", [96, 97, 128, 129, 160, 161, 330])
 def test_heig_spectra(dmrg_amd, ops, n, kind, cplx):
     rng = np.random.default_rng(n)
     U = np.linalg.qr(rand(rng, (n, n), cplx))[0]
